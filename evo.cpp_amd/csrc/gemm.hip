@@ -28,6 +28,8 @@
 #include <type_traits>
 
 #include "common.hpp"
+#include "gemm_epilogue.hpp"
+#include "gemm_tile.hpp"
 #include "row_norm.hpp"
 #include "ops.hpp"
 
@@ -39,18 +41,6 @@ constexpr int kBN = 256;
 constexpr int kBK = 32;
 constexpr int kThreads = 256;
 constexpr int kStride = kBK + 8;  // BF16 per LDS row
-
-struct Epilogue {
-  int mode;              // GemmEpilogue
-  const uint16_t *bias;  // BF16 [N]
-  const float *residual; // F32 [M, ldc]
-  int gelu;              // gated: erf-GELU on the l1 half
-  int gated_width;       // gated: valid output columns
-};
-
-__device__ inline float gelu_erf(const float x) {
-  return 0.5F * x * (1.0F + erff(x * 0.7071067811865475244F));
-}
 
 template <bool kSplit>
 __global__ __launch_bounds__(kThreads) void gemm_staged_kernel(
@@ -970,22 +960,53 @@ Status gemm_impl(const Activation &a, const RowNorm *norm, bool split, const uin
   if (K % kBK == 0) {
     // Few tiles (short prompts against W-wide outputs): split K so that about
     // one tile per CU runs, partials in the workspace, then one reduction.
-    int splits = 1;
     // (The reduction reads the partials as 16-byte vectors.)
-    if (mode != kGemmGated && split_workspace != nullptr &&
-        reinterpret_cast<uintptr_t>(split_workspace) % 16 == 0 && N % 4 == 0 && tiles < 128) {
+    const bool partials = mode != kGemmGated && split_workspace != nullptr &&
+                          reinterpret_cast<uintptr_t>(split_workspace) % 16 == 0 && N % 4 == 0;
+    int splits = 1;
+    if (partials && tiles < 128) {
       for (int s = 2; s <= 16 && tiles * s <= 256; s *= 2)
         if (K % (static_cast<size_t>(s) * kBK) == 0 && K / s >= 8 * kBK &&
             static_cast<size_t>(s) * M * N * sizeof(float) <= split_workspace_bytes)
           splits = s;
     }
+    // Tail split: when the last round would hold at most half the CUs, its
+    // tiles run as two K halves each (raw partials in the workspace), and
+    // gemm_tail_kernel sums them in order and applies the epilogue.
+    size_t tail = tiles > static_cast<size_t>(kGemmCUs) ? tiles % kGemmCUs : 0;
+    if (tail == 0 || 2 * tail > static_cast<size_t>(kGemmCUs) || split_workspace == nullptr ||
+        reinterpret_cast<uintptr_t>(split_workspace) % 16 != 0 || K % (2 * kBK) != 0 ||
+        K / 2 < 8 * static_cast<size_t>(kBK) ||
+        2 * tail * kBM * kBN * sizeof(float) > split_workspace_bytes)
+      tail = 0;
+    // The small tiles of gemm_tile.hip where their measured cost is lower. A
+    // tail-split launch stays here: more than one full round of 256 x 256
+    // tiles, no CU left idle (7B MLP l1/l2 of 1000 rows: 296 us against 335
+    // on the best small tile, 348 without the tail split).
+    TileChoice tile;
+    if (tail == 0)
+      tile = choose_gemm_tile(M, N, K, split, mode == kGemmGated, static_cast<size_t>(splits),
+                              partials ? split_workspace_bytes : 0, deferred != nullptr && ldc == n);
+    if (tile.tile >= 0)
+      splits = tile.splits;
+    const Epilogue store{kGemmStore, nullptr, nullptr, 0, 0};
+    const size_t plane = M * N;
+    if (tile.tile >= 0) {
+      const bool parted = splits > 1;
+      const TileCall call{a.hi, split ? a.lo : nullptr, lda, a.f16, W, m, n, k, splits,
+                          parted ? split_workspace : out.f32, parted ? plane : 0, out.hi, out.lo,
+                          parted ? n : ldc, parted ? store : epi};
+      EVO_TRY(gemm_tile(tile.tile, call, stream));
+      if (!parted)
+        return Status::Ok();
+    }
     if (splits > 1) {
-      const Epilogue store{kGemmStore, nullptr, nullptr, 0, 0};
       const dim3 split_grid(static_cast<unsigned>(tiles), static_cast<unsigned>(splits));
       const int ks = k / splits;
-      const size_t plane = M * N;
       const int all = static_cast<int>(tiles);
-      if (split)
+      if (tile.tile >= 0)
+        ;  // the partials are stored
+      else if (split)
         hipLaunchKernelGGL(gemm_kernel<true>, split_grid, dim3(512), 0, stream, a.hi, a.lo,
                            lda, W, k, m, n, ks, split_workspace, plane, nullptr, nullptr, n,
                            store, all, nullptr);
@@ -1014,15 +1035,6 @@ Status gemm_impl(const Activation &a, const RowNorm *norm, bool split, const uin
                          split_workspace, splits, m, n, out.f32, ldc, epi, vec);
       return launch_status("split_k_reduce_kernel");
     }
-    // Tail split: when the last round would hold at most half the CUs, its
-    // tiles run as two K halves each (raw partials in the workspace), and
-    // gemm_tail_kernel sums them in order and applies the epilogue.
-    size_t tail = tiles > static_cast<size_t>(kGemmCUs) ? tiles % kGemmCUs : 0;
-    if (tail == 0 || 2 * tail > static_cast<size_t>(kGemmCUs) || split_workspace == nullptr ||
-        reinterpret_cast<uintptr_t>(split_workspace) % 16 != 0 || K % (2 * kBK) != 0 ||
-        K / 2 < 8 * static_cast<size_t>(kBK) ||
-        2 * tail * kBM * kBN * sizeof(float) > split_workspace_bytes)
-      tail = 0;
     const int full = static_cast<int>(tiles - tail);
     const dim3 main_grid(static_cast<unsigned>(tiles + tail));
     if (split)

@@ -1,0 +1,394 @@
+// SPDX-License-Identifier: Apache-2.0
+// Dense linears on small block tiles: the products C[M,N] = A[M,K] . W[N,K]^T
+// of 5 to a few thousand rows, where 256 x 256 tiles (gemm.hip) leave most
+// CUs idle or multiply padding. Same operands, split-plane products and
+// epilogues as gemm.hip.
+//
+// Few rows are bound by the weight's bytes, so every CU has to stream its own
+// weight rows: a block tile is as narrow as the shape needs to fill 256 CUs
+// without splitting K across blocks (no workspace). Operands reach LDS by DMA
+// in row pieces of 128 or 256 bytes (64-byte pieces, what a 32-K step reads,
+// move 24-45 bytes per clock and CU from L2, 128-byte ones 58-60), 3-6 steps
+// deep, so the LDS holds up to 150 KB of reads in flight per CU. (Fragments
+// loaded straight to registers, 16 rows x 64 bytes per instruction, reached
+// 16-20 bytes per clock: 62 us against 37 for 61 rows of 4096 x 11264.)
+// The 32-K slices of a step go to different waves, which halves or quarters
+// the fragment reads a wave shape of the whole step would repeat; their sums
+// meet in LDS at the end.
+//
+// Measured (MI355X, split planes, weights from HBM; floor: their bytes at
+// the copy rate of 5 TB/s), against 256 x 256 tiles without a workspace:
+//   N = 22528, K = 4096 (gated):   5 rows 156 -> 34 us, 61 rows 150 -> 46,
+//     200 rows 157 -> 83, 700 rows 336 -> 239 (floor 37)
+//   N = 4096, K = 11264: 5 rows 390 -> 21 us, 61 rows 398 -> 37, 300 rows
+//     406 -> 89, 1000 rows 428 -> 157 (floor 18)
+//   N = K = 1920: 61 rows 79 -> 8 us, 1000 rows 88 -> 22.
+#include <algorithm>
+#include <cmath>
+#include <type_traits>
+
+#include "common.hpp"
+#include "gemm_epilogue.hpp"
+#include "gemm_tile.hpp"
+
+namespace evo::hip {
+namespace {
+
+// One block tile. kSeg K elements (64 or 128: 128- or 256-byte row pieces)
+// are staged per step; the waves are kWK (32-K slices of a step) x kWM x kWN.
+template <int kBM_, int kBN_, int kSeg_, int kWK_, int kWM_, int kWN_, int kStages_>
+struct TileShape {
+  static constexpr int kBM = kBM_, kBN = kBN_, kSeg = kSeg_, kWK = kWK_, kWM = kWM_, kWN = kWN_,
+                       kStages = kStages_;
+  static constexpr int kWaves = kWK * kWM * kWN;
+  static constexpr int kMI = kBM / 16 / kWM, kNJ = kBN / 16 / kWN;
+};
+
+// LDS of one row of kUnits 16-byte units: 16 consecutive rows read at one
+// logical unit (a fragment's rows) fall on 16 distinct 16-byte bank groups.
+template <int kUnits> __device__ inline int tile_unit(int row, int unit) {
+  return row * kUnits + (unit ^ (kUnits == 8 ? ((row >> 1) & 7) : (row & 15)));
+}
+
+// Waits until at most `later` (capped at kMax) steps of kPer DMAs are in flight.
+template <int kPer, int kMax> __device__ inline void wait_steps(int later) {
+  if constexpr (kMax <= 0) {
+    wait_dma<0>();
+  } else {
+    if (later >= kMax)
+      wait_dma<kPer * kMax>();
+    else
+      wait_steps<kPer, kMax - 1>(later);
+  }
+}
+
+template <typename T, bool kSplit, bool kF16>
+__global__ __launch_bounds__(T::kWaves * 64) void gemm_tile_kernel(
+    const uint16_t *__restrict__ a_hi, const uint16_t *__restrict__ a_lo, int lda,
+    const uint16_t *__restrict__ W, int ldw, int M, int N, int K, float *__restrict__ C,
+    size_t c_split, uint16_t *__restrict__ c_hi, uint16_t *__restrict__ c_lo, int ldc,
+    const Epilogue epi) {
+  using Frag = std::conditional_t<kF16, f16x8, bf16x8>;
+  constexpr int kPlanes = kSplit ? 2 : 1;
+  constexpr int kBM = T::kBM, kBN = T::kBN, kUnits = T::kSeg / 8;
+  constexpr int kMI = T::kMI, kNJ = T::kNJ, kTM = kBM / 16, kTN = kBN / 16;
+  constexpr int kStageBytes = (kPlanes * kBM + kBN) * T::kSeg * 2;
+  constexpr int kDma = kStageBytes / 1024 / T::kWaves;  // per wave and step
+  static_assert(kStageBytes % (1024 * T::kWaves) == 0 && kDma * (T::kStages - 2) < 64, "DMA split");
+  extern __shared__ __attribute__((aligned(16))) uint8_t tile_lds[];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wave_k = wave % T::kWK, wave_mn = wave / T::kWK;
+  const int wave_m = wave_mn / T::kWN, wave_n = wave_mn % T::kWN;
+  const int r16 = lane & 15, g = lane >> 4;
+  const bool gated = epi.mode == kGemmGated;
+  const int m_blocks = (M + kBM - 1) / kBM;
+  const int linear = xcd_linear(blockIdx.x, gridDim.x);
+  const int m0 = (linear % m_blocks) * kBM, block_n = linear / m_blocks;
+  {
+    const size_t k_first = static_cast<size_t>(blockIdx.y) * K;
+    a_hi += k_first;
+    if (kSplit)
+      a_lo += k_first;
+    W += k_first;
+    C += blockIdx.y * c_split;
+  }
+  // Weight row of tile column x. Gated: the first half of the tile holds the
+  // l1 rows, the second half the l2 rows of the same kBN / 2 gated columns.
+  auto weight_row = [&](int x) {
+    if (!gated)
+      return block_n * kBN + x;
+    const int half = x < kBN / 2 ? 0 : 1;
+    const int column = block_n * (kBN / 2) + x - half * (kBN / 2);
+    return (column / 32) * 64 + half * 32 + column % 32;
+  };
+  // This lane's DMA sources: rows of A hi, (A lo,) W in stage order.
+  const uint16_t *src[kDma];
+#pragma unroll
+  for (int i = 0; i < kDma; ++i) {
+    const int flat = (wave * kDma + i) * 64 + lane;
+    const int row = flat / kUnits;
+    const int unit = tile_unit<kUnits>(row, flat % kUnits) - row * kUnits;
+    const uint16_t *base;
+    if (row < kBM)
+      base = a_hi + static_cast<size_t>(min(m0 + row, M - 1)) * lda;
+    else if (kSplit && row < 2 * kBM)
+      base = a_lo + static_cast<size_t>(min(m0 + row - kBM, M - 1)) * lda;
+    else
+      base = W + static_cast<size_t>(min(weight_row(row - kPlanes * kBM), N - 1)) * ldw;
+    src[i] = base + unit * 8;
+  }
+  const int steps = (K + T::kSeg - 1) / T::kSeg;
+  // The last step of a K that is no multiple of kSeg reads the last kSeg
+  // elements and skips the 32-K slices the step before has multiplied.
+  auto issue = [&](int step) {
+    uint8_t *stage = tile_lds + (step % T::kStages) * kStageBytes;
+    const int k0 = min(step * T::kSeg, K - T::kSeg);
+#pragma unroll
+    for (int i = 0; i < kDma; ++i)
+      dma16(src[i] + k0, stage + (wave * kDma + i) * 1024);
+  };
+
+  f32x4 acc[kMI][kNJ];
+#pragma unroll
+  for (int i = 0; i < kMI; ++i)
+#pragma unroll
+    for (int j = 0; j < kNJ; ++j)
+      acc[i][j] = f32x4{0.0F, 0.0F, 0.0F, 0.0F};
+#pragma unroll
+  for (int s = 0; s + 1 < T::kStages; ++s)
+    if (s < steps)
+      issue(s);
+  for (int s = 0; s < steps; ++s) {
+    wait_steps<kDma, T::kStages - 2>(steps - 1 - s);
+    // Every wave's DMA of step s has landed, and every wave has left the
+    // buffer of step s - 1, which the next issue overwrites.
+    __syncthreads();
+    if (s + T::kStages - 1 < steps)
+      issue(s + T::kStages - 1);
+    const uint8_t *stage = tile_lds + (s % T::kStages) * kStageBytes;
+    const int skip = s + 1 < steps ? 0 : (steps * T::kSeg - K) / 32;
+#pragma unroll
+    for (int h = 0; h < T::kSeg / 32 / T::kWK; ++h) {
+      const int slice = h * T::kWK + wave_k;
+      if (slice < skip)
+        continue;
+      auto fragment = [&](int row) {
+        return *reinterpret_cast<const Frag *>(stage + tile_unit<kUnits>(row, slice * 4 + g) * 16);
+      };
+      Frag b[kNJ], ah[kMI], al[kMI];
+#pragma unroll
+      for (int j = 0; j < kNJ; ++j)
+        b[j] = fragment(kPlanes * kBM + (wave_n * kNJ + j) * 16 + r16);
+#pragma unroll
+      for (int i = 0; i < kMI; ++i) {
+        ah[i] = fragment((wave_m * kMI + i) * 16 + r16);
+        if (kSplit)
+          al[i] = fragment(kBM + (wave_m * kMI + i) * 16 + r16);
+      }
+#pragma unroll
+      for (int i = 0; i < kMI; ++i)
+#pragma unroll
+        for (int j = 0; j < kNJ; ++j) {
+          if constexpr (kF16)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[i], b[j], acc[i][j], 0, 0, 0);
+          else
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[i], b[j], acc[i][j], 0, 0, 0);
+        }
+      if constexpr (kSplit) {
+#pragma unroll
+        for (int i = 0; i < kMI; ++i)
+#pragma unroll
+          for (int j = 0; j < kNJ; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al[i], b[j], acc[i][j], 0, 0, 0);
+      }
+    }
+  }
+
+  // The block's 16 x 16 tiles through LDS, [wave_k][tile row][tile column]:
+  // the K slices are summed in order, and a gated pair meets in one lane.
+  __syncthreads();
+  f32x4 *part = reinterpret_cast<f32x4 *>(tile_lds);
+#pragma unroll
+  for (int i = 0; i < kMI; ++i)
+#pragma unroll
+    for (int j = 0; j < kNJ; ++j)
+      part[((wave_k * kTM + wave_m * kMI + i) * kTN + wave_n * kNJ + j) * 64 + lane] = acc[i][j];
+  __syncthreads();
+  auto total = [&](int ti, int tj) {
+    f32x4 v = part[(ti * kTN + tj) * 64 + lane];
+#pragma unroll
+    for (int w = 1; w < T::kWK; ++w) {
+      const f32x4 p = part[((w * kTM + ti) * kTN + tj) * 64 + lane];
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        v[e] = v[e] + p[e];
+    }
+    return v;
+  };
+  // Accumulator e of a tile: row 4 * (lane / 16) + e, column lane % 16.
+  if constexpr (kTN % 2 == 0) {
+    if (gated) {
+      for (int t = wave; t < kTM * (kTN / 2); t += T::kWaves) {
+        const int ti = t / (kTN / 2), tj = t % (kTN / 2);
+        const f32x4 first = total(ti, tj), second = total(ti, tj + kTN / 2);
+        const int col = block_n * (kBN / 2) + tj * 16 + r16;
+        if (col >= epi.gated_width)
+          continue;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int row = m0 + ti * 16 + 4 * g + e;
+          if (row < M) {
+            const float value = (epi.gelu ? gelu_erf(first[e]) : first[e]) * second[e];
+            const size_t index = static_cast<size_t>(row) * ldc + col;
+            const uint16_t hi = f32_to_bf16(value);
+            c_hi[index] = hi;
+            if (c_lo != nullptr)
+              c_lo[index] = f32_to_bf16(value - bf16_to_f32(hi));
+          }
+        }
+      }
+      return;
+    }
+  }
+  const bool bias_mode = epi.mode == kGemmBias || epi.mode == kGemmBiasResidual;
+  const bool res_mode = epi.mode == kGemmResidual || epi.mode == kGemmBiasResidual;
+  // Residuals ahead of the stores: C may alias the residual, so a load after
+  // a store would wait for it.
+  constexpr int kPerWave = (kTM * kTN + T::kWaves - 1) / T::kWaves;
+  float addend[kPerWave][4];
+#pragma unroll
+  for (int q = 0; q < kPerWave; ++q) {
+    const int t = min(wave + q * T::kWaves, kTM * kTN - 1);
+    const int col = min(block_n * kBN + (t % kTN) * 16 + r16, N - 1);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int row = min(m0 + (t / kTN) * 16 + 4 * g + e, M - 1);
+      addend[q][e] = res_mode ? epi.residual[static_cast<size_t>(row) * ldc + col] : 0.0F;
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < kPerWave; ++q) {
+    const int t = wave + q * T::kWaves;
+    const int col = block_n * kBN + (t % kTN) * 16 + r16;
+    if (t >= kTM * kTN || col >= N)
+      continue;
+    const f32x4 v = total(t / kTN, t % kTN);
+    const float bias = bias_mode ? bf16_to_f32(epi.bias[col]) : 0.0F;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int row = m0 + (t / kTN) * 16 + 4 * g + e;
+      if (row < M) {
+        float value = v[e];
+        if (bias_mode)
+          value = value + bias;
+        if (res_mode)
+          value = value + addend[q][e];
+        C[static_cast<size_t>(row) * ldc + col] = value;
+      }
+    }
+  }
+}
+
+template <typename T, bool kSplit, bool kF16>
+Status launch(const TileCall &c, hipStream_t stream) {
+  constexpr size_t stage = ((kSplit ? 2 : 1) * T::kBM + T::kBN) * T::kSeg * 2;
+  constexpr size_t lds = std::max<size_t>(T::kStages * stage,
+                                          static_cast<size_t>(T::kWK) * T::kBM * T::kBN * 4);
+  static_assert(lds <= 160 * 1024, "LDS");
+  const auto kernel = gemm_tile_kernel<T, kSplit, kF16>;
+  if (lds > 64 * 1024)
+    EVO_TRY(hip_status(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
+                                           hipFuncAttributeMaxDynamicSharedMemorySize,
+                                           static_cast<int>(lds)),
+                       "gemm_tile_kernel LDS opt-in"));
+  const dim3 grid(ceil_div(c.M, T::kBM) * ceil_div(c.N, T::kBN), static_cast<unsigned>(c.splits));
+  hipLaunchKernelGGL(kernel, grid, dim3(T::kWaves * 64), lds, stream, c.a_hi, c.a_lo, c.lda, c.W,
+                     c.K, c.M, c.N, c.K / c.splits, c.C, c.c_split, c.c_hi, c.c_lo, c.ldc, c.epi);
+  return launch_status("gemm_tile_kernel");
+}
+
+template <typename T> Status launch_planes(const TileCall &c, hipStream_t stream) {
+  if (c.a_lo != nullptr)
+    return launch<T, true, false>(c, stream);
+  return c.f16 ? launch<T, false, true>(c, stream) : launch<T, false, false>(c, stream);
+}
+
+// Measured time of a launch on one tile, in us: launch + rounds * (epilogue +
+// steps * step) + load * steps * blocks / 256, where a round fills every CU
+// with `slots` blocks (step[r - 1]: a K step of a CU's r blocks) and `load` is
+// what a step slows down by as the whole chip fills.
+struct TileCost {
+  float launch, epilogue, load;
+  int slots;
+  float step[3];
+};
+struct TileEntry {
+  int bm, bn, seg;
+  TileCost split, plane;  // hi + lo activation planes, one plane
+};
+// Least-squares fits over 5 to 8192 rows of the nine (N, K) of the 7B and 1B
+// topologies (median error 3-7 %; on that grid the tile the fit picks is
+// within 1 % of the fastest one in the geometric mean).
+constexpr TileEntry kTiles[] = {
+    {16, 16, 128, {2.11F, 1.10F, 0.027F, 2, {0.186F, 0.292F}}, {2.59F, 0.66F, 0.004F, 3, {0.185F, 0.269F, 0.347F}}},
+    {16, 32, 128, {2.57F, 0.77F, 0.050F, 2, {0.256F, 0.379F}}, {2.40F, 0.94F, 0.017F, 2, {0.234F, 0.310F}}},
+    {32, 32, 128, {1.30F, 2.12F, 0.088F, 1, {0.276F}}, {1.75F, 1.83F, 0.030F, 1, {0.249F}}},
+    {32, 64, 128, {1.21F, 2.63F, 0.147F, 1, {0.350F}}, {1.53F, 2.18F, 0.055F, 1, {0.310F}}},
+    {32, 96, 128, {1.22F, 2.85F, 0.181F, 1, {0.429F}}, {1.56F, 2.32F, 0.095F, 1, {0.375F}}},
+    {64, 64, 64, {1.41F, 2.70F, 0.103F, 1, {0.276F}}, {2.01F, 2.15F, 0.040F, 2, {0.251F, 0.404F}}},
+    {64, 128, 64, {1.37F, 4.30F, 0.139F, 1, {0.406F}}, {1.63F, 3.55F, 0.074F, 1, {0.329F}}},
+    {64, 192, 64, {1.17F, 5.72F, 0.144F, 1, {0.577F}}, {1.61F, 4.82F, 0.077F, 1, {0.474F}}},
+    {128, 128, 64, {0.68F, 7.12F, 0.180F, 1, {0.691F}}, {1.06F, 6.14F, 0.149F, 1, {0.410F}}},
+    {128, 192, 64, {1.28F, 7.28F, 0.280F, 1, {1.034F}}, {1.97F, 5.55F, 0.321F, 1, {0.709F}}},
+};
+constexpr int kTileCount = static_cast<int>(sizeof(kTiles) / sizeof(kTiles[0]));
+// The 256 x 256 tile of gemm.hip, the other candidate.
+constexpr TileEntry kLargeTile = {256, 256, 32, {0.0F, 9.34F, 0.294F, 1, {1.094F}},
+                                  {0.0F, 9.14F, 0.165F, 1, {0.737F}}};
+
+double tile_us(const TileEntry &t, bool split, size_t M, size_t N, size_t K, size_t parts) {
+  const TileCost &c = split ? t.split : t.plane;
+  const double blocks = static_cast<double>(ceil_div(M, t.bm)) * ceil_div(N, t.bn) * parts;
+  const double steps = ceil_div(K / parts, t.seg);
+  const double per_round = 256.0 * c.slots;
+  const double rounds = std::floor(blocks / per_round);
+  const int rest = static_cast<int>(std::ceil((blocks - rounds * per_round) / 256.0));
+  double us = c.launch + rounds * (c.epilogue + steps * c.step[c.slots - 1]) +
+              c.load * steps * blocks / 256.0;
+  if (rest > 0)
+    us += c.epilogue + steps * c.step[rest - 1];
+  // The weights from HBM at the measured copy rate (5 TB/s).
+  return std::max(us, 3.0 + 2.0 * static_cast<double>(N) * K / 5.0e6);
+}
+
+}  // namespace
+
+TileChoice choose_gemm_tile(size_t M, size_t N, size_t K, bool split, bool gated,
+                            size_t large_parts, size_t workspace_bytes, bool deferred) {
+  // Partial products cost their reduction: a launch unless the next norm
+  // sums them as it reads its rows, and their bytes at ~4 TB/s.
+  auto reduction = [&](size_t parts) {
+    return parts == 1 ? 0.0
+                      : (deferred ? 0.0 : 3.0) + 4.0 * static_cast<double>(parts) * M * N / 4.0e6;
+  };
+  TileChoice best;
+  double best_us = tile_us(kLargeTile, split, M, N, K, large_parts) + reduction(large_parts);
+  for (int t = 0; t < kTileCount; ++t) {
+    const size_t seg = static_cast<size_t>(kTiles[t].seg);
+    if (gated && kTiles[t].bn % 32 != 0)
+      continue;  // a gated tile pairs whole 16-column tiles
+    for (size_t parts = 1; parts <= 8; parts *= 2) {
+      if (K % (32 * parts) != 0 || K / parts < seg)
+        continue;
+      if (parts > 1 && (K / parts < 4 * seg || N % 4 != 0 || gated ||
+                        parts * M * N * sizeof(float) > workspace_bytes))
+        continue;
+      const double us = tile_us(kTiles[t], split, M, N, K, parts) + reduction(parts);
+      if (us < best_us) {
+        best_us = us;
+        best = TileChoice{t, static_cast<int>(parts)};
+      }
+    }
+  }
+  return best;
+}
+
+Status gemm_tile(int tile, const TileCall &call, hipStream_t stream) {
+  // The shapes of kTiles, in its order.
+  switch (tile) {
+  case 0: return launch_planes<TileShape<16, 16, 128, 4, 1, 1, 6>>(call, stream);
+  case 1: return launch_planes<TileShape<16, 32, 128, 4, 1, 1, 5>>(call, stream);
+  case 2: return launch_planes<TileShape<32, 32, 128, 4, 2, 1, 6>>(call, stream);
+  case 3: return launch_planes<TileShape<32, 64, 128, 4, 2, 1, 5>>(call, stream);
+  case 4: return launch_planes<TileShape<32, 96, 128, 4, 2, 1, 4>>(call, stream);
+  case 5: return launch_planes<TileShape<64, 64, 64, 2, 4, 1, 4>>(call, stream);
+  case 6: return launch_planes<TileShape<64, 128, 64, 2, 4, 1, 4>>(call, stream);
+  case 7: return launch_planes<TileShape<64, 192, 64, 2, 4, 1, 4>>(call, stream);
+  case 8: return launch_planes<TileShape<128, 128, 64, 2, 4, 1, 3>>(call, stream);
+  case 9: return launch_planes<TileShape<128, 192, 64, 1, 4, 2, 2>>(call, stream);
+  default: return {ErrorCode::kInternal, "gemm_tile: unknown tile"};
+  }
+}
+
+}  // namespace evo::hip

@@ -232,6 +232,86 @@ def test_linear_tail_split_matches_unsplit(m, n, k, bias, residual):
     assert np.array_equal(host(parted), plain)
 
 
+@pytest.mark.parametrize("m,n,k", [
+    (5, 40, 128), (17, 333, 224), (61, 4096, 256), (65, 4100, 288), (100, 4104, 416),
+    (129, 5000, 352), (150, 8200, 160), (300, 8200, 224), (1000, 4098, 352), (520, 9000, 288),
+    (130, 77, 64)])
+@pytest.mark.parametrize("planes,bias,residual", [(2, True, True), (1, False, False)])
+def test_linear_small_tiles_match_oracle(m, n, k, planes, bias, residual):
+    """Each block tile of the few-to-thousand-row products: ragged last tiles
+    in M and N, K of one step, of whole steps and with a last step of 1-3
+    32-K slices. The error of a split product is its activation's rounding,
+    2^-17 per term; F32 sums of K <= 416 terms add less. Rows past the
+    output stay untouched."""
+    r = rng(m + n + k + planes)
+    x = r.standard_normal((m, k)).astype(np.float32)
+    w = bf16_bits(r.standard_normal((n, k)).astype(np.float32) / np.sqrt(k))
+    b = bf16_bits(r.standard_normal(n).astype(np.float32) * 0.1) if bias else None
+    res = r.standard_normal((m, n)).astype(np.float32) if residual else None
+    hi, lo = split_gpu(x)
+    out = empty((m + 1, n))
+    out.fill_(7.0)
+    N.call("evo_hip_linear", p(hi), p(lo) if planes == 2 else None, p(dev(w)),
+           p(dev(b) if bias else None), p(dev(res) if residual else None), m, n, k, p(out),
+           stream())
+    got = host(out)
+    expected = O.linear_bf16w(x if planes == 2 else bf16_to_f32(bf16_bits(x)), w, b)
+    if residual:
+        expected = expected + res
+    assert rel_err(got[:m], expected) < 2e-5
+    assert np.all(got[m] == 7.0)
+
+
+@pytest.mark.parametrize("m,n,k", [(5, 512, 4096), (61, 4096, 11264), (300, 4096, 11264)])
+def test_linear_small_tiles_split_k(m, n, k):
+    """With a workspace the small tiles run as K parts where that is the
+    cheaper product: equal to the unsplit one up to the F32 summation order
+    (~sqrt(K) ulps of the partial sums)."""
+    r = rng(m + n + k)
+    x = r.standard_normal((m, k)).astype(np.float32)
+    w = bf16_bits(r.standard_normal((n, k)).astype(np.float32) / np.sqrt(k))
+    res = r.standard_normal((m, n)).astype(np.float32)
+    hi, lo = split_gpu(x)
+    args = (p(hi), p(lo), p(dev(w)), None, p(dev(res)), m, n, k)
+    plain, parted = empty((m, n)), empty((m, n))
+    N.call("evo_hip_linear", *args, p(plain), stream())
+    workspace = empty((8 * m * n,))
+    N.call("evo_hip_linear_split", *args, p(parted), p(workspace), 8 * m * n * 4, stream())
+    assert rel_err(host(parted), host(plain)) < 1e-5
+    cols = slice(n - 80, n)
+    expected = O.linear_bf16w(x, w[cols], None) + res[:, cols]
+    assert rel_err(host(parted)[:, cols], expected) < 2e-5
+
+
+@pytest.mark.parametrize("m,width,inner", [(5, 128, 80), (16, 256, 1000), (61, 288, 2048),
+                                           (100, 416, 2064), (150, 160, 4100 // 8 * 8),
+                                           (300, 224, 4096), (520, 288, 4504)])
+@pytest.mark.parametrize("gelu,planes", [(1, 2), (0, 1)])
+def test_gated_mlp_small_tiles(m, width, inner, gelu, planes):
+    """The gated epilogue of each small tile (l1 and l2 columns of one tile
+    pair up), inner widths that end inside a 32-row block. One plane rounds
+    the gated activation to BF16: 2^-9 relative per term of the l3 sums."""
+    from scipy.special import erf
+    r = rng(m + width + inner + planes)
+    x = r.standard_normal((m, width)).astype(np.float32)
+    l1 = bf16_bits(r.standard_normal((inner, width)).astype(np.float32) / np.sqrt(width))
+    l2 = bf16_bits(r.standard_normal((inner, width)).astype(np.float32) / np.sqrt(width))
+    l3 = bf16_bits(r.standard_normal((width, inner)).astype(np.float32) / np.sqrt(inner))
+    padded = (inner + 31) // 32 * 32
+    w12 = zeros((2 * padded, width), np.uint16)
+    N.call("evo_hip_pack_mlp", p(dev(l1)), p(dev(l2)), inner, width, p(w12), stream())
+    scratch, out = empty((planes * m * inner,), np.uint16), empty((m, width))
+    hi, lo = split_gpu(x)
+    N.call("evo_hip_gated_mlp", p(hi), p(lo) if planes == 2 else None, p(w12), p(dev(l3)), m,
+           width, inner, gelu, p(scratch), None, p(out), stream())
+    a = x if planes == 2 else bf16_to_f32(bf16_bits(x))
+    first = O.linear_bf16w(a, l1).astype(np.float64)
+    second = O.linear_bf16w(a, l2).astype(np.float64)
+    act = 0.5 * first * (1 + erf(first / np.sqrt(2))) if gelu else first
+    expected = O.linear_bf16w((act * second).astype(np.float32), l3)
+    assert rel_err(host(out), expected) < (1e-4 if planes == 2 else 2.0 ** -8)
+
+
 def split_gpu(x):
     hi, lo = empty(x.shape, np.uint16), empty(x.shape, np.uint16)
     N.call("evo_hip_split_f32", p(dev(x)), x.size, p(hi), p(lo), stream())
