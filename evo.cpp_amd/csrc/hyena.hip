@@ -21,6 +21,7 @@
 #include "common.hpp"
 #include "ops.hpp"
 
+#include <cmath>
 #include <mutex>
 #include <type_traits>
 
@@ -360,7 +361,7 @@ __global__ __launch_bounds__(256) void hyena_fir_kernel(
 // Each lane owns two adjacent channels: their six interleaved projection
 // columns are 12 (BF16) or 24 (F32) contiguous bytes of a row, and the two
 // outputs are one packed 32-bit store per plane. A wave streams a segment of
-// 64 or 128 rows (kStreamRows, kStreamMaxRows); it starts kLead rows early
+// 16 to 128 rows (kStreamRows, kStreamMaxRows); it starts kLead rows early
 // so that its short-FIR window and its FIR window of u are full when the
 // segment begins (the lead rows are recomputed, not stored). Both windows
 // hold their taps right-aligned with zeros in front, so every sum runs oldest
@@ -372,10 +373,14 @@ __global__ __launch_bounds__(256) void hyena_fir_kernel(
 // are non-temporal: the outputs are never re-read here, and streaming them
 // past the L2 keeps it for the projection rows (-23 % kernel time on the 7B
 // shape).
-// Segment length: 64 rows, doubled to 128 when the grid keeps at least
+// Segment length: 16 rows, doubled up to 128 while the grid keeps at least
 // kStreamMinBlocks blocks (two per CU): longer segments recompute fewer lead
-// rows (7B, L = 8192: 58 -> 54 us; 256 rows measured no better).
-constexpr int kStreamRows = 64;
+// rows (7B, L = 8192: 64 rows 58 us, 128 rows 54; 256 measured no better),
+// shorter ones are what fills the chip for a short prompt, where a block's
+// serial walk is the time (611 rows at W = 4096, BF16, with both histories:
+// 23.5 us with 64-row segments, 16.2; W = 1920, whose odd groups ran tile by
+// tile in LDS before: 54.3 -> 13.9 us, 8192 rows 302 -> 26).
+constexpr int kStreamRows = 16;
 constexpr int kStreamMaxRows = 128;
 constexpr unsigned kStreamMinBlocks = 512;
 constexpr int kStreamBatch = 4;
@@ -502,9 +507,11 @@ template <> struct PairOut<SplitOut> {
   }
 };
 
-template <typename T, int kWin, int kTaps, bool kDirect>
+template <typename T, int kWin, int kTaps, bool kDirect, bool kPairTaps>
 struct PairFir {
-  float stap[6][kWin], ftap[kTaps], d[2];
+  // kPairTaps: the pair's channels lie in filter groups of their own (odd
+  // group sizes); otherwise both use ftap[0].
+  float stap[6][kWin], ftap[kPairTaps ? 2 : 1][kTaps], d[2];
   float swin[6][kWin], uwin[2][kTaps];  // slot kWin-1 / kTaps-1 is the newest
 
   // One row: shifts the six projection values and u into the windows and
@@ -533,7 +540,7 @@ struct PairFir {
       float total = 0.0F;
 #pragma unroll
       for (int i = 0; i < kTaps; ++i)
-        total += uwin[ch][i] * ftap[i];
+        total += uwin[ch][i] * ftap[kPairTaps ? ch : 0][i];
       if constexpr (kDirect)
         total += d[ch] * u;
       y[ch] = fir[3 * ch] * total;
@@ -541,7 +548,7 @@ struct PairFir {
   }
 };
 
-template <typename T, typename O, int kWin, int kTaps, bool kDirect>
+template <typename T, typename O, int kWin, int kTaps, bool kDirect, bool kPairTaps>
 __global__ __launch_bounds__(kStreamWaves * 64) void hyena_fir_stream_kernel(
     const T *__restrict__ P, const float *__restrict__ short_history,
     const uint16_t *__restrict__ short_filter, int short_len,
@@ -566,7 +573,7 @@ __global__ __launch_bounds__(kStreamWaves * 64) void hyena_fir_stream_kernel(
   const uint32_t seg_rows = static_cast<uint32_t>(min(L - t0, static_cast<size_t>(seg_len)));
   const size_t cols3 = 3 * W;
 
-  PairFir<T, kWin, kTaps, kDirect> fir;
+  PairFir<T, kWin, kTaps, kDirect, kPairTaps> fir;
 #pragma unroll
   for (int ch = 0; ch < 2; ++ch) {
     float t3[3][kWin];
@@ -577,11 +584,14 @@ __global__ __launch_bounds__(kStreamWaves * 64) void hyena_fir_stream_kernel(
       for (int i = 0; i < kWin; ++i)
         fir.stap[3 * ch + s][i] = t3[s][i];
   }
-  const float *h = filter + (c / group_size) * k;
 #pragma unroll
-  for (int i = 0; i < kTaps; ++i) {
-    const int j = i - (kTaps - k);
-    fir.ftap[i] = j >= 0 ? h[causal ? k - 1 - j : j] : 0.0F;
+  for (int ch = 0; ch < (kPairTaps ? 2 : 1); ++ch) {
+    const float *h = filter + ((c + ch) / group_size) * k;
+#pragma unroll
+    for (int i = 0; i < kTaps; ++i) {
+      const int j = i - (kTaps - k);
+      fir.ftap[ch][i] = j >= 0 ? h[causal ? k - 1 - j : j] : 0.0F;
+    }
   }
   if constexpr (kDirect) {
     fir.d[0] = direct[c];
@@ -1253,10 +1263,8 @@ __global__ __launch_bounds__(256) void hcl_output_pair_kernel(
 
 // ---- Grouped FIR with k <= 128 (HCM) as a row stream on MFMA.
 // A block owns 64 channels (four 16-channel slices, one per wave; each slice
-// lies in one filter group) and a segment of kMsSegment output rows (fewer,
-// down to kMsMinSegment, while the grid would have under kMsMinBlocks
-// blocks: a 1024-token prompt at W = 4096 gets 256 blocks, not 64), walked
-// in steps of 32 rows:
+// lies in one filter group) and a segment of kMsSegment output rows or fewer
+// (ms_segment), walked in steps of 32 rows:
 //  1. production (all lanes, two adjacent channels x 4 rows each): short FIR
 //     and gates from the projection rows, u as split BF16 planes into LDS
 //     ([channel][row], so one ds_read_b128 is a B fragment) and x2 into LDS;
@@ -1275,8 +1283,7 @@ constexpr int kMsStep = 32;
 constexpr int kMsK = 5;             // K steps in the window
 constexpr int kMsChannels = 64;
 constexpr int kMsSegment = 1024;
-constexpr int kMsMinSegment = 256;
-constexpr unsigned kMsMinBlocks = 256;
+constexpr int kMsMinSegment = 128;  // a later segment's lead starts inside the sequence
 constexpr int kMsLead = 4;
 constexpr int kMsUStride = 40;      // BF16 per channel in the u stage (80 B)
 
@@ -1354,8 +1361,47 @@ template <> struct MsOut<SplitOut> {
 
 // Two blocks per CU for BF16 projections (71 KB of LDS); F32 projection
 // rows double the DMA stage (97 KB), so one block per CU.
-template <typename T, typename O>
-__global__ __launch_bounds__(256, sizeof(T) == 2 ? 2 : 1) void hyena_fir_mfma_stream_kernel(
+// Y + d u of one output, tap by tap in the reference's order (short FIR of
+// 3), u recomputed from the projection or read from the inner history.
+template <typename T>
+__device__ float hcm_window_sum(const T *P, const float *short_history,
+                                const uint16_t *short_filter, const float *inner_history,
+                                const float *h, int k, int causal, float d, size_t W, long t,
+                                size_t c) {
+  float total = 0.0F, u = 0.0F;
+#pragma unroll 1
+  for (int old = 0; old < k; ++old) {
+    const long row = t - (k - 1) + old;
+    if (row >= 0) {
+      float fir[2] = {0.0F, 0.0F};
+#pragma unroll
+      for (int s = 0; s < 2; ++s)
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+          fir[s] += p_at(P, short_history, 3 * W, 2, row - 2 + j, 3 * c + 1 + s) *
+                    bf16_to_f32(short_filter[(3 * c + 1 + s) * 3 + j]);
+      u = fir[0] * fir[1];
+    } else {
+      u = inner_history != nullptr ? inner_history[static_cast<size_t>(k - 1 + row) * W + c] : 0.0F;
+    }
+    total += u * h[causal ? k - 1 - old : old];
+  }
+  return total + d * u;
+}
+
+// kTwoGroups: group sizes that are no multiple of 16 (at least 15, so a
+// 16-channel slice touches at most two groups; the 1B topology has 15): each
+// slice multiplies with both groups' Toeplitz fragments and every lane keeps
+// its channel's result. u is split in three BF16 planes there (24 bits), the
+// precision of the F32 FIR on the VALU that these shapes ran before (error
+// against 64 bits 1.4e-7, before 2.0e-7); 60 MFMAs of 16 cycles per wave and
+// step still fit beside the production's VALU work. In a Toeplitz product an
+// infinity or NaN in u would reach every row of its 32-row steps through the
+// zero taps: production flags such steps, and outputs whose window holds one
+// are summed tap by tap (hcm_window_sum). 8192 rows at W = 1920:
+// 2505 -> 74 us (BF16), 2529 -> 97 us (F32).
+template <typename T, typename O, bool kTwoGroups>
+__global__ __launch_bounds__(256, sizeof(T) == 2 && !kTwoGroups ? 2 : 1) void hyena_fir_mfma_stream_kernel(
     const T *__restrict__ P, const float *__restrict__ short_history,
     const uint16_t *__restrict__ short_filter, int short_len,
     const float *__restrict__ inner_history, const float *__restrict__ filter,
@@ -1372,12 +1418,19 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? 2 : 1) void hyena_fir_mfma_st
   constexpr int kDmaPerStep = (kUnits + 255) / 256;        // per thread
   constexpr int kDmaMin = kUnits / 256;                    // per wave, at least
   constexpr int kStages = 2;
+  constexpr int kUPlanes = kTwoGroups ? 3 : 2;              // u = sum of BF16 planes
   // Software pipeline: in phase s the block flushes step s-1, produces step
   // s+1 and multiplies step s, so u is double buffered and x2 (overwritten in
   // place by y) triple buffered.
   __shared__ __attribute__((aligned(16))) unsigned char p_s[kStages][kStageRows * kRowBytes];
-  __shared__ __attribute__((aligned(16))) uint16_t u_s[2][2][kMsChannels][kMsUStride];
+  __shared__ __attribute__((aligned(16))) uint16_t u_s[2][kUPlanes][kMsChannels][kMsUStride];
   __shared__ __attribute__((aligned(16))) float xy_s[3][kMsStep][kMsChannels];
+  // kTwoGroups: steps (mod 8) with a u value the planes do not hold.
+  __shared__ unsigned flag_s[kTwoGroups ? 8 : 1];
+  constexpr float kUMax = 3.38e38F;  // rounds to a finite BF16 value
+  if (kTwoGroups && threadIdx.x < 8)
+    flag_s[threadIdx.x] = 0U;
+  bool history_flag = false;
 
   const unsigned total = channel_blocks * segments;
   const unsigned xcd = blockIdx.x % 8, q8 = total / 8, r8 = total % 8;
@@ -1478,7 +1531,10 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? 2 : 1) void hyena_fir_mfma_st
   // ---- MFMA lane: channel slice `wave`, fragment group g.
   const int col = lane & 15, g = lane >> 4;
   const size_t cw = c0 + 16 * wave + col;
-  const float *h = filter + ((c0 + 16 * wave) / group_size) * k;
+  constexpr int kFilters = kTwoGroups ? 2 : 1;
+  const size_t slice_group[2] = {(c0 + 16 * wave) / group_size,
+                                 (c0 + 16 * wave + 15) / group_size};
+  const bool second = kTwoGroups && cw / group_size != slice_group[0];  // this lane's filter
   // The wave's filter (k <= 128 taps of its group) goes to LDS between 160
   // zeros on either side, so that the Toeplitz fragments gather from there
   // after the first barrier with unconditional reads (80 taps per lane read
@@ -1488,32 +1544,41 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? 2 : 1) void hyena_fir_mfma_st
   // covers them; otherwise by plain loads before the stages are issued (a
   // wait for a load issued behind the DMA would wait for the DMA too). The
   // scratch is the third x2 / y buffer, which the production first writes in
-  // phase 1: 448 floats per wave, then the block's 64 direct terms.
+  // phase 1: 448 floats per wave, then the block's 64 direct terms; a second
+  // filter's is the second buffer, first written in phase 0.
   constexpr int kTapPad = 160;
-  float *taps_s = &xy_s[2][0][0] + wave * (2 * kTapPad + 128);
+  float *taps_s[2] = {&xy_s[2][0][0] + wave * (2 * kTapPad + 128),
+                      &xy_s[1][0][0] + wave * (2 * kTapPad + 128)};
   float *direct_s = &xy_s[2][0][0] + 4 * (2 * kTapPad + 128);
   const bool dma_consts = k % 4 == 0 && reinterpret_cast<uintptr_t>(filter) % 16 == 0 &&
                           reinterpret_cast<uintptr_t>(direct) % 16 == 0;
-  for (int i = lane; i < kTapPad; i += 64)
-    taps_s[i] = 0.0F;
-  for (int i = kTapPad + k + lane; i < 2 * kTapPad + 128; i += 64)
-    taps_s[i] = 0.0F;
+#pragma unroll
+  for (int f = 0; f < kFilters; ++f) {
+    for (int i = lane; i < kTapPad; i += 64)
+      taps_s[f][i] = 0.0F;
+    for (int i = kTapPad + k + lane; i < 2 * kTapPad + 128; i += 64)
+      taps_s[f][i] = 0.0F;
+  }
   float d = 0.0F;
   if (dma_consts) {
-    if (lane < k / 4)
-      dma16(h + 4 * lane, taps_s + kTapPad);
+#pragma unroll
+    for (int f = 0; f < kFilters; ++f)
+      if (lane < k / 4)
+        dma16(filter + slice_group[f] * k + 4 * lane, taps_s[f] + kTapPad);
     if (wave == 0 && lane < kMsChannels / 4)
       dma16(direct + c0 + 4 * lane, direct_s);
   } else {
-    for (int i = lane; i < k; i += 64)
-      taps_s[kTapPad + i] = h[i];
+#pragma unroll
+    for (int f = 0; f < kFilters; ++f)
+      for (int i = lane; i < k; i += 64)
+        taps_s[f][kTapPad + i] = filter[slice_group[f] * k + i];
     d = direct[cw];
     asm volatile("" : "+v"(d));
   }
   for (int step = 0; step < kStages && step < steps; ++step)
     issue(step);
-  u32x4 a[2][kMsK];
-  u32x4 ring_hi[kMsK], ring_lo[kMsK];  // BF16 x 8 fragments as raw words
+  u32x4 a[kFilters][2][kMsK];
+  u32x4 ring[kUPlanes][kMsK];  // BF16 x 8 fragments as raw words
 #pragma unroll
   for (int q = 0; q < kMsK; ++q) {
     // Window rows before the first step (only the first segment has them:
@@ -1521,19 +1586,25 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? 2 : 1) void hyena_fir_mfma_st
     // step 0 window slot q is register q + 1 (slot 4, register 0, receives
     // step 0), so register q holds rows of step q - 1 relative to the first
     // window.
-    uint16_t hi[8] = {}, lo[8] = {};
+    uint16_t plane[kUPlanes][8] = {};
     if (lead == 0 && inner_history != nullptr && q > 0) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         const long row = 32 * q + 8 * g + e - 160;
         const long hrow = static_cast<long>(k - 1) + row;
-        const float u = hrow >= 0 ? inner_history[static_cast<size_t>(hrow) * W + cw] : 0.0F;
-        hi[e] = f32_to_bf16(u);
-        lo[e] = f32_to_bf16(u - bf16_to_f32(hi[e]));
+        float u = hrow >= 0 ? inner_history[static_cast<size_t>(hrow) * W + cw] : 0.0F;
+        if constexpr (kTwoGroups)
+          history_flag |= !(__builtin_fabsf(u) <= kUMax);
+#pragma unroll
+        for (int p = 0; p < kUPlanes; ++p) {
+          plane[p][e] = f32_to_bf16(u);
+          u -= bf16_to_f32(plane[p][e]);
+        }
       }
     }
-    ring_hi[q] = __builtin_bit_cast(u32x4, hi);
-    ring_lo[q] = __builtin_bit_cast(u32x4, lo);
+#pragma unroll
+    for (int p = 0; p < kUPlanes; ++p)
+      ring[p][q] = __builtin_bit_cast(u32x4, plane[p]);
   }
 
   // ---- Production of step `step`: rows t_start + 32 step + 4 rg .. + 3
@@ -1577,22 +1648,31 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? 2 : 1) void hyena_fir_mfma_st
       u[1][j] = fir[4] * fir[5];
       *reinterpret_cast<float2 *>(x2 + j * kMsChannels) = make_float2(fir[0], fir[3]);
     }
-    // Rows (0, 1) and (2, 3) of a channel pack into one word per plane.
-    uint32_t uh[2][2], ul[2][2];
+    if constexpr (kTwoGroups) {
+      bool flag = false;
 #pragma unroll
-    for (int ch = 0; ch < 2; ++ch)
-#pragma unroll
-      for (int w = 0; w < 2; ++w) {
-        uh[ch][w] = pack_bf16(u[ch][2 * w], u[ch][2 * w + 1]);
-        ul[ch][w] = pack_bf16(u[ch][2 * w] - __builtin_bit_cast(float, uh[ch][w] << 16),
-                              u[ch][2 * w + 1] - __builtin_bit_cast(float, uh[ch][w] & 0xffff0000U));
-      }
-#pragma unroll
-    for (int ch = 0; ch < 2; ++ch) {
-      *reinterpret_cast<uint2 *>(uplanes + u_prod[ch]) = make_uint2(uh[ch][0], uh[ch][1]);
-      *reinterpret_cast<uint2 *>(uplanes + kUPlane + u_prod[ch]) =
-          make_uint2(ul[ch][0], ul[ch][1]);
+      for (int j = 0; j < 4; ++j)
+        flag |= !(__builtin_fabsf(u[0][j]) <= kUMax && __builtin_fabsf(u[1][j]) <= kUMax);
+      if (flag)
+        atomicOr(&flag_s[step % 8], 1U);
     }
+    // Rows (0, 1) and (2, 3) of a channel pack into one word per plane.
+#pragma unroll
+    for (int p = 0; p < kUPlanes; ++p)
+#pragma unroll
+      for (int ch = 0; ch < 2; ++ch) {
+        uint32_t word[2];
+#pragma unroll
+        for (int w = 0; w < 2; ++w) {
+          word[w] = pack_bf16(u[ch][2 * w], u[ch][2 * w + 1]);
+          if (p + 1 < kUPlanes) {
+            u[ch][2 * w] -= __builtin_bit_cast(float, word[w] << 16);
+            u[ch][2 * w + 1] -= __builtin_bit_cast(float, word[w] & 0xffff0000U);
+          }
+        }
+        *reinterpret_cast<uint2 *>(uplanes + p * kUPlane + u_prod[ch]) =
+            make_uint2(word[0], word[1]);
+      }
   };
 
   // ---- Products of step `step`: ring update from u_s[step % 2]; when the
@@ -1611,35 +1691,76 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? 2 : 1) void hyena_fir_mfma_st
   auto multiply = [&](auto rot, int step) __attribute__((always_inline)) {
     constexpr int kRot = decltype(rot)::value;
     const uint16_t *uplanes = &u_s[step & 1][0][0][0];
-    ring_hi[(kMsK - 1 + kRot) % kMsK] = *reinterpret_cast<const u32x4 *>(uplanes + u_ring);
-    ring_lo[(kMsK - 1 + kRot) % kMsK] =
-        *reinterpret_cast<const u32x4 *>(uplanes + kUPlane + u_ring);
+#pragma unroll
+    for (int p = 0; p < kUPlanes; ++p)
+      ring[p][(kMsK - 1 + kRot) % kMsK] =
+          *reinterpret_cast<const u32x4 *>(uplanes + p * kUPlane + u_ring);
     if (step < lead)
       return;
-    // Two independent accumulator chains, interleaved.
-    f32x4 accs[2] = {{0.0F, 0.0F, 0.0F, 0.0F}, {0.0F, 0.0F, 0.0F, 0.0F}};
+    // Two independent accumulator chains (per filter), interleaved.
+    f32x4 accs[2], accs2[2];
+#pragma unroll
+    for (int half = 0; half < 2; ++half)
+      accs[half] = accs2[half] = f32x4{0.0F, 0.0F, 0.0F, 0.0F};
 #pragma unroll
     for (int q = 0; q < kMsK; ++q)
 #pragma unroll
       for (int half = 0; half < 2; ++half) {
-        const bf16x8 t = __builtin_bit_cast(bf16x8, a[half][q]);
-        accs[half] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-            t, __builtin_bit_cast(bf16x8, ring_hi[(q + kRot) % kMsK]), accs[half], 0, 0, 0);
-        accs[half] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-            t, __builtin_bit_cast(bf16x8, ring_lo[(q + kRot) % kMsK]), accs[half], 0, 0, 0);
+        const bf16x8 t = __builtin_bit_cast(bf16x8, a[0][half][q]);
+#pragma unroll
+        for (int p = 0; p < kUPlanes; ++p)
+          accs[half] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              t, __builtin_bit_cast(bf16x8, ring[p][(q + kRot) % kMsK]), accs[half], 0, 0, 0);
+        if constexpr (kTwoGroups) {
+          const bf16x8 t2 = __builtin_bit_cast(bf16x8, a[kFilters - 1][half][q]);
+#pragma unroll
+          for (int p = 0; p < kUPlanes; ++p)
+            accs2[half] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                t2, __builtin_bit_cast(bf16x8, ring[p][(q + kRot) % kMsK]), accs2[half], 0, 0, 0);
+        }
       }
     float *xy = &xy_s[step % 3][0][0] + y_lane;
+    if constexpr (kTwoGroups) {
+      unsigned flags = 0U;
+#pragma unroll
+      for (int q = 0; q < kMsK; ++q)
+        flags |= flag_s[(step + 8 - q) % 8];
+      if (__builtin_expect(flags != 0U, 0)) {
+        const float *h = filter + (cw / group_size) * k;
+#pragma unroll 1
+        for (int i = 0; i < 8; ++i) {
+          const int r = 16 * (i >> 2) + (i & 3);
+          const long t = static_cast<long>(t_start) + step * kMsStep + r + 4 * g;
+          if (t < static_cast<long>(L))
+            xy[r * kMsChannels] *=
+                hcm_window_sum(P, short_history, short_filter, inner_history, h, k, causal, d, W,
+                               t, cw);
+        }
+        return;
+      }
+    }
 #pragma unroll
     for (int half = 0; half < 2; ++half) {
-      const f32x4 acc = accs[half];
-      const uint2 uhi = *reinterpret_cast<const uint2 *>(uplanes + u_epi[half]);
-      const uint2 ulo = *reinterpret_cast<const uint2 *>(uplanes + kUPlane + u_epi[half]);
-      const uint32_t hw[4] = {uhi.x << 16, uhi.x & 0xffff0000U, uhi.y << 16, uhi.y & 0xffff0000U};
-      const uint32_t lw[4] = {ulo.x << 16, ulo.x & 0xffff0000U, ulo.y << 16, ulo.y & 0xffff0000U};
+      f32x4 acc = accs[half];
+      if constexpr (kTwoGroups) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          acc[e] = second ? accs2[half][e] : acc[e];
+      }
+      uint2 up[kUPlanes];
+#pragma unroll
+      for (int p = 0; p < kUPlanes; ++p)
+        up[p] = *reinterpret_cast<const uint2 *>(uplanes + p * kUPlane + u_epi[half]);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const float total =
-            acc[e] + d * (__builtin_bit_cast(float, hw[e]) + __builtin_bit_cast(float, lw[e]));
+        float u = 0.0F;  // smallest plane first
+#pragma unroll
+        for (int p = kUPlanes - 1; p >= 0; --p) {
+          const uint32_t word = e < 2 ? up[p].x : up[p].y;
+          const float v = __builtin_bit_cast(float, e % 2 == 0 ? word << 16 : word & 0xffff0000U);
+          u = p == kUPlanes - 1 ? v : v + u;
+        }
+        const float total = acc[e] + d * u;
         xy[(16 * half + e) * kMsChannels] *= total;
       }
     }
@@ -1667,23 +1788,31 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? 2 : 1) void hyena_fir_mfma_st
   __syncthreads();
   if (dma_consts)
     d = direct_s[16 * wave + col];
+  if (kTwoGroups && history_flag) {
+    // The history's rows are steps -4 .. -1.
+#pragma unroll
+    for (int q = 4; q < 8; ++q)
+      atomicOr(&flag_s[q], 1U);
+  }
   // Keep d in a register: a load re-issued inside the step loop would make
   // the wait for it also wait for every DMA in flight.
   asm volatile("" : "+v"(d));
   // The taps are BF16 values, so T has no lo plane.
 #pragma unroll
-  for (int half = 0; half < 2; ++half)
+  for (int f = 0; f < kFilters; ++f)
 #pragma unroll
-    for (int q = 0; q < kMsK; ++q) {
-      uint16_t taps[8];
+    for (int half = 0; half < 2; ++half)
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int i = 32 * q + 8 * g + e;
-        const int o = i - 16 * half - col - 128 + (k - 1);  // -160 <= o < k + 31
-        taps[e] = f32_to_bf16(taps_s[kTapPad + (causal ? k - 1 - o : o)]);
+      for (int q = 0; q < kMsK; ++q) {
+        uint16_t taps[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const int i = 32 * q + 8 * g + e;
+          const int o = i - 16 * half - col - 128 + (k - 1);  // -160 <= o < k + 31
+          taps[e] = f32_to_bf16(taps_s[f][kTapPad + (causal ? k - 1 - o : o)]);
+        }
+        a[f][half][q] = __builtin_bit_cast(u32x4, taps);
       }
-      a[half][q] = __builtin_bit_cast(u32x4, taps);
-    }
   produce(0);
   wait_dma<0>();
   __syncthreads();
@@ -1701,6 +1830,8 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? 2 : 1) void hyena_fir_mfma_st
     if (step + 1 < steps)
       produce(step + 1);
     multiply(rot, step);
+    if (kTwoGroups && threadIdx.x == 0)
+      flag_s[(step + 2) % 8] = 0U;  // step - 6's, read by no phase any more
     if (step + 2 < steps)
       wait_dma<0>();
     __syncthreads();
@@ -2432,37 +2563,34 @@ __global__ __launch_bounds__(kHmThreads<O>, 1) void hcl_mfma_kernel(
   }
 }
 
-// Rewrites the inner (u) history with the last k-1 rows of [history ; u].
-// Runs after the main kernel and before the short history moves on.
+// Rewrites the inner (u) history with the last hist = k - 1 rows of u
+// (L >= hist), one block row per history row. Runs after the main kernel.
+// With shared rows (gridDim.y > hist, L >= hist + short_len - 1, so that no u
+// row reads the short history) the further block rows rewrite the short
+// history, one per row, three columns per thread: both caches in one launch
+// instead of two.
 template <typename T>
-__global__ void inner_history_kernel(const T *__restrict__ P,
-                                     const float *__restrict__ short_history,
+__global__ void inner_history_kernel(const T *__restrict__ P, float *short_history,
                                      const uint16_t *__restrict__ short_filter,
                                      int short_len, size_t L, size_t W, size_t planar,
-                                     float *inner_history, int hist) {
+                                     float *__restrict__ inner_history, int hist) {
   const size_t c = blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x;
   if (c >= W)
     return;
+  const size_t cols3 = 3 * W;
+  const int h = static_cast<int>(blockIdx.y);
+  if (h >= hist) {
+    const size_t row = L - (short_len - 1) + (h - hist);
+    for (size_t col = c; col < cols3; col += W)
+      short_history[static_cast<size_t>(h - hist) * cols3 + col] = load_act(P, row * cols3 + col);
+    return;
+  }
   float taps[3][kMaxShort];
   load_short_taps(short_filter, short_len, c, taps);
-  const size_t cols3 = 3 * W;
-  // With L >= hist every new row comes from u and rows are independent: one
-  // block row per history row. Otherwise rows shift in place, oldest first.
-  const int h_begin = gridDim.y > 1 ? static_cast<int>(blockIdx.y) : 0;
-  const int h_end = gridDim.y > 1 ? h_begin + 1 : hist;
-  for (int h = h_begin; h < h_end; ++h) {
-    const long source = static_cast<long>(h) + static_cast<long>(L);  // in [hist ; u]
-    float value;
-    if (source < hist) {
-      value = inner_history[static_cast<size_t>(source) * W + c];
-    } else {
-      const long t = source - hist;
-      float x2, u;
-      gates(P, short_history, taps, short_len, cols3, planar, t, c, &x2, &u);
-      value = u;
-    }
-    inner_history[static_cast<size_t>(h) * W + c] = value;
-  }
+  float x2, u;
+  gates(P, short_history, taps, short_len, cols3, planar,
+        static_cast<long>(h) + static_cast<long>(L) - hist, c, &x2, &u);
+  inner_history[static_cast<size_t>(h) * W + c] = u;
 }
 
 // Short continuation (L < hist): history <- last hist rows of [history ; u]
@@ -2674,16 +2802,19 @@ void launch_fir_stream_taps(const T *projection, const float *short_history,
     seg_len *= 2;
   const unsigned segments = ceil_div(length, seg_len);
   const dim3 grid(cblocks * segments), block(kStreamWaves * 64);
+  auto run = [&](auto direct_c, auto pair_c) {
+    hipLaunchKernelGGL((hyena_fir_stream_kernel<T, O, kWin, kTaps, decltype(direct_c)::value,
+                                                decltype(pair_c)::value>),
+                       grid, block, 0, stream, projection, short_history, wt.short_filter,
+                       short_len, inner_history, wt.inner_filter, group_size, k, causal, direct,
+                       length, width, cblocks, segments, seg_len, out);
+  };
   if (direct != nullptr)
-    hipLaunchKernelGGL((hyena_fir_stream_kernel<T, O, kWin, kTaps, true>), grid, block, 0, stream,
-                       projection, short_history, wt.short_filter, short_len, inner_history,
-                       wt.inner_filter, group_size, k, causal, direct, length, width, cblocks,
-                       segments, seg_len, out);
+    group_size % 2 == 0 ? run(std::true_type{}, std::false_type{})
+                        : run(std::true_type{}, std::true_type{});
   else
-    hipLaunchKernelGGL((hyena_fir_stream_kernel<T, O, kWin, kTaps, false>), grid, block, 0,
-                       stream, projection, short_history, wt.short_filter, short_len,
-                       inner_history, wt.inner_filter, group_size, k, causal, direct, length,
-                       width, cblocks, segments, seg_len, out);
+    group_size % 2 == 0 ? run(std::false_type{}, std::false_type{})
+                        : run(std::false_type{}, std::true_type{});
 }
 
 // Exact window widths for the 7B shape (short FIR 3, HCS 7 taps); other
@@ -2738,6 +2869,31 @@ Status launch_fir_mfma(const T *projection, const float *short_history,
                        fragments, group_size, k, causal, direct, length, width, planar, out);
   }
   return launch_status("hyena_fir_mfma_kernel");
+}
+
+// Rows per block of the HCM row stream: the length whose busiest CU walks the
+// fewest steps. A block walks its rows and, past the first segment, the
+// kMsLead steps before them, plus a prologue worth about four steps; a CU
+// that holds two blocks (`pairs`: BF16 projections and one filter group per
+// slice, 71 KB of LDS) takes 1.3 times as long for both as for one. Measured
+// (W = 4096, BF16, 301 / 611 / 1024 / 2049 rows): segments of 256 rows or,
+// under 256 blocks, no less: 31 / 32 / 19 / 45 us; this rule 27 / 30 / 18 /
+// 45. F32 at 1024 rows: 24 us with 256 rows (this rule), 33 with 128.
+unsigned ms_segment(unsigned channel_blocks, size_t length, bool pairs) {
+  unsigned best = kMsSegment;
+  double best_steps = 0.0;
+  for (unsigned rows = kMsSegment; rows >= static_cast<unsigned>(kMsMinSegment); rows /= 2) {
+    const double segments = std::ceil(static_cast<double>(length) / rows);
+    const double per_cu = std::ceil(channel_blocks * segments / 256.0);
+    const double walks = pairs ? std::floor(per_cu / 2) * 1.3 + std::fmod(per_cu, 2.0) : per_cu;
+    const double steps = walks * (std::min<double>(rows, length) / kMsStep + 4.0 +
+                                  (segments > 1 ? kMsLead : 0));
+    if (best_steps == 0.0 || steps < best_steps) {
+      best_steps = steps;
+      best = rows;
+    }
+  }
+  return best;
 }
 
 }  // namespace
@@ -2844,21 +3000,25 @@ Status hyena_forward(int kind, const T *projection, size_t length,
     const int causal = kind == kHyenaHcm ? 1 : 0;
     const float *direct = kind == kHyenaHcm ? wt.direct : nullptr;
     const size_t group_size = width / wt.groups;
-    if (k <= 8 && planar == 0 && width % 2 == 0 && group_size % 2 == 0) {
+    // (Odd group sizes only with the exact windows: in the padded ones an
+    // infinity would reach rows past the filter through a zero tap.)
+    if (k <= 8 && planar == 0 && width % 2 == 0 &&
+        (group_size % 2 == 0 || (short_len == 3 && k == 7))) {
       EVO_TRY((launch_fir_stream<T, O>(projection, short_history, wt, short_len, inner_history,
                                        group_size, k, causal, direct, length, width, out,
                                        stream)));
     } else if (wt.taps_bf16 && short_len == 3 && planar == 0 && width % kMsChannels == 0 &&
-               group_size % 16 == 0 && direct != nullptr) {
+               group_size >= 15 && direct != nullptr) {
       const unsigned cblocks = static_cast<unsigned>(width / kMsChannels);
-      unsigned seg_len = kMsSegment;
-      while (seg_len > kMsMinSegment && cblocks * ceil_div(length, seg_len) < kMsMinBlocks)
-        seg_len /= 2;
+      const bool two_groups = group_size % 16 != 0;
+      const unsigned seg_len = ms_segment(cblocks, length, sizeof(T) == 2 && !two_groups);
       const unsigned segments = ceil_div(length, seg_len);
-      hipLaunchKernelGGL((hyena_fir_mfma_stream_kernel<T, O>), dim3(cblocks * segments),
-                         dim3(256), 0, stream, projection, short_history, wt.short_filter,
-                         short_len, inner_history, wt.inner_filter, group_size, k, causal, direct,
-                         length, width, cblocks, segments, seg_len, out);
+      const auto kernel = two_groups ? hyena_fir_mfma_stream_kernel<T, O, true>
+                                     : hyena_fir_mfma_stream_kernel<T, O, false>;
+      hipLaunchKernelGGL(kernel, dim3(cblocks * segments), dim3(256), 0, stream, projection,
+                         short_history, wt.short_filter, short_len, inner_history,
+                         wt.inner_filter, group_size, k, causal, direct, length, width, cblocks,
+                         segments, seg_len, out);
       EVO_TRY(launch_status("hyena_fir_mfma_stream_kernel"));
     } else if (width % kChannels == 0 && group_size % 16 == 0) {
       const size_t steps = k <= 8 ? FirMfmaShape<8>::kSteps : FirMfmaShape<128>::kSteps;
@@ -2899,9 +3059,14 @@ Status hyena_forward(int kind, const T *projection, size_t length,
     EVO_TRY(launch_status("hyena_fir_kernel"));
     if (inner_history != nullptr && k > 1) {
       if (length >= static_cast<size_t>(k - 1)) {
-        hipLaunchKernelGGL(inner_history_kernel<T>, dim3(ceil_div(width, 256), k - 1),
+        const bool both = short_history != nullptr && short_len > 1 &&
+                          length >= static_cast<size_t>(k - 1 + short_len - 1);
+        hipLaunchKernelGGL(inner_history_kernel<T>,
+                           dim3(ceil_div(width, 256), k - 1 + (both ? short_len - 1 : 0)),
                            dim3(256), 0, stream, projection, short_history, wt.short_filter,
                            short_len, length, width, planar, inner_history, k - 1);
+        if (both)
+          return launch_status("inner_history_kernel");
       } else {
         const size_t lds = static_cast<size_t>(k - 1) * 64 * sizeof(float);  // <= 32.5 KB
         hipLaunchKernelGGL(inner_history_shift_kernel<T>, dim3(ceil_div(width, 64)), dim3(256),

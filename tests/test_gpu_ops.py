@@ -709,6 +709,69 @@ def test_hcm_stream_mfma_matches_oracle(inner_len, length, width, groups, dtype)
     assert rel_err(actual, expected) < 2e-5
 
 
+@pytest.mark.parametrize("kind,inner_len,groups,width", [
+    (N.HYENA_HCM, 128, 64, 960), (N.HYENA_HCM, 33, 4, 192), (N.HYENA_HCM, 128, 12, 192),
+    (N.HYENA_HCS, 7, 64, 960), (N.HYENA_HCS, 7, 2, 34)])
+@pytest.mark.parametrize("length", [2, 31, 129, 300, 1025])
+@pytest.mark.parametrize("dtype", [N.DTYPE_F32, N.DTYPE_SPLIT, N.DTYPE_BF16_F16])
+def test_hyena_group_sizes_off_16(kind, inner_len, groups, width, length, dtype):
+    """Filter groups whose size is no multiple of 16 (15 channels in the 1B
+    topology; 48, 16 and 17 here too): slices with two groups' filters. F32
+    output: u in three BF16 planes (2^-24) and F32 sums of 128 terms; the
+    16-bit outputs round once (2^-17, 2^-11)."""
+    case = hyena_case(length + width + inner_len, kind, length, width, groups=groups,
+                      inner_len=inner_len)
+    proj = case["projection"]
+    if dtype == N.DTYPE_BF16_F16:
+        proj = bf16_to_f32(bf16_bits(proj))
+    expected = hyena_oracle(kind, case, projection=proj)
+    actual = hyena_gpu(kind, case, dtype=dtype, projection=proj, bf16_taps=True)
+    bound = {N.DTYPE_F32: 2e-6, N.DTYPE_SPLIT: 1e-5, N.DTYPE_BF16_F16: 2.0 ** -11}[dtype]
+    if kind == N.HYENA_HCM and width // groups % 16 == 0:
+        bound = max(bound, 2e-5)  # one group per slice: u in two planes
+    assert rel_err(actual, expected) < bound
+
+
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan])
+@pytest.mark.parametrize("kind,inner_len", [(N.HYENA_HCM, 128), (N.HYENA_HCM, 33),
+                                            (N.HYENA_HCS, 7)])
+def test_hyena_group_size_15_keeps_infinities_local(kind, inner_len, value):
+    """An infinity or NaN in the projection reaches the rows its short FIR
+    and inner filter span, of its own channel, and no other."""
+    length, width = 400, 960
+    case = hyena_case(5, kind, length, width, groups=64, inner_len=inner_len)
+    proj = case["projection"].copy()
+    rows, channels = [150, 301], [17, 944]
+    for row, channel in zip(rows, channels):
+        proj[row, 3 * channel + 2] = value
+    with np.errstate(invalid="ignore"):
+        expected = hyena_oracle(kind, case, projection=proj)
+    actual = hyena_gpu(kind, case, projection=proj, bf16_taps=True)
+    finite = np.isfinite(expected)
+    for row, channel in zip(rows, channels):
+        assert finite[:row, channel].all() and not finite[row:row + 2, channel].any()
+    assert np.array_equal(np.isnan(actual), np.isnan(expected))
+    assert np.array_equal(actual[~finite], expected[~finite], equal_nan=True)
+    assert rel_err(actual[finite], expected[finite]) < 2e-6
+
+
+@pytest.mark.parametrize("kind,inner_len", [(N.HYENA_HCM, 128), (N.HYENA_HCS, 7)])
+@pytest.mark.parametrize("split", [1, 2, 7, 128, 129, 130, 131, 300])
+def test_hyena_group_size_15_continuation(kind, inner_len, split):
+    """Two calls through the caches equal one: prompts around the length from
+    which both histories are rewritten in one launch (k + 1 rows)."""
+    length, width = 460, 960
+    case = hyena_case(9, kind, length, width, groups=64, inner_len=inner_len)
+    whole = hyena_gpu(kind, case, bf16_taps=True)
+    caches = dict(short=zeros((2, 3 * width)), inner=zeros((inner_len - 1, width)))
+    parts = [hyena_gpu(kind, case, projection=case["projection"][:split], caches=caches,
+                       bf16_taps=True),
+             hyena_gpu(kind, case, projection=case["projection"][split:], caches=caches,
+                       bf16_taps=True)]
+    assert rel_err(np.concatenate(parts), whole) < 1e-6
+    assert np.array_equal(host(caches["short"]), case["projection"][-2:])
+
+
 @pytest.mark.parametrize("split", [1, 31, 32, 300, 1024, 1500])
 def test_hcm_stream_continuation(split):
     """Continuation through the caches with the streaming kernel: the first
