@@ -68,6 +68,18 @@ __device__ inline void wait_dma() {
   asm volatile("s_waitcnt vmcnt(%0)" :: "n"(kPending) : "memory");
 }
 
+// Waits until at most `later` (capped at kMax) steps of kPer DMAs are in flight.
+template <int kPer, int kMax> __device__ inline void wait_steps(int later) {
+  if constexpr (kMax <= 0) {
+    wait_dma<0>();
+  } else {
+    if (later >= kMax)
+      wait_dma<kPer * kMax>();
+    else
+      wait_steps<kPer, kMax - 1>(later);
+  }
+}
+
 // ---- GEMM tile order.
 // Linear tile of hardware block `id` among `total` blocks: consecutive ids
 // go to different XCDs, so id -> (xcd, slot) -> contiguous band per XCD.

@@ -27,6 +27,7 @@
 #include "common.hpp"
 #include "row_norm.hpp"
 #include "ops.hpp"
+#include "tile_cost.hpp"
 
 namespace evo::hip {
 namespace {
@@ -136,8 +137,9 @@ __global__ __launch_bounds__(256) void qgmma_exact_kernel(
     put(out, static_cast<size_t>(row) * N + col, round_bf16(acc * output_scale));
 }
 
-// MFMA path. Block 128 (M) x 192 (N) outputs, 4 waves as 2 (M) x 2 (N) of
-// 64 x 96 (2 x 3 MFMA 32x32 tiles); two blocks share a CU (80 KB of LDS
+// MFMA path. The tile of long chunks is 128 (M) x 192 (N) outputs, 4 waves as
+// 2 (M) x 2 (N) of 64 x 96 (2 x 3 MFMA 32x32 tiles), two stages (others:
+// kFp8Tiles); two blocks share a CU (80 KB of LDS
 // each), so two waves per SIMD and one block's barrier wait runs under the
 // other block's MFMAs; the 96 accumulators
 // per lane stay in VGPRs, so the E8M13 truncation after each promotion is
@@ -150,30 +152,40 @@ __global__ __launch_bounds__(256) void qgmma_exact_kernel(
 // hit 8 distinct bank groups; two stages alternate. A 1024-row projection
 // is 8 x 64 = 512 tiles: two per CU. Rows beyond M or N load a clamped
 // valid row and are never stored.
-constexpr int kBM = 128, kBN = 192, kBK = 128, kStages = 2;
-constexpr int kWaves = 4;
-constexpr int kStageBytes = (kBM + kBN) * kBK;            // 40 KB
-constexpr int kDmaPerWave = kStageBytes / 1024 / kWaves;  // 10
-constexpr size_t kMfmaLds = static_cast<size_t>(kStages) * kStageBytes;
+constexpr int kBK = 128;
+// Block tile kBM x kBN on kWM x kWN waves of kMI x kNJ MFMA tiles, K steps
+// staged kStages deep.
+template <int kBM_, int kBN_, int kWM_, int kWN_, int kStages_> struct Fp8Tile {
+  static constexpr int kBM = kBM_, kBN = kBN_, kWM = kWM_, kWN = kWN_, kStages = kStages_;
+  static constexpr int kWaves = kWM * kWN;
+  static constexpr int kMI = kBM / 32 / kWM, kNJ = kBN / 32 / kWN;
+  static constexpr int kStageBytes = (kBM + kBN) * kBK;
+  static constexpr int kDmaPerWave = kStageBytes / 1024 / kWaves;
+  static constexpr size_t kLds = static_cast<size_t>(kStages) * kStageBytes;
+  static_assert(kStageBytes % (1024 * kWaves) == 0 && kLds <= 80 * 1024, "two blocks per CU");
+};
 
 __device__ inline int fp8_unit(int row, int unit) { return row * 8 + (unit ^ ((row >> 1) & 7)); }
 
-template <int kChunk, typename Out>
-__global__ __launch_bounds__(kWaves * 64, 2) void fp8_mfma_kernel(
+template <typename T, int kChunk, typename Out>
+__global__ __launch_bounds__(T::kWaves * 64, 2) void fp8_mfma_kernel(
     const uint8_t *__restrict__ a, const uint8_t *__restrict__ w,
     Out *__restrict__ out, int M, int N, int K, float output_scale) {
+  constexpr int kBM = T::kBM, kBN = T::kBN, kStages = T::kStages, kMI = T::kMI, kNJ = T::kNJ;
+  constexpr int kStageBytes = T::kStageBytes, kDmaPerWave = T::kDmaPerWave;
+  constexpr int kTiles = kMI * kNJ;  // per wave; tile t = (t / kNJ, t % kNJ)
   extern __shared__ __attribute__((aligned(16))) uint8_t fp8_lds[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int half = lane >> 5, col = lane & 31;
-  const int wave_m = wave >> 1, wave_n = wave & 1;  // 2 x 2
+  const int wave_m = wave / T::kWN, wave_n = wave % T::kWN;
   const int tiles_m = (M + kBM - 1) / kBM, tiles_n = (N + kBN - 1) / kBN;
   int tm, tn;
   tile_of(blockIdx.x, tiles_m, tiles_n, &tm, &tn);
   const int block_m = tm * kBM, block_n = tn * kBN;
 
-  // DMA op g = wave*10 + i: 1 KB chunk g of the stage (chunks 0..15 = A rows
-  // 8g.., 16..39 = W rows 8(g-16)..); lane l fills unit 64 g' + l. Each op
+  // DMA op g = wave * kDmaPerWave + i: 1 KB chunk g of the stage (the first
+  // kBM / 8 chunks are A rows, 8 per chunk, then W rows); lane l fills unit l. Each op
   // reads from a wave-uniform base (the block's first A or W row, advanced
   // by the step's K offset) plus a fixed 32-bit per-lane offset.
   const uint8_t *a_base = a + static_cast<size_t>(block_m) * K;
@@ -202,11 +214,11 @@ __global__ __launch_bounds__(kWaves * 64, 2) void fp8_mfma_kernel(
       dma16((from_a[i] ? a_base : w_base) + k0, src[i], stage + dst[i]);
   };
 
-  f32x16 acc[2][3];
+  f32x16 acc[kMI][kNJ];
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < kMI; ++i)
 #pragma unroll
-    for (int j = 0; j < 3; ++j)
+    for (int j = 0; j < kNJ; ++j)
 #pragma unroll
       for (int e = 0; e < 16; ++e)
         acc[i][j][e] = 0.0F;
@@ -218,9 +230,12 @@ __global__ __launch_bounds__(kWaves * 64, 2) void fp8_mfma_kernel(
   };
 
   const int steps = K / kBK;
-  issue(0);
+#pragma unroll
+  for (int s = 0; s + 1 < kStages; ++s)
+    if (s < steps)
+      issue(s);
   for (int s = 0; s < steps; ++s) {
-    wait_dma<0>();
+    wait_steps<kDmaPerWave, kStages - 2>(steps - 1 - s);
     // Every wave's DMA of step s has landed and every wave has left the
     // buffer of step s-1, which the next issue overwrites.
     __syncthreads();
@@ -228,37 +243,37 @@ __global__ __launch_bounds__(kWaves * 64, 2) void fp8_mfma_kernel(
     const uint8_t *w_s = a_s + kBM * kBK;
     if constexpr (kChunk == 128) {
       // Two K=64 MFMAs per tile, then one promotion (truncation) per 128 K.
-      i32x8 av[2][2], bv[2][3];
+      i32x8 av[2][kMI], bv[2][kNJ];
 #pragma unroll
       for (int ks = 0; ks < 2; ++ks) {
 #pragma unroll
-        for (int j = 0; j < 3; ++j)
-          bv[ks][j] = frag32(w_s, wave_n * 96 + j * 32 + col, ks * 4 + half * 2);
+        for (int j = 0; j < kNJ; ++j)
+          bv[ks][j] = frag32(w_s, (wave_n * kNJ + j) * 32 + col, ks * 4 + half * 2);
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
-          av[ks][i] = frag32(a_s, wave_m * 64 + i * 32 + col, ks * 4 + half * 2);
+        for (int i = 0; i < kMI; ++i)
+          av[ks][i] = frag32(a_s, (wave_m * kMI + i) * 32 + col, ks * 4 + half * 2);
       }
       // The next step's DMA (into the buffer of step s-1, which every wave
       // has left) goes out behind the fragment reads and ahead of the MFMAs:
       // placed between the two K halves instead it measured 3 % slower
       // (config 3: 54.5 -> 56 us; M = 8192: 420 -> 435 us, bit-identical).
-      if (s + 1 < steps)
-        issue(s + 1);
+      if (s + kStages - 1 < steps)
+        issue(s + kStages - 1);
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
+      for (int i = 0; i < kMI; ++i)
 #pragma unroll
-        for (int j = 0; j < 3; ++j)
+        for (int j = 0; j < kNJ; ++j)
           acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(
               av[0][i], bv[0][j], acc[i][j], 0, 0, 0, 127, 0, 127);
       // Second K half: each tile's promotion runs while the next tile's
       // MFMA executes (only the last tile's truncation is left at the end).
 #pragma unroll
-      for (int t = 0; t < 6; ++t) {
-        const int i = t / 3, j = t % 3;
+      for (int t = 0; t < kTiles; ++t) {
+        const int i = t / kNJ, j = t % kNJ;
         acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(
             av[1][i], bv[1][j], acc[i][j], 0, 0, 0, 127, 0, 127);
         if (t > 0) {
-          const int pi = (t - 1) / 3, pj = (t - 1) % 3;
+          const int pi = (t - 1) / kNJ, pj = (t - 1) % kNJ;
 #pragma unroll
           for (int e = 0; e < 16; ++e)
             acc[pi][pj][e] = truncate_e8m13(acc[pi][pj][e]);
@@ -266,7 +281,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void fp8_mfma_kernel(
       }
 #pragma unroll
       for (int e = 0; e < 16; ++e)
-        acc[1][2][e] = truncate_e8m13(acc[1][2][e]);
+        acc[kMI - 1][kNJ - 1][e] = truncate_e8m13(acc[kMI - 1][kNJ - 1][e]);
     } else {
       // Four 32-K chunks, each two K=16 MFMAs per tile then a promotion.
       // A tile's promotion is issued right behind the next tile's second
@@ -282,39 +297,39 @@ __global__ __launch_bounds__(kWaves * 64, 2) void fp8_mfma_kernel(
         // banks): the chunk's first MFMA takes codes 0-7 of each half, the
         // second codes 8-15. A and W are split the same way, so the chunk
         // still sums exactly its 32 products before the promotion.
-        long bv[2][3], av[2][2];
+        long bv[2][kNJ], av[2][kMI];
 #pragma unroll
-        for (int j = 0; j < 3; ++j) {
-          const int row = wave_n * 96 + j * 32 + col;
+        for (int j = 0; j < kNJ; ++j) {
+          const int row = (wave_n * kNJ + j) * 32 + col;
           const uint4 v = *reinterpret_cast<const uint4 *>(w_s + fp8_unit(row, 2 * c + half) * 16);
           bv[0][j] = static_cast<long>((static_cast<unsigned long>(v.y) << 32) | v.x);
           bv[1][j] = static_cast<long>((static_cast<unsigned long>(v.w) << 32) | v.z);
         }
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          const int row = wave_m * 64 + i * 32 + col;
+        for (int i = 0; i < kMI; ++i) {
+          const int row = (wave_m * kMI + i) * 32 + col;
           const uint4 v = *reinterpret_cast<const uint4 *>(a_s + fp8_unit(row, 2 * c + half) * 16);
           av[0][i] = static_cast<long>((static_cast<unsigned long>(v.y) << 32) | v.x);
           av[1][i] = static_cast<long>((static_cast<unsigned long>(v.w) << 32) | v.z);
         }
 #pragma unroll
-        for (int t = 0; t < 6; ++t) {
-          if (t == 5) {  // truncating the initial zeros is harmless
+        for (int t = 0; t < kTiles; ++t) {
+          if (t == kTiles - 1) {  // truncating the initial zeros is harmless
 #pragma unroll
             for (int e = 0; e < 16; ++e)
-              acc[1][2][e] = truncate_e8m13(acc[1][2][e]);
+              acc[kMI - 1][kNJ - 1][e] = truncate_e8m13(acc[kMI - 1][kNJ - 1][e]);
           }
-          acc[t / 3][t % 3] = __builtin_amdgcn_mfma_f32_32x32x16_fp8_fp8(
-              av[0][t / 3], bv[0][t % 3], acc[t / 3][t % 3], 0, 0, 0);
+          acc[t / kNJ][t % kNJ] = __builtin_amdgcn_mfma_f32_32x32x16_fp8_fp8(
+              av[0][t / kNJ], bv[0][t % kNJ], acc[t / kNJ][t % kNJ], 0, 0, 0);
         }
-        if (c == 0 && s + 1 < steps)
-          issue(s + 1);  // the next step's DMA, after the first chunk's reads
+        if (c == 0 && s + kStages - 1 < steps)
+          issue(s + kStages - 1);  // after the first chunk's reads
 #pragma unroll
-        for (int t = 0; t < 6; ++t) {
-          acc[t / 3][t % 3] = __builtin_amdgcn_mfma_f32_32x32x16_fp8_fp8(
-              av[1][t / 3], bv[1][t % 3], acc[t / 3][t % 3], 0, 0, 0);
+        for (int t = 0; t < kTiles; ++t) {
+          acc[t / kNJ][t % kNJ] = __builtin_amdgcn_mfma_f32_32x32x16_fp8_fp8(
+              av[1][t / kNJ], bv[1][t % kNJ], acc[t / kNJ][t % kNJ], 0, 0, 0);
           if (t > 0) {
-            const int pi = (t - 1) / 3, pj = (t - 1) % 3;
+            const int pi = (t - 1) / kNJ, pj = (t - 1) % kNJ;
 #pragma unroll
             for (int e = 0; e < 16; ++e)
               acc[pi][pj][e] = truncate_e8m13(acc[pi][pj][e]);
@@ -327,7 +342,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void fp8_mfma_kernel(
     // The last chunk's deferred promotion of the last tile.
 #pragma unroll
     for (int e = 0; e < 16; ++e)
-      acc[1][2][e] = truncate_e8m13(acc[1][2][e]);
+      acc[kMI - 1][kNJ - 1][e] = truncate_e8m13(acc[kMI - 1][kNJ - 1][e]);
   }
   if constexpr (std::is_same<Out, uint16_t>::value) {
     if (N % 2 == 0 && reinterpret_cast<uintptr_t>(out) % 4 == 0) {
@@ -337,18 +352,18 @@ __global__ __launch_bounds__(kWaves * 64, 2) void fp8_mfma_kernel(
       // two values.
       const bool even = (col & 1) == 0;
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
+      for (int i = 0; i < kMI; ++i)
 #pragma unroll
         for (int e = 0; e < 16; e += 2) {
-          const int row = block_m + wave_m * 64 + i * 32 + (e >> 2) * 8 + half * 4 + (e & 3);
+          const int row = block_m + (wave_m * kMI + i) * 32 + (e >> 2) * 8 + half * 4 + (e & 3);
 #pragma unroll
-          for (int j = 0; j < 3; ++j) {
+          for (int j = 0; j < kNJ; ++j) {
             const uint32_t first = f32_to_bf16(round_bf16(acc[i][j][e] * output_scale));
             const uint32_t second = f32_to_bf16(round_bf16(acc[i][j][e + 1] * output_scale));
             const uint32_t other = static_cast<uint32_t>(__shfl_xor(
                 static_cast<int>(even ? second : first), 1, 64));
             const int out_row = even ? row : row + 1;
-            const int column = block_n + wave_n * 96 + j * 32 + (col & ~1);
+            const int column = block_n + (wave_n * kNJ + j) * 32 + (col & ~1);
             if (out_row < M && column < N)
               *reinterpret_cast<uint32_t *>(out + static_cast<size_t>(out_row) * N + column) =
                   even ? (first | (other << 16)) : (other | (second << 16));
@@ -358,15 +373,15 @@ __global__ __launch_bounds__(kWaves * 64, 2) void fp8_mfma_kernel(
     }
   }
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < kMI; ++i)
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
-      const int row = block_m + wave_m * 64 + i * 32 + (e >> 2) * 8 + half * 4 + (e & 3);
+      const int row = block_m + (wave_m * kMI + i) * 32 + (e >> 2) * 8 + half * 4 + (e & 3);
       if (row >= M)
         continue;
 #pragma unroll
-      for (int j = 0; j < 3; ++j) {
-        const int column = block_n + wave_n * 96 + j * 32 + col;
+      for (int j = 0; j < kNJ; ++j) {
+        const int column = block_n + (wave_n * kNJ + j) * 32 + col;
         if (column < N)
           put(out, static_cast<size_t>(row) * N + column,
               round_bf16(acc[i][j][e] * output_scale));
@@ -495,6 +510,43 @@ __global__ __launch_bounds__(256) void fp8_gemv_kernel(
   put(out, static_cast<size_t>(m) * N + row, round_bf16(acc * output_scale));
 }
 
+// Block tiles of the MFMA path and their measured cost (least-squares fits
+// over 5 to 8192 rows of the two topologies' projections; the tile the fit
+// picks is within 1 % of the fastest there). 128 x 192 is the tile of long
+// chunks; a prompt of a few hundred rows or less fills the chip, and streams
+// the weight near the copy rate, only on smaller ones, whose deeper stages
+// keep as many bytes in flight. Every tile gives the same bits. Measured at
+// W = 4096, K128: 16 rows 38 -> 13 us, 64 rows 39 -> 14.5, 200 rows 39.8 ->
+// 26.5, 300 rows 39 -> 28, 1000 rows 54 (128 x 192); K32: 200 rows 52 -> 34.
+struct Fp8TileEntry {
+  int bm, bn;
+  TileCost k128, k32;
+};
+constexpr Fp8TileEntry kFp8Tiles[] = {
+    {128, 192, {0.85F, 0.81F, 0.113F, 2, {1.131F, 1.413F}}, {5.50F, 0.35F, 0.099F, 2, {1.404F, 2.248F}}},
+    {96, 128, {0.44F, 0.0F, 0.047F, 2, {0.901F, 0.931F}}, {3.00F, 0.89F, 0.086F, 2, {0.912F, 1.163F}}},
+    {64, 128, {2.39F, 0.0F, 0.013F, 2, {0.551F, 0.717F}}, {3.72F, 0.14F, 0.048F, 2, {0.633F, 0.876F}}},
+    {64, 64, {2.23F, 1.10F, 0.0F, 2, {0.327F, 0.436F}}, {2.27F, 1.19F, 0.0F, 2, {0.438F, 0.554F}}},
+    {32, 128, {2.14F, 0.38F, 0.0F, 2, {0.362F, 0.516F}}, {2.26F, 1.09F, 0.0F, 2, {0.462F, 0.600F}}},
+    {32, 64, {2.23F, 1.20F, 0.0F, 2, {0.285F, 0.369F}}, {2.27F, 1.21F, 0.0F, 2, {0.428F, 0.499F}}},
+};
+
+int choose_fp8_tile(size_t M, size_t N, size_t K, bool k32) {
+  int best = 0;
+  double best_us = 0.0;
+  for (int t = 0; t < static_cast<int>(sizeof(kFp8Tiles) / sizeof(kFp8Tiles[0])); ++t) {
+    const Fp8TileEntry &e = kFp8Tiles[t];
+    const double us = tile_us(k32 ? e.k32 : e.k128,
+                              static_cast<double>(ceil_div(M, e.bm)) * ceil_div(N, e.bn),
+                              static_cast<double>(K / kBK), static_cast<double>(N) * K);
+    if (t == 0 || us < best_us) {
+      best = t;
+      best_us = us;
+    }
+  }
+  return best;
+}
+
 unsigned elementwise_grid(size_t n) {
   const size_t blocks = (n + 255) / 256;
   return static_cast<unsigned>(blocks < 16384 ? blocks : 16384);
@@ -578,17 +630,28 @@ Status fp8_linear_impl(const uint8_t *in_codes, const uint8_t *w_codes, Out *out
                        output_scale, folded, code_scale);
     return launch_status("fp8_gemv_kernel");
   }
-  const auto kernel = mode == kFp8MfmaK32 ? fp8_mfma_kernel<32, Out> : fp8_mfma_kernel<128, Out>;
-  // 80 KB of the CU's 160 KB LDS (two blocks per CU): opt in above the
-  // 64 KB default.
-  EVO_TRY(hip_status(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
-                                         hipFuncAttributeMaxDynamicSharedMemorySize,
-                                         static_cast<int>(kMfmaLds)),
-                     "fp8_mfma_kernel LDS opt-in"));
-  const unsigned blocks = static_cast<unsigned>(ceil_div(M, kBM) * ceil_div(N, kBN));
-  hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kWaves * 64), kMfmaLds, stream, in_codes, w_codes, out,
-                     m, n, k, output_scale);
-  return launch_status("fp8_mfma_kernel");
+  auto launch = [&](auto tile) -> Status {
+    using T = decltype(tile);
+    const auto kernel =
+        mode == kFp8MfmaK32 ? fp8_mfma_kernel<T, 32, Out> : fp8_mfma_kernel<T, 128, Out>;
+    if (T::kLds > 64 * 1024)  // opt in above the 64 KB default
+      EVO_TRY(hip_status(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize,
+                                             static_cast<int>(T::kLds)),
+                         "fp8_mfma_kernel LDS opt-in"));
+    const unsigned blocks = ceil_div(M, T::kBM) * ceil_div(N, T::kBN);
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(T::kWaves * 64), T::kLds, stream, in_codes,
+                       w_codes, out, m, n, k, output_scale);
+    return launch_status("fp8_mfma_kernel");
+  };
+  switch (choose_fp8_tile(M, N, K, mode == kFp8MfmaK32)) {
+  case 1: return launch(Fp8Tile<96, 128, 1, 4, 2>{});
+  case 2: return launch(Fp8Tile<64, 128, 2, 2, 3>{});
+  case 3: return launch(Fp8Tile<64, 64, 2, 2, 5>{});
+  case 4: return launch(Fp8Tile<32, 128, 1, 4, 4>{});
+  case 5: return launch(Fp8Tile<32, 64, 1, 2, 5>{});
+  default: return launch(Fp8Tile<128, 192, 2, 2, 2>{});
+  }
 }
 
 Status fp8_linear(const uint8_t *in_codes, const uint8_t *w_codes, float *out,

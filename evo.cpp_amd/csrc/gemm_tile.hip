@@ -24,12 +24,12 @@
 //     406 -> 89, 1000 rows 428 -> 157 (floor 18)
 //   N = K = 1920: 61 rows 79 -> 8 us, 1000 rows 88 -> 22.
 #include <algorithm>
-#include <cmath>
 #include <type_traits>
 
 #include "common.hpp"
 #include "gemm_epilogue.hpp"
 #include "gemm_tile.hpp"
+#include "tile_cost.hpp"
 
 namespace evo::hip {
 namespace {
@@ -48,18 +48,6 @@ struct TileShape {
 // logical unit (a fragment's rows) fall on 16 distinct 16-byte bank groups.
 template <int kUnits> __device__ inline int tile_unit(int row, int unit) {
   return row * kUnits + (unit ^ (kUnits == 8 ? ((row >> 1) & 7) : (row & 15)));
-}
-
-// Waits until at most `later` (capped at kMax) steps of kPer DMAs are in flight.
-template <int kPer, int kMax> __device__ inline void wait_steps(int later) {
-  if constexpr (kMax <= 0) {
-    wait_dma<0>();
-  } else {
-    if (later >= kMax)
-      wait_dma<kPer * kMax>();
-    else
-      wait_steps<kPer, kMax - 1>(later);
-  }
 }
 
 template <typename T, bool kSplit, bool kF16>
@@ -294,15 +282,6 @@ template <typename T> Status launch_planes(const TileCall &c, hipStream_t stream
   return c.f16 ? launch<T, false, true>(c, stream) : launch<T, false, false>(c, stream);
 }
 
-// Measured time of a launch on one tile, in us: launch + rounds * (epilogue +
-// steps * step) + load * steps * blocks / 256, where a round fills every CU
-// with `slots` blocks (step[r - 1]: a K step of a CU's r blocks) and `load` is
-// what a step slows down by as the whole chip fills.
-struct TileCost {
-  float launch, epilogue, load;
-  int slots;
-  float step[3];
-};
 struct TileEntry {
   int bm, bn, seg;
   TileCost split, plane;  // hi + lo activation planes, one plane
@@ -327,19 +306,10 @@ constexpr int kTileCount = static_cast<int>(sizeof(kTiles) / sizeof(kTiles[0]));
 constexpr TileEntry kLargeTile = {256, 256, 32, {0.0F, 9.34F, 0.294F, 1, {1.094F}},
                                   {0.0F, 9.14F, 0.165F, 1, {0.737F}}};
 
-double tile_us(const TileEntry &t, bool split, size_t M, size_t N, size_t K, size_t parts) {
-  const TileCost &c = split ? t.split : t.plane;
-  const double blocks = static_cast<double>(ceil_div(M, t.bm)) * ceil_div(N, t.bn) * parts;
-  const double steps = ceil_div(K / parts, t.seg);
-  const double per_round = 256.0 * c.slots;
-  const double rounds = std::floor(blocks / per_round);
-  const int rest = static_cast<int>(std::ceil((blocks - rounds * per_round) / 256.0));
-  double us = c.launch + rounds * (c.epilogue + steps * c.step[c.slots - 1]) +
-              c.load * steps * blocks / 256.0;
-  if (rest > 0)
-    us += c.epilogue + steps * c.step[rest - 1];
-  // The weights from HBM at the measured copy rate (5 TB/s).
-  return std::max(us, 3.0 + 2.0 * static_cast<double>(N) * K / 5.0e6);
+double entry_us(const TileEntry &t, bool split, size_t M, size_t N, size_t K, size_t parts) {
+  return tile_us(split ? t.split : t.plane,
+                 static_cast<double>(ceil_div(M, t.bm)) * ceil_div(N, t.bn) * parts,
+                 ceil_div(K / parts, t.seg), 2.0 * static_cast<double>(N) * K);
 }
 
 }  // namespace
@@ -353,7 +323,7 @@ TileChoice choose_gemm_tile(size_t M, size_t N, size_t K, bool split, bool gated
                       : (deferred ? 0.0 : 3.0) + 4.0 * static_cast<double>(parts) * M * N / 4.0e6;
   };
   TileChoice best;
-  double best_us = tile_us(kLargeTile, split, M, N, K, large_parts) + reduction(large_parts);
+  double best_us = entry_us(kLargeTile, split, M, N, K, large_parts) + reduction(large_parts);
   for (int t = 0; t < kTileCount; ++t) {
     const size_t seg = static_cast<size_t>(kTiles[t].seg);
     if (gated && kTiles[t].bn % 32 != 0)
@@ -364,7 +334,7 @@ TileChoice choose_gemm_tile(size_t M, size_t N, size_t K, bool split, bool gated
       if (parts > 1 && (K / parts < 4 * seg || N % 4 != 0 || gated ||
                         parts * M * N * sizeof(float) > workspace_bytes))
         continue;
-      const double us = tile_us(kTiles[t], split, M, N, K, parts) + reduction(parts);
+      const double us = entry_us(kTiles[t], split, M, N, K, parts) + reduction(parts);
       if (us < best_us) {
         best_us = us;
         best = TileChoice{t, static_cast<int>(parts)};
