@@ -15,10 +15,15 @@
 // Reference semantics: `src/cpu/model.cpp:510-544` (full softmax; the online
 // form below equals it up to F32 rounding).
 //
-// MFMA kernel (head_dim 32/64/128): one block = 8 waves x 32 queries of one
-// head (two waves per SIMD share each K/V tile). K [64 keys][d] and V^T [d][64 keys] tiles of both
-// planes are DMA'd (global_load_lds) into XOR-swizzled LDS, double buffered,
-// so the next tile streams in while this one computes. Each wave computes
+// MFMA kernel (head_dim 32/64/128): one block = 8 or 4 waves x 32 queries of
+// one head, over all of its keys or, with a workspace, a part of them
+// (plan_flash; flash_combine_kernel joins the parts). K [32 keys][d] and V^T
+// [d][32 keys] tiles of both planes are DMA'd (global_load_lds) into
+// XOR-swizzled LDS, double buffered, so the next tile streams in while this
+// one computes. 8192 x 4096 and 4096 x 4096 on a prefix of 28672 take 1350 and
+// 4850 us (64-key tiles, per-lane DMA addresses and fragment reads right
+// before their MFMAs: 1530 and 5150); the matrix cores run at 1.3 PFLOP/s of
+// three-pass work there, near what random operands sustain. Each wave computes
 // S^T = K Q^T (keys x queries) with v_mfma_f32_32x32x16_bf16, so every lane
 // owns one query: the running max and sum stay in-lane (plus one exchange
 // with the lane holding the other half of the keys), and P^T is already in
@@ -28,6 +33,9 @@
 // head_dim 16 uses a VALU kernel (four lanes per query).
 #include "common.hpp"
 #include "ops.hpp"
+
+#include <algorithm>
+#include <cmath>
 
 namespace evo::hip {
 
@@ -158,9 +166,9 @@ __global__ __launch_bounds__(256) void v_transpose_kernel(
 }
 
 // ------------------------------------------------------------ MFMA kernel
+constexpr int kKeys = 64;            // cache capacity granule
 constexpr int kQueriesPerWave = 32;
-constexpr int kKeys = 64;
-constexpr int kFlashWaves = 8;  // waves (query groups of 32) sharing a K/V tile
+constexpr int kTileKeys = 32;        // keys of a K/V tile
 
 // Swizzle of a row of kUnits 16-byte units: 8 consecutive rows read at one
 // logical unit hit 8 distinct 16-byte bank groups.
@@ -169,49 +177,93 @@ __device__ inline int swizzle(int row, int unit) {
   return unit ^ ((row * kUnits / 16) & (kUnits - 1));
 }
 
-template <int kD, int kFlashWaves = kFlashWaves>
+template <int kD, int kWaves>
 struct FlashShape {
+  static constexpr int kQueries = kWaves * kQueriesPerWave;
   static constexpr int kKUnits = kD / 8;             // 16-byte units per K row
-  static constexpr int kKPlane = kKeys * kD;         // BF16 per K plane
-  static constexpr int kVPlane = kD * kKeys;         // BF16 per V^T plane
-  static constexpr int kStage = 2 * kKPlane + 2 * kVPlane;
+  static constexpr int kVUnits = kTileKeys / 8;      // and per V^T row
+  static constexpr int kPlane = kTileKeys * kD;      // BF16 per K or V^T plane
+  static constexpr int kStage = 4 * kPlane;          // {K hi, K lo, V hi, V lo}
   static constexpr size_t kLdsBytes = 2 * kStage * sizeof(uint16_t);
-  static constexpr int kChunksPerPlane = kD / 8;     // 1 KB chunks per K or V^T plane
-  static constexpr int kDmaPerWave = 4 * kChunksPerPlane / kFlashWaves;
+  static constexpr int kChunksPerPlane = kPlane / 512;  // 1 KB chunks
+  static constexpr int kDmaPerWave = 4 * kChunksPerPlane / kWaves;
+  static_assert(4 * kChunksPerPlane % kWaves == 0, "DMA split");
 };
 
-template <int kD, typename O, int kFlashWaves = kFlashWaves>
-__global__ __launch_bounds__(kFlashWaves * 64) void flash_attention_kernel(
+// Key split of a launch: query block qb of T key tiles runs as
+// ceil(T / chunk_tiles) blocks over equal parts of its tiles (at most
+// max_chunks), each leaving its unnormalised output, running maximum (log2
+// domain) and sum in `part` for flash_combine_kernel; a query block of one
+// part writes its output itself. max_chunks == 1: no split.
+struct KeySplit {
+  uint32_t chunk_tiles, max_chunks;
+  float *part;  // [heads][query blocks][max_chunks][kQueries][kD + 2]
+};
+__device__ inline uint32_t key_chunks(const KeySplit &split, uint32_t tiles) {
+  return split.max_chunks == 1 ? 1 : (tiles + split.chunk_tiles - 1) / split.chunk_tiles;
+}
+__device__ inline uint32_t key_tiles(size_t prefix, size_t rows, size_t block_row, int queries) {
+  const size_t last = min(rows, block_row + queries) - 1;
+  return static_cast<uint32_t>((prefix + last) / kTileKeys + 1);
+}
+
+// Order of kGroups groups of {two LDS fragment reads, three MFMAs on them}
+// between the surrounding scheduling barriers: the reads run kAhead groups
+// ahead of the MFMAs that use them. (Left to itself the compiler reads each
+// pair right before its MFMAs and waits out the LDS latency every time.)
+template <int kGroups, int kAhead, int kReadGroups> __device__ inline void schedule_reads_ahead() {
+  if (kAhead > 0)
+    __builtin_amdgcn_sched_group_barrier(0x100, 2 * kAhead, 0);
+#pragma unroll
+  for (int i = 0; i < kGroups; ++i) {
+    if (i + kAhead < kReadGroups)
+      __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+    __builtin_amdgcn_sched_group_barrier(0x008, 3, 0);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+// kWide: V^T row offsets within a DMA need more than 32 bits (2^27 positions).
+template <int kD, typename O, int kWaves, bool kWide>
+__global__ __launch_bounds__(kWaves * 64, 2) void flash_attention_kernel(
     const uint16_t *__restrict__ q, size_t q_plane, const uint16_t *__restrict__ k_cache,
     const uint16_t *__restrict__ vt_cache, size_t cache_plane, size_t capacity, size_t rows,
-    size_t prefix, size_t heads, O out) {
-  using Shape = FlashShape<kD, kFlashWaves>;
+    size_t prefix, size_t heads, const KeySplit split, O out) {
+  using Shape = FlashShape<kD, kWaves>;
   constexpr int kDSteps = kD / 16;  // K-steps of S^T over head_dim
   constexpr int kDTiles = kD / 32;  // 32-row tiles of O^T
   extern __shared__ __attribute__((aligned(16))) uint16_t flash_lds[];
 
   const size_t width = heads * kD;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int half = lane >> 5, col = lane & 31;
-  // Block -> (head, query block): heaviest (latest) query blocks first; with
-  // heads % 8 == 0 the blocks of a head share an XCD (blocks are dealt to
-  // the 8 XCDs round-robin), so its K/V tiles are reused from one L2.
-  constexpr int kBlockQueries = kFlashWaves * kQueriesPerWave;
-  const size_t query_blocks = (rows + kBlockQueries - 1) / kBlockQueries;
+  // Block -> (head, query block, key chunk): heaviest (latest) query blocks
+  // first; with heads % 8 == 0 the blocks of a head share an XCD (blocks are
+  // dealt to the 8 XCDs round-robin), so its K/V tiles are reused from one L2.
+  const size_t query_blocks = (rows + Shape::kQueries - 1) / Shape::kQueries;
   const size_t b = blockIdx.x;
-  size_t head, qb;
+  size_t head, rest;
   if (heads % 8 == 0) {
     const size_t per_xcd = heads / 8, idx = b / 8;
     head = (b % 8) + 8 * (idx % per_xcd);
-    qb = query_blocks - 1 - idx / per_xcd;
+    rest = idx / per_xcd;
   } else {
     head = b % heads;
-    qb = query_blocks - 1 - b / heads;
+    rest = b / heads;
   }
-  const size_t block_row = qb * kBlockQueries;
+  const size_t qb = query_blocks - 1 - rest / split.max_chunks;
+  const uint32_t chunk = static_cast<uint32_t>(rest % split.max_chunks);
+  const size_t block_row = qb * Shape::kQueries;
+  const uint32_t all_tiles = key_tiles(prefix, rows, block_row, Shape::kQueries);
+  const uint32_t chunks = key_chunks(split, all_tiles);
+  if (chunk >= chunks)
+    return;
+  const uint32_t first_tile = static_cast<uint32_t>(static_cast<uint64_t>(all_tiles) * chunk / chunks);
+  const uint32_t end_tile =
+      static_cast<uint32_t>(static_cast<uint64_t>(all_tiles) * (chunk + 1) / chunks);
   const size_t row = block_row + wave * kQueriesPerWave + col;  // this lane's query
   const bool active = row < rows;
-  const size_t position = prefix + row;
   // exp(x * scale) = exp2(x * scale * log2(e))
   const float scale2 = 1.4426950408889634F / sqrtf(static_cast<float>(kD));
 
@@ -231,35 +283,46 @@ __global__ __launch_bounds__(kFlashWaves * 64) void flash_attention_kernel(
     }
   }
 
-  // Per-lane DMA sources of tile 0 (op g of this wave: part g / kChunksPerPlane
-  // of {K hi, K lo, V hi, V lo}, 1 KB chunk g % kChunksPerPlane of that plane).
-  const uint16_t *src[Shape::kDmaPerWave];
-  int dst[Shape::kDmaPerWave];
+  // DMA op g of this wave: part g / kChunksPerPlane of {K hi, K lo, V hi, V
+  // lo}, 1 KB chunk g % kChunksPerPlane of that plane: a wave-uniform base
+  // that advances with the tile, a fixed 32-bit byte offset per lane and a
+  // wave-uniform LDS address (per-lane 64-bit sources and generic LDS
+  // pointers cost ~10 instructions per DMA, ahead of each tile's first MFMA).
+  const char *base[Shape::kDmaPerWave];
+  uint32_t offset[Shape::kDmaPerWave];
 #pragma unroll
   for (int i = 0; i < Shape::kDmaPerWave; ++i) {
     const int g = wave * Shape::kDmaPerWave + i;
-    const int part = g / Shape::kChunksPerPlane, chunk = g % Shape::kChunksPerPlane;
-    const int flat = chunk * 64 + lane;  // 16-byte unit within the plane
+    const int part = g / Shape::kChunksPerPlane, first = (g % Shape::kChunksPerPlane) * 64;
+    const size_t plane = (part & 1) != 0 ? cache_plane : 0;
     if (part < 2) {
-      const int key = flat / Shape::kKUnits, unit = swizzle<Shape::kKUnits>(key, flat % Shape::kKUnits);
-      src[i] = k_cache + (part == 1 ? cache_plane : 0) + static_cast<size_t>(key) * width +
-               head * kD + unit * 8;
-      dst[i] = part * Shape::kKPlane + chunk * 512;
+      const int key = (first + lane) / Shape::kKUnits;
+      const int unit = swizzle<Shape::kKUnits>(key, (first + lane) % Shape::kKUnits);
+      base[i] = reinterpret_cast<const char *>(k_cache + plane + head * kD);
+      offset[i] = static_cast<uint32_t>(key * width + unit * 8) * 2;
     } else {
-      const int d = flat / 8, unit = swizzle<8>(d, flat % 8);
-      src[i] = vt_cache + (part == 3 ? cache_plane : 0) +
-               (head * kD + d) * capacity + unit * 8;
-      dst[i] = 2 * Shape::kKPlane + (part - 2) * Shape::kVPlane + chunk * 512;
+      // 64 lanes cover 16 rows of V^T: the first one's goes into the base.
+      const int d = (first + lane) / Shape::kVUnits, d0 = first / Shape::kVUnits;
+      const int unit = swizzle<Shape::kVUnits>(d, lane % Shape::kVUnits);
+      base[i] = reinterpret_cast<const char *>(vt_cache + plane + (head * kD + d0) * capacity);
+      offset[i] = static_cast<uint32_t>((d - d0) * capacity + unit * 8) * 2;
     }
   }
-  auto issue = [&](size_t tile) {
-    uint16_t *stage = flash_lds + (tile & 1) * Shape::kStage;
-    const size_t k0 = tile * kKeys;
+  const unsigned lds = lds_address(flash_lds);
+  auto issue = [&](uint32_t tile) {
+    const size_t k0 = static_cast<size_t>(tile) * kTileKeys;
 #pragma unroll
     for (int i = 0; i < Shape::kDmaPerWave; ++i) {
-      const int g = wave * Shape::kDmaPerWave + i;
-      const bool is_k = g / Shape::kChunksPerPlane < 2;
-      dma16(src[i] + (is_k ? k0 * width : k0), stage + dst[i]);
+      const bool is_k = (wave * Shape::kDmaPerWave + i) / Shape::kChunksPerPlane < 2;
+      const unsigned to = wave * Shape::kDmaPerWave * 1024 + (tile & 1) * (Shape::kStage * 2) +
+                          i * 1024;
+      const char *from = base[i] + (is_k ? k0 * width : k0) * 2;
+      if (kWide && !is_k) {
+        const size_t down = (lane / Shape::kVUnits) * capacity * 2;
+        dma16(from + down + (offset[i] - static_cast<uint32_t>(down)), flash_lds + to / 2);
+      } else {
+        dma16_at(from, offset[i], lds + to);
+      }
     }
   };
 
@@ -271,57 +334,65 @@ __global__ __launch_bounds__(kFlashWaves * 64) void flash_attention_kernel(
       o_acc[t][e] = 0.0F;
   float running_max = -INFINITY, partial_sum = 0.0F;
 
-  const size_t last_row = min(rows, block_row + kBlockQueries) - 1;
-  const size_t tiles = (prefix + last_row + 1 + kKeys - 1) / kKeys;
-  const size_t wave_first = prefix + block_row + wave * kQueriesPerWave;  // lowest position
-  issue(0);
-  for (size_t tile = 0; tile < tiles; ++tile) {
+  // Lowest position of the wave's queries, and whether it has any.
+  const size_t wave_first = prefix + block_row + wave * kQueriesPerWave;
+  const bool wave_rows = block_row + wave * kQueriesPerWave < rows;
+  issue(first_tile);
+  for (uint32_t tile = first_tile; tile < end_tile; ++tile) {
     // This wave's DMA of the tile (the only one in flight), then one
     // barrier: every wave's DMA of the tile has landed and every wave has
     // left buffer (tile+1)&1 (tile-1's), which the next DMA overwrites.
     wait_dma<0>();
     __syncthreads();
-    if (tile + 1 < tiles)
+    if (tile + 1 < end_tile)
       issue(tile + 1);
+    const size_t k0 = static_cast<size_t>(tile) * kTileKeys;
+    // Every key of the tile lies beyond every query of the wave.
+    if (!wave_rows || k0 > wave_first + (kQueriesPerWave - 1))
+      continue;
     const uint16_t *stage = flash_lds + (tile & 1) * Shape::kStage;
-    const uint16_t *k_hi = stage, *k_lo = stage + Shape::kKPlane;
-    const uint16_t *v_hi = stage + 2 * Shape::kKPlane, *v_lo = v_hi + Shape::kVPlane;
-    const size_t k0 = tile * kKeys;
+    const uint16_t *k_hi = stage, *k_lo = stage + Shape::kPlane;
+    const uint16_t *v_hi = stage + 2 * Shape::kPlane, *v_lo = v_hi + Shape::kPlane;
 
-    // S^T tiles: st[kt] holds keys kt*32 + (e/4)*8 + half*4 + e%4 for query col.
-    f32x16 st[2];
+    // S^T: entry e holds key (e/4)*8 + half*4 + e%4 of the tile for query col.
+    f32x16 st;
 #pragma unroll
-    for (int kt = 0; kt < 2; ++kt) {
+    for (int e = 0; e < 16; ++e)
+      st[e] = 0.0F;
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int s = 0; s < kDSteps; ++s) {
+      const int off = (col * Shape::kKUnits + swizzle<Shape::kKUnits>(col, 2 * s + half)) * 8;
+      const bf16x8 kh = *reinterpret_cast<const bf16x8 *>(k_hi + off);
+      const bf16x8 kl = *reinterpret_cast<const bf16x8 *>(k_lo + off);
+      st = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kh, qh[s], st, 0, 0, 0);
+      st = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kh, ql[s], st, 0, 0, 0);
+      st = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kl, qh[s], st, 0, 0, 0);
+    }
+    schedule_reads_ahead<kDSteps, kDSteps < 2 ? kDSteps : 2, kDSteps>();
+    // Causal mask on the diagonal tiles, tile maximum (log2 domain: the
+    // scale is positive, so it commutes with the maximum).
+    if (k0 + kTileKeys - 1 > wave_first) {
+      // Keys from the tile's first up to this query's position.
+      const int visible = static_cast<int>(wave_first - k0) + col;
 #pragma unroll
       for (int e = 0; e < 16; ++e)
-        st[kt][e] = 0.0F;
-      const int key = kt * 32 + col;
-#pragma unroll
-      for (int s = 0; s < kDSteps; ++s) {
-        const int off = (key * Shape::kKUnits + swizzle<Shape::kKUnits>(key, 2 * s + half)) * 8;
-        const bf16x8 kh = *reinterpret_cast<const bf16x8 *>(k_hi + off);
-        const bf16x8 kl = *reinterpret_cast<const bf16x8 *>(k_lo + off);
-        st[kt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kh, qh[s], st[kt], 0, 0, 0);
-        st[kt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kh, ql[s], st[kt], 0, 0, 0);
-        st[kt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kl, qh[s], st[kt], 0, 0, 0);
-      }
+        st[e] = (e >> 2) * 8 + half * 4 + (e & 3) <= visible ? st[e] : -INFINITY;
     }
-    // Scale (log2 domain), causal mask on the diagonal tiles, tile maximum.
+    auto read_v = [&](int kk, int t, bf16x8 &vh, bf16x8 &vl) {
+      const int d = t * 32 + col;
+      const int off = (d * Shape::kVUnits + swizzle<Shape::kVUnits>(d, 2 * kk + half)) * 8;
+      vh = *reinterpret_cast<const bf16x8 *>(v_hi + off);
+      vl = *reinterpret_cast<const bf16x8 *>(v_lo + off);
+    };
+    // The first V^T fragments arrive under the softmax.
+    bf16x8 vh, vl;
+    read_v(0, 0, vh, vl);
     float tile_max = -INFINITY;
-    const bool diagonal = k0 + kKeys - 1 > wave_first;
 #pragma unroll
-    for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        float value = st[kt][e] * scale2;
-        if (diagonal) {
-          const size_t key = k0 + kt * 32 + (e >> 2) * 8 + half * 4 + (e & 3);
-          value = key <= position ? value : -INFINITY;
-        }
-        st[kt][e] = value;
-        tile_max = fmaxf(tile_max, value);
-      }
-    tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 32, 64));
+    for (int e = 0; e < 16; ++e)
+      tile_max = fmaxf(tile_max, st[e]);
+    tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 32, 64)) * scale2;
     const float new_max = fmaxf(running_max, tile_max);
     if (__any(new_max != running_max)) {
       // A query with no visible key yet keeps new_max = -inf: nothing to scale.
@@ -335,38 +406,60 @@ __global__ __launch_bounds__(kFlashWaves * 64) void flash_attention_kernel(
           o_acc[t][e] *= correction;
       running_max = new_max;
     }
-    const float base = new_max == -INFINITY ? 0.0F : new_max;
-    // P = exp2(S - max) as B operands; with the permuted V^T key order, the
-    // 8 entries e0..e0+7 of this lane are the 8 consecutive V^T columns of
-    // 16-key step kk at half*8.
+    const float base_max = new_max == -INFINITY ? 0.0F : new_max;
+    // P = exp2(S * scale - max) as B operands; with the permuted V^T key
+    // order, the 8 entries e0..e0+7 of this lane are the 8 consecutive V^T
+    // columns of 16-key step kk at half*8.
 #pragma unroll
-    for (int kk = 0; kk < 4; ++kk) {
-      const int kt = kk >> 1, e0 = (kk & 1) * 8;
+    for (int kk = 0; kk < 2; ++kk) {
       bf16x8 ph, pl;
 #pragma unroll
       for (int slot = 0; slot < 8; ++slot) {
-        const float p = __builtin_amdgcn_exp2f(st[kt][e0 + slot] - base);
+        const float p = __builtin_amdgcn_exp2f(fmaf(st[kk * 8 + slot], scale2, -base_max));
         partial_sum += p;
         const __bf16 h = static_cast<__bf16>(p);
         ph[slot] = h;
         pl[slot] = static_cast<__bf16>(p - static_cast<float>(h));
       }
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int t = 0; t < kDTiles; ++t) {
-        const int d = t * 32 + col;
-        const int off = (d * 8 + swizzle<8>(d, 2 * kk + half)) * 8;
-        const bf16x8 vh = *reinterpret_cast<const bf16x8 *>(v_hi + off);
-        const bf16x8 vl = *reinterpret_cast<const bf16x8 *>(v_lo + off);
+        bf16x8 next_h = vh, next_l = vl;
+        if (t + 1 < kDTiles)
+          read_v(kk, t + 1, next_h, next_l);
+        else if (kk == 0)
+          read_v(1, 0, next_h, next_l);
         o_acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vh, ph, o_acc[t], 0, 0, 0);
         o_acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vh, pl, o_acc[t], 0, 0, 0);
         o_acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vl, ph, o_acc[t], 0, 0, 0);
+        vh = next_h;
+        vl = next_l;
       }
+      if (kk == 0)
+        schedule_reads_ahead<kDTiles, 0, kDTiles>();
+      else
+        schedule_reads_ahead<kDTiles, 0, kDTiles - 1>();
     }
   }
   const float total = partial_sum + __shfl_xor(partial_sum, 32, 64);
   if (!active)
     return;
   // O^T entry e of tile t: d = t*32 + (e/4)*8 + half*4 + e%4, query = col.
+  if (chunks > 1) {
+    float *dst = split.part + (((head * query_blocks + qb) * split.max_chunks + chunk) *
+                                   Shape::kQueries + wave * kQueriesPerWave + col) * (kD + 2);
+    if (half == 0) {
+      dst[0] = running_max;
+      dst[1] = total;
+    }
+#pragma unroll
+    for (int t = 0; t < kDTiles; ++t)
+#pragma unroll
+      for (int e = 0; e < 16; e += 2)
+        *reinterpret_cast<float2 *>(dst + 2 + t * 32 + (e >> 2) * 8 + half * 4 + (e & 3)) =
+            make_float2(o_acc[t][e], o_acc[t][e + 1]);
+    return;
+  }
 #pragma unroll
   for (int t = 0; t < kDTiles; ++t)
 #pragma unroll
@@ -374,6 +467,46 @@ __global__ __launch_bounds__(kFlashWaves * 64) void flash_attention_kernel(
       const int d = t * 32 + (e >> 2) * 8 + half * 4 + (e & 3);
       put(out, row * width + head * kD + d, o_acc[t][e] / total);
     }
+}
+
+// Rows of split query blocks: the chunks rescaled to their common maximum and
+// summed in chunk order. One wave per (row, head), two dims per lane (kD / 2
+// lanes).
+template <int kD, typename O, int kWaves>
+__global__ __launch_bounds__(256) void flash_combine_kernel(size_t rows, size_t prefix,
+                                                            size_t heads, const KeySplit split,
+                                                            O out) {
+  using Shape = FlashShape<kD, kWaves>;
+  const size_t index = blockIdx.x * 4ULL + (threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const size_t row = index / heads, head = index % heads;
+  if (row >= rows || lane >= kD / 2)
+    return;
+  const size_t query_blocks = (rows + Shape::kQueries - 1) / Shape::kQueries;
+  const size_t qb = row / Shape::kQueries;
+  const uint32_t chunks =
+      key_chunks(split, key_tiles(prefix, rows, qb * Shape::kQueries, Shape::kQueries));
+  if (chunks == 1)
+    return;
+  const float *src = split.part + ((head * query_blocks + qb) * split.max_chunks * Shape::kQueries +
+                                   row % Shape::kQueries) * (kD + 2);
+  constexpr size_t kStep = Shape::kQueries * (kD + 2);  // chunk to chunk
+  float top = -INFINITY;
+  for (uint32_t c = 0; c < chunks; ++c)
+    top = fmaxf(top, src[c * kStep]);
+  float sum = 0.0F, o0 = 0.0F, o1 = 0.0F;
+  for (uint32_t c = 0; c < chunks; ++c) {
+    // (A chunk whose keys all lie beyond the query has maximum -inf, sum 0.)
+    const float m = src[c * kStep];
+    const float scale = m == -INFINITY ? 0.0F : __builtin_amdgcn_exp2f(m - top);
+    const float2 o = *reinterpret_cast<const float2 *>(src + c * kStep + 2 + 2 * lane);
+    sum = fmaf(src[c * kStep + 1], scale, sum);
+    o0 = fmaf(o.x, scale, o0);
+    o1 = fmaf(o.y, scale, o1);
+  }
+  const size_t at = row * heads * kD + head * kD + 2 * lane;
+  put(out, at, o0 / sum);
+  put(out, at + 1, o1 / sum);
 }
 
 // ------------------------------------------------------------ VALU kernel
@@ -453,30 +586,122 @@ __global__ __launch_bounds__(256) void attention_kernel(
   }
 }
 
+// Block size and key split of a launch: the plan of least fitted time (us,
+// head_dim 128, 130 (rows, prefix, heads) from 5 x 0 to 4096 x 28000; the
+// plan it picks is within 6 % of the fastest one there). Blocks of 8 waves
+// (256 queries, one per CU) need 1.67 us per 32-key tile of the longest one,
+// blocks of 4 waves (128 queries) 1.36, or 2.11 when two share a CU; a full
+// chip 2.63 / 1.60 us per tile and CU; keys and values come from HBM at
+// 5 TB/s; a split costs its second launch and its partials' bytes. Few
+// queries on a long prefix leave most CUs idle without a split (64 rows,
+// prefix 8000, 32 heads: 390 -> 59 us), and so do the last query blocks of a
+// prompt (1500 rows, 15 heads: 94 -> 52 us); chunks of a few thousand rows
+// and more fill the chip and stay unsplit.
+struct FlashPlan {
+  int waves;
+  uint32_t chunk_tiles, max_chunks;
+};
+double flash_plan_us(size_t rows, size_t prefix, size_t heads, size_t head_dim,
+                     const FlashPlan &plan, size_t *part_bytes) {
+  const size_t queries = static_cast<size_t>(plan.waves) * kQueriesPerWave;
+  const size_t query_blocks = (rows + queries - 1) / queries;
+  double total = 0.0, longest = 0.0, items = 0.0, parts = 0.0;
+  for (size_t qb = 0; qb < query_blocks; ++qb) {
+    const size_t last = std::min(rows, (qb + 1) * queries) - 1;
+    const double tiles = static_cast<double>((prefix + last) / kTileKeys + 1);
+    const double chunks = plan.max_chunks == 1 ? 1.0 : std::ceil(tiles / plan.chunk_tiles);
+    total += tiles;
+    items += chunks;
+    longest = std::max(longest, std::ceil(tiles / chunks));
+    parts += chunks > 1.0 ? chunks : 0.0;
+  }
+  const double heads_d = static_cast<double>(heads);
+  total *= heads_d;
+  items *= heads_d;
+  const double row_bytes = static_cast<double>((head_dim + 2) * sizeof(float));
+  *part_bytes = query_blocks * heads * plan.max_chunks * queries * (head_dim + 2) * sizeof(float);
+  double us, fill;
+  if (plan.waves == 8) {
+    us = longest * 1.67;
+    fill = total / 256.0 * 2.63 + (items > 256.0 ? 0.31 * us : 0.0);
+  } else {
+    us = longest * (items > 256.0 ? 2.11 : 1.36);
+    fill = total / 256.0 * 1.60 + (items > 512.0 ? 0.08 * longest : 0.0);
+  }
+  const double key_bytes = 8.0 * static_cast<double>(prefix + rows) * heads_d * head_dim;
+  us = std::max({us, fill, key_bytes / 5.0e6}) + 6.0;
+  if (plan.max_chunks > 1)
+    us += 2.7 + 2.0 * parts * heads_d * queries * row_bytes / 4.3e6;
+  return us;
+}
+FlashPlan plan_flash(size_t rows, size_t prefix, size_t heads, size_t head_dim,
+                     size_t workspace_bytes) {
+  FlashPlan best{8, 0, 1};
+  size_t part_bytes = 0;
+  double best_us = flash_plan_us(rows, prefix, heads, head_dim, best, &part_bytes);
+  auto consider = [&](const FlashPlan &plan) {
+    const double us = flash_plan_us(rows, prefix, heads, head_dim, plan, &part_bytes);
+    if (us < best_us && (plan.max_chunks == 1 || part_bytes <= workspace_bytes)) {
+      best_us = us;
+      best = plan;
+    }
+  };
+  consider(FlashPlan{4, 0, 1});
+  // Two and more rounds of the larger blocks: nothing idle to fill.
+  if (workspace_bytes == 0 || ceil_div(rows, 8 * kQueriesPerWave) * heads >= 768)
+    return best;
+  const size_t tiles = (prefix + rows - 1) / kTileKeys + 1;
+  for (uint32_t chunk : {8U, 12U, 16U, 24U, 32U, 48U, 64U, 96U, 128U, 192U, 256U, 384U, 768U,
+                         1536U}) {
+    const size_t chunks = (tiles + chunk - 1) / chunk;
+    if (chunks < 2 || chunks > 64)
+      continue;
+    consider(FlashPlan{4, chunk, static_cast<uint32_t>(chunks)});
+    consider(FlashPlan{8, chunk, static_cast<uint32_t>(chunks)});
+  }
+  return best;
+}
+
+template <int kD, typename O, int kWaves>
+Status launch_flash_waves(const uint16_t *q, size_t q_plane, const uint16_t *k_cache,
+                          const uint16_t *v_cache, size_t cache_plane, size_t capacity,
+                          size_t rows, size_t prefix, size_t heads, const KeySplit &split, O out,
+                          hipStream_t stream) {
+  using Shape = FlashShape<kD, kWaves>;
+  static_assert(Shape::kLdsBytes <= 64 * 1024, "default LDS limit, two blocks per CU");
+  const size_t blocks = ceil_div(rows, Shape::kQueries) * heads * split.max_chunks;
+  if (blocks > (1U << 31))
+    return {ErrorCode::kInvalidArgument, "causal_attention: grid too large"};
+  const auto kernel = capacity < (size_t{1} << 27)
+                          ? flash_attention_kernel<kD, O, kWaves, false>
+                          : flash_attention_kernel<kD, O, kWaves, true>;
+  hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(kWaves * 64),
+                     Shape::kLdsBytes, stream, q, q_plane, k_cache, v_cache, cache_plane,
+                     capacity, rows, prefix, heads, split, out);
+  EVO_TRY(launch_status("flash_attention_kernel"));
+  if (split.max_chunks == 1)
+    return Status::Ok();
+  hipLaunchKernelGGL((flash_combine_kernel<kD, O, kWaves>), dim3(ceil_div(rows * heads, 4)),
+                     dim3(256), 0, stream, rows, prefix, heads, split, out);
+  return launch_status("flash_combine_kernel");
+}
+
 template <int kD, typename O>
 Status launch_flash(const uint16_t *q, size_t q_plane, const uint16_t *k_cache,
                     const uint16_t *v_cache, size_t cache_plane, size_t capacity, size_t rows,
-                    size_t prefix, size_t heads, O out, hipStream_t stream) {
-  constexpr size_t lds = FlashShape<kD>::kLdsBytes;
-  static_assert(lds <= 160 * 1024, "LDS");
-  // Blocks of 8 waves share each K/V tile among 256 queries; when that
-  // leaves CUs idle (short chunks: 1024 rows x 32 heads = 128 blocks), blocks
-  // of 4 waves (128 queries) fill twice as many.
-  const bool half = ceil_div(rows, kFlashWaves * kQueriesPerWave) * heads < 256;
-  const int waves = half ? kFlashWaves / 2 : kFlashWaves;
-  auto kernel = half ? flash_attention_kernel<kD, O, kFlashWaves / 2>
-                     : flash_attention_kernel<kD, O, kFlashWaves>;
-  EVO_TRY(hip_status(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
-                                         hipFuncAttributeMaxDynamicSharedMemorySize,
-                                         static_cast<int>(lds)),
-                     "flash_attention_kernel LDS opt-in"));
-  const size_t blocks = ceil_div(rows, static_cast<size_t>(waves) * kQueriesPerWave) * heads;
-  hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(waves * 64), lds, stream,
-                     q, q_plane, k_cache, v_cache, cache_plane, capacity, rows, prefix, heads,
-                     out);
-  return launch_status("flash_attention_kernel");
+                    size_t prefix, size_t heads, float *workspace, size_t workspace_bytes, O out,
+                    hipStream_t stream) {
+  // The parts are stored as float2.
+  const bool usable = workspace != nullptr &&
+                      reinterpret_cast<uintptr_t>(workspace) % sizeof(float2) == 0;
+  const FlashPlan plan = plan_flash(rows, prefix, heads, kD, usable ? workspace_bytes : 0);
+  const KeySplit split{plan.chunk_tiles, plan.max_chunks, workspace};
+  if (plan.waves == 4)
+    return launch_flash_waves<kD, O, 4>(q, q_plane, k_cache, v_cache, cache_plane, capacity, rows,
+                                        prefix, heads, split, out, stream);
+  return launch_flash_waves<kD, O, 8>(q, q_plane, k_cache, v_cache, cache_plane, capacity, rows,
+                                      prefix, heads, split, out, stream);
 }
-
 
 // ---- Single-query (decode) attention, split over the keys: one block per
 // (head, chunk of 256 keys). Each lane scores one key (F32 dot of q with
@@ -620,8 +845,8 @@ Status launch_decode(const uint16_t *q, size_t q_plane, const uint16_t *k_cache,
 template <typename O>
 Status launch_attention(const uint16_t *q, size_t q_plane, const uint16_t *k_cache,
                         const uint16_t *v_cache, size_t cache_plane, size_t capacity,
-                        size_t rows, size_t prefix, size_t heads, size_t head_dim, O out,
-                        hipStream_t stream) {
+                        size_t rows, size_t prefix, size_t heads, size_t head_dim,
+                        float *workspace, size_t workspace_bytes, O out, hipStream_t stream) {
   switch (head_dim) {
   case 16:
     hipLaunchKernelGGL((attention_kernel<16, O>), dim3(ceil_div(rows, 64), heads), dim3(256),
@@ -630,13 +855,13 @@ Status launch_attention(const uint16_t *q, size_t q_plane, const uint16_t *k_cac
     return launch_status("attention_kernel");
   case 32:
     return launch_flash<32, O>(q, q_plane, k_cache, v_cache, cache_plane, capacity, rows,
-                               prefix, heads, out, stream);
+                               prefix, heads, workspace, workspace_bytes, out, stream);
   case 64:
     return launch_flash<64, O>(q, q_plane, k_cache, v_cache, cache_plane, capacity, rows,
-                               prefix, heads, out, stream);
+                               prefix, heads, workspace, workspace_bytes, out, stream);
   case 128:
     return launch_flash<128, O>(q, q_plane, k_cache, v_cache, cache_plane, capacity, rows,
-                                prefix, heads, out, stream);
+                               prefix, heads, workspace, workspace_bytes, out, stream);
   default:
     return {ErrorCode::kUnsupported,
             "causal_attention: head_dim must be 16, 32, 64 or 128"};
@@ -707,12 +932,12 @@ Status causal_attention(const uint16_t *q, size_t q_plane, const uint16_t *k_cac
   }
   if (out_f32 != nullptr)
     return launch_attention(q, q_plane, k_cache, v_cache, cache_plane, capacity, rows, prefix,
-                            heads, head_dim, out_f32, stream);
+                            heads, head_dim, workspace, workspace_bytes, out_f32, stream);
   if (out_f16)
     return launch_attention(q, q_plane, k_cache, v_cache, cache_plane, capacity, rows, prefix,
-                            heads, head_dim, F16Plane{out_hi}, stream);
-  return launch_attention(q, q_plane, k_cache, v_cache, cache_plane, capacity, rows, prefix,
-                          heads, head_dim, SplitOut{out_hi, out_lo}, stream);
+                            heads, head_dim, workspace, workspace_bytes, F16Plane{out_hi}, stream);
+  return launch_attention(q, q_plane, k_cache, v_cache, cache_plane, capacity, rows, prefix, heads,
+                          head_dim, workspace, workspace_bytes, SplitOut{out_hi, out_lo}, stream);
 }
 
 }  // namespace evo::hip

@@ -63,6 +63,16 @@ __device__ inline void dma16(const void *base, uint32_t offset, const void *lds)
                :: "v"(offset), "s"(base), "s"(address) : "memory");
 }
 
+// The same DMA to an LDS byte address held in a wave-uniform register: no
+// per-lane pointer, conversion or readfirstlane per instruction.
+__device__ inline unsigned lds_address(const void *lds) {
+  return static_cast<unsigned>(reinterpret_cast<size_t>((const lds_void *)(lds)));
+}
+__device__ inline void dma16_at(const void *base, uint32_t offset, unsigned lds) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+               :: "v"(offset), "s"(base), "s"(lds) : "memory");
+}
+
 template <int kPending>
 __device__ inline void wait_dma() {
   asm volatile("s_waitcnt vmcnt(%0)" :: "n"(kPending) : "memory");

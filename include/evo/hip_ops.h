@@ -253,7 +253,10 @@ EVO_API evo_status evo_hip_attention(const float *projected, size_t rows,
 /* evo_hip_attention with an F32 device workspace: a single query (rows == 1,
  * head_dim 32/64/128) is then split over its keys in chunks of 256 (per
  * chunk and head: max, sum and head_dim partial outputs in the workspace),
- * the decode step's path. The same reference interface. */
+ * the decode step's path; and a few rows, or the last rows of a prompt, over
+ * parts of their keys where the workspace holds the parts (rows x heads x
+ * parts x (head_dim + 2) floats) and that is faster. The same reference
+ * interface. */
 EVO_API evo_status evo_hip_attention_ws(const float *projected, size_t rows,
                                         size_t width, size_t heads,
                                         int column_split, const float *inv_freq,

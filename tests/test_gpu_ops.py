@@ -927,6 +927,84 @@ def test_single_query_attention_split_over_keys(oracle, heads, head_dim, prefix)
     assert rel_err(results[0], results[1]) < 1e-5
 
 
+@pytest.mark.parametrize("heads,head_dim,rows,prefix", [
+    (2, 128, 2, 3000), (3, 64, 64, 2031), (8, 32, 33, 1500), (2, 128, 300, 700),
+    (4, 128, 1000, 0), (3, 128, 257, 255), (16, 64, 128, 4000)])
+def test_attention_split_over_keys(oracle, heads, head_dim, rows, prefix):
+    """Several queries with a workspace: query blocks run as parts of their
+    keys and the parts are combined. Against the oracle and the call without a
+    workspace in the root mean square: values, keys and probabilities are two
+    BF16 terms each (2^-17 of them, of either sign), and averaging over keys
+    shrinks the sum's terms as it shrinks the sum, so 2^-16 of the output. A
+    workspace below two parts falls back; the caches are appended as without
+    one."""
+    r = rng(prefix + heads + head_dim + rows)
+    width, total = heads * head_dim, prefix + rows
+    proj = r.standard_normal((total, 3 * width)).astype(np.float32)
+    inv_freq = (1.0 / 10000 ** (np.arange(0, head_dim, 2) / head_dim)).astype(np.float32)
+    qkv = proj.reshape(total, heads, 3, head_dim)
+    q, k, v = (np.ascontiguousarray(qkv[:, :, i]).reshape(-1) for i in range(3))
+    O.check(oracle.oracle_apply_rope(O.ptr(q), O.ptr(k), total, heads, head_dim,
+                                     O.ptr(inv_freq), 0, 8.0))
+    expected = np.zeros_like(q)
+    O.check(oracle.oracle_causal_attention(O.ptr(q), O.ptr(k), O.ptr(v), total, heads,
+                                           head_dim, O.ptr(expected)))
+    expected = expected.reshape(total, width)[prefix:]
+    capacity = (total + 63) // 64 * 64
+    part = -(-rows // 128) * 128 * heads * (head_dim + 2)
+    outs, caches = [], []
+    for floats in (64 * 2 * part, 2 * part - 1, 0):
+        kc, vc = zeros((2, capacity, width), np.uint16), zeros((2, width, capacity), np.uint16)
+        query, out = empty((2, total, width), np.uint16), empty((total, width))
+        if prefix:
+            N.call("evo_hip_attention", p(dev(proj[:prefix])), prefix, width, heads, 1,
+                   p(dev(inv_freq)), 8.0, 0, p(query), p(kc), p(vc), capacity, p(out), stream())
+        workspace = empty((max(floats, 1) + 64,))
+        workspace.fill_(7.0)
+        out.fill_(7.0)
+        N.call("evo_hip_attention_ws", p(dev(proj[prefix:])), rows, width, heads, 1,
+               p(dev(inv_freq)), 8.0, prefix, p(query), p(kc), p(vc), capacity, p(out),
+               p(workspace), floats * 4, stream())
+        assert np.all(host(workspace)[floats:] == 7.0)
+        assert np.all(host(out)[rows:] == 7.0)
+        outs.append(host(out)[:rows].copy())
+        caches.append((host(kc), host(vc)))
+    for other in (expected.astype(np.float64), outs[2].astype(np.float64)):
+        assert np.linalg.norm(outs[0] - other) < 2.0**-16 * np.linalg.norm(other)
+    assert np.array_equal(outs[1], outs[2])
+    for kc, vc in caches[1:]:
+        assert np.array_equal(kc, caches[0][0]) and np.array_equal(vc, caches[0][1])
+
+
+@pytest.mark.parametrize("value", [np.inf, np.nan])
+def test_attention_split_keeps_non_finite_rows(value):
+    """A non-finite value at one position of one head reaches that head's
+    queries from there on, split over the keys or not, and nothing else."""
+    heads, head_dim, rows = 4, 128, 700
+    width = heads * head_dim
+    r = rng(8)
+    proj = r.standard_normal((rows, heads, 3, head_dim)).astype(np.float32)
+    proj[450, 2, 2, 5] = value
+    inv_freq = dev(np.ones(head_dim // 2, np.float32))
+    masks = []
+    for floats in (64 << 20, 0):
+        kc, vc = zeros((2, 704, width), np.uint16), zeros((2, width, 704), np.uint16)
+        query, out = empty((2, rows, width), np.uint16), empty((rows, width))
+        workspace = empty((max(floats // 4, 1),))
+        N.call("evo_hip_attention_ws", p(dev(proj.reshape(rows, -1))), rows, width, heads, 1,
+               p(inv_freq), 8.0, 0, p(query), p(kc), p(vc), 704, p(out), p(workspace), floats,
+               stream())
+        masks.append(np.isfinite(host(out)))
+    expected = np.ones((rows, width), bool)
+    expected[450:, 2 * head_dim + 5] = False
+    # V^T shares 16-key MFMA steps: rows of the value's 32-key tile before it
+    # multiply it by a zero probability
+    for mask in masks:
+        assert np.array_equal(mask[:448], expected[:448])
+        assert np.array_equal(mask[480:], expected[480:])
+    assert np.array_equal(masks[0], masks[1])
+
+
 def test_attention_rejects_unaligned_capacity():
     width, heads = 64, 2
     proj = zeros((4, 3 * width))
