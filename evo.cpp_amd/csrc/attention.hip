@@ -72,37 +72,89 @@ __device__ inline size_t qkv_column(int column_split, size_t width, size_t head,
                       : component * width + head * head_dim + dim;
 }
 
-// One block per row; thread t owns rotation pair t % (head_dim / 2) of
-// heads t / (head_dim / 2) + k * (512 / head_dim), so the pair's cosine and
-// sine are evaluated once per row (head_dim / 2 divides 256 for head_dim 16
-// to 128) and every wave reads and writes whole runs of consecutive dims.
-__global__ __launch_bounds__(256) void qkv_rope_kernel(
-    const float *__restrict__ projected, size_t width, size_t heads, int half,
-    int column_split, const float *__restrict__ inv_freq, float rope_scale, size_t prefix,
-    uint16_t *__restrict__ q, size_t q_plane, uint16_t *__restrict__ k_cache,
-    size_t cache_plane) {
-  const size_t row = blockIdx.x;
-  const size_t head_dim = 2 * static_cast<size_t>(half);
-  const int pair = static_cast<int>(threadIdx.x) % half;
-  const int head_step = 256 / half;
-  const float *src = projected + row * width * 3;
-  const float position = static_cast<float>(prefix + row) / rope_scale;
-  const float angle = position * inv_freq[pair];
-  const float cosine = cosf(angle), sine = sinf(angle);
-  for (size_t head = threadIdx.x / half; head < heads; head += head_step) {
-    const size_t qi = row * width + head * head_dim;
-    const size_t ki = (prefix + row) * width + head * head_dim;
-    {
-      const float first = src[qkv_column(column_split, width, head, head_dim, 0, pair)];
-      const float second = src[qkv_column(column_split, width, head, head_dim, 0, half + pair)];
-      put_split(q, q + q_plane, qi + pair, first * cosine - second * sine);
-      put_split(q, q + q_plane, qi + half + pair, second * cosine + first * sine);
+// Consecutive split-BF16 elements: kVec planes' words in one store each.
+template <int kVec>
+__device__ inline void put_split_vec(uint16_t *hi, uint16_t *lo, const float (&v)[kVec]) {
+  if constexpr (kVec == 1) {
+    put_split(hi, lo, 0, v[0]);
+  } else {
+    uint16_t h[kVec], l[kVec];
+#pragma unroll
+    for (int e = 0; e < kVec; ++e) {
+      h[e] = f32_to_bf16(v[e]);
+      l[e] = f32_to_bf16(v[e] - bf16_to_f32(h[e]));
     }
-    {
-      const float first = src[qkv_column(column_split, width, head, head_dim, 1, pair)];
-      const float second = src[qkv_column(column_split, width, head, head_dim, 1, half + pair)];
-      put_split(k_cache, k_cache + cache_plane, ki + pair, first * cosine - second * sine);
-      put_split(k_cache, k_cache + cache_plane, ki + half + pair, second * cosine + first * sine);
+    *reinterpret_cast<uint2 *>(hi) = __builtin_bit_cast(uint2, h);
+    *reinterpret_cast<uint2 *>(lo) = __builtin_bit_cast(uint2, l);
+  }
+}
+template <int kVec>
+__device__ inline void load_floats(const float *src, float (&v)[kVec]) {
+  if constexpr (kVec == 1) {
+    v[0] = src[0];
+  } else {
+    const float4 f = *reinterpret_cast<const float4 *>(src);
+    v[0] = f.x;
+    v[1] = f.y;
+    v[2] = f.z;
+    v[3] = f.w;
+  }
+}
+
+struct QkvAppend {
+  const float *projected;
+  size_t rows, width, heads;
+  int half;  // rotation pairs per head
+  int column_split;
+  const float *inv_freq;
+  float rope_scale;
+  size_t prefix;
+  uint16_t *q;
+  size_t q_plane;
+  uint16_t *k_cache, *vt_cache;
+  size_t cache_plane, capacity;
+  int *range_flag;
+  unsigned value_blocks, row_parts;
+};
+
+// Rotated q and k of one row (or, with row_parts > 1, of a part of its
+// heads): a thread owns kVec rotation pairs of every head_step-th head, so
+// their cosines and sines are evaluated once.
+template <int kVec>
+__device__ inline void rotate_row(const QkvAppend &a, size_t row, int part) {
+  const size_t head_dim = 2 * static_cast<size_t>(a.half);
+  const int lanes = a.half / kVec;  // threads per head
+  const int head_step = 256 / lanes;
+  const int pair = static_cast<int>(threadIdx.x) % lanes * kVec;
+  const float *src = a.projected + row * a.width * 3;
+  const float position = static_cast<float>(a.prefix + row) / a.rope_scale;
+  float cosine[kVec], sine[kVec];
+#pragma unroll
+  for (int e = 0; e < kVec; ++e) {
+    const float angle = position * a.inv_freq[pair + e];
+    cosine[e] = cosf(angle);
+    sine[e] = sinf(angle);
+  }
+  for (size_t head = threadIdx.x / lanes + static_cast<size_t>(part) * head_step; head < a.heads;
+       head += static_cast<size_t>(head_step) * a.row_parts) {
+#pragma unroll
+    for (int component = 0; component < 2; ++component) {
+      float first[kVec], second[kVec], x[kVec], y[kVec];
+      load_floats(src + qkv_column(a.column_split, a.width, head, head_dim, component, pair),
+                  first);
+      load_floats(
+          src + qkv_column(a.column_split, a.width, head, head_dim, component, a.half + pair),
+          second);
+#pragma unroll
+      for (int e = 0; e < kVec; ++e) {
+        x[e] = first[e] * cosine[e] - second[e] * sine[e];
+        y[e] = second[e] * cosine[e] + first[e] * sine[e];
+      }
+      const size_t at = (component == 0 ? row : a.prefix + row) * a.width + head * head_dim + pair;
+      uint16_t *hi = (component == 0 ? a.q : a.k_cache) + at;
+      uint16_t *lo = hi + (component == 0 ? a.q_plane : a.cache_plane);
+      put_split_vec(hi, lo, x);
+      put_split_vec(hi + a.half, lo + a.half, y);
     }
   }
 }
@@ -110,58 +162,82 @@ __global__ __launch_bounds__(256) void qkv_rope_kernel(
 // V rows [rows, W] of the projection -> V^T planes at positions prefix..:
 // a 64-position x 64-channel tile is read row-wise, transposed through LDS
 // and written position-contiguous.
-__global__ __launch_bounds__(256) void v_transpose_kernel(
-    const float *__restrict__ projected, size_t rows, size_t width, size_t head_dim,
-    int column_split, size_t prefix, uint16_t *__restrict__ vt_cache, size_t cache_plane,
-    size_t capacity, int *range_flag) {
-  __shared__ float tile[64][65];
+template <int kVec>
+__device__ inline void transpose_values(const QkvAppend &a, size_t r0, size_t c0,
+                                        float (*tile)[65]) {
+  constexpr int kLanes = 64 / kVec, kStep = 256 / kLanes;  // lanes per row, rows per pass
   const int tid = threadIdx.x;
-  const size_t r0 = blockIdx.x * 64ULL, c0 = blockIdx.y * 64ULL;
-  const size_t channel = c0 + (tid & 63);
+  const size_t head_dim = 2 * static_cast<size_t>(a.half);
+  const int offset = tid % kLanes * kVec;
+  const size_t channel = c0 + offset;
+  const float *src = a.projected + qkv_column(a.column_split, a.width, channel / head_dim,
+                                              head_dim, 2, channel % head_dim);
   bool out_of_range = false;
-  for (int i = tid >> 6; i < 64; i += 4) {
-    const size_t row = r0 + i;
-    float value = 0.0F;
-    if (row < rows && channel < width)
-      value = projected[row * width * 3 +
-                        qkv_column(column_split, width, channel / head_dim, head_dim, 2,
-                                   channel % head_dim)];
-    out_of_range |= !(__builtin_fabsf(value) <= 65504.0F);
-    tile[tid & 63][i] = value;
+#pragma unroll
+  for (int i0 = 0; i0 < 64; i0 += kStep) {
+    const int i = i0 + tid / kLanes;
+    float value[kVec] = {};
+    if (r0 + i < a.rows && channel < a.width)
+      load_floats(src + (r0 + i) * a.width * 3, value);
+#pragma unroll
+    for (int e = 0; e < kVec; ++e) {
+      out_of_range |= !(__builtin_fabsf(value[e]) <= 65504.0F);
+      tile[offset + e][i] = value[e];
+    }
   }
-  if (range_flag != nullptr && out_of_range)
-    atomicOr(range_flag, kFlagF16Range);
+  if (a.range_flag != nullptr && out_of_range)
+    atomicOr(a.range_flag, kFlagF16Range);
   __syncthreads();
-  if (prefix % 16 == 0 && r0 + 64 <= rows && c0 + 64 <= width) {
+  if (a.prefix % 16 == 0 && r0 + 64 <= a.rows && c0 + 64 <= a.width) {
     // Whole tile from a 16-aligned position: its 64 V^T columns per channel
     // are [prefix + r0, +64) in the permuted order; each lane packs 8 of
     // them (column j holds row vt_column(j), the permutation being its own
     // inverse) into one 16-byte store per plane.
-    uint16_t *base = vt_cache + prefix + r0;
+    uint16_t *base = a.vt_cache + a.prefix + r0;
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
       const int idx = tid + 256 * k, i = idx >> 3, unit = idx & 7;
       uint32_t hi[4], lo[4];
 #pragma unroll
       for (int e = 0; e < 8; e += 2) {
-        const float a = tile[i][vt_column(8 * unit + e)];
-        const float b = tile[i][vt_column(8 * unit + e + 1)];
-        const uint16_t ha = f32_to_bf16(a), hb = f32_to_bf16(b);
-        hi[e / 2] = ha | (static_cast<uint32_t>(hb) << 16);
-        lo[e / 2] = f32_to_bf16(a - bf16_to_f32(ha)) |
-                    (static_cast<uint32_t>(f32_to_bf16(b - bf16_to_f32(hb))) << 16);
+        const float v0 = tile[i][vt_column(8 * unit + e)];
+        const float v1 = tile[i][vt_column(8 * unit + e + 1)];
+        const uint16_t h0 = f32_to_bf16(v0), h1 = f32_to_bf16(v1);
+        hi[e / 2] = h0 | (static_cast<uint32_t>(h1) << 16);
+        lo[e / 2] = f32_to_bf16(v0 - bf16_to_f32(h0)) |
+                    (static_cast<uint32_t>(f32_to_bf16(v1 - bf16_to_f32(h1))) << 16);
       }
-      const size_t at = (c0 + i) * capacity + 8 * unit;
+      const size_t at = (c0 + i) * a.capacity + 8 * unit;
       *reinterpret_cast<uint4 *>(base + at) = make_uint4(hi[0], hi[1], hi[2], hi[3]);
-      *reinterpret_cast<uint4 *>(base + cache_plane + at) = make_uint4(lo[0], lo[1], lo[2], lo[3]);
+      *reinterpret_cast<uint4 *>(base + a.cache_plane + at) =
+          make_uint4(lo[0], lo[1], lo[2], lo[3]);
     }
     return;
   }
-  for (int i = tid >> 6; i < 64; i += 4) {
-    const size_t ch = c0 + i, row = r0 + (tid & 63);
-    if (row < rows && ch < width)
-      put_split(vt_cache, vt_cache + cache_plane, ch * capacity + vt_column(prefix + row),
-                tile[i][tid & 63]);
+  const int rows_here = static_cast<int>(min(static_cast<size_t>(64), a.rows - r0));
+  const int channels = static_cast<int>(min(static_cast<size_t>(64), a.width - c0));
+  // A few rows (the decode step): lanes on the channels, else on the rows.
+  for (int j = tid; j < rows_here * channels; j += 256) {
+    const int i = j / rows_here, row = j % rows_here;
+    put_split(a.vt_cache, a.vt_cache + a.cache_plane,
+              (c0 + i) * a.capacity + vt_column(a.prefix + r0 + row), tile[i][row]);
+  }
+}
+
+// q, k and v of a projection in one launch: the first value_blocks blocks
+// write V^T tiles, the others rotate rows. Bound by bytes (F32 in, two
+// planes out): 1500 x 1920 takes 18 us, one decode row of 4096 5.0 (a launch
+// each, one scalar pair or channel per thread: 26.6 and 13.8).
+template <int kVec>
+__global__ __launch_bounds__(256) void append_qkv_kernel(const QkvAppend a) {
+  __shared__ float tile[64][65];
+  const unsigned b = blockIdx.x;
+  if (b < a.value_blocks) {
+    const unsigned columns = static_cast<unsigned>((a.width + 63) / 64);
+    transpose_values<kVec>(a, b / columns * 64ULL, b % columns * 64ULL, tile);
+  } else {
+    const unsigned r = b - a.value_blocks;
+    rotate_row<kVec>(a, r / a.row_parts, static_cast<int>(r % a.row_parts));
   }
 }
 
@@ -884,15 +960,26 @@ Status qkv_rope(const float *projected, size_t rows, size_t width, size_t heads,
   const size_t half = width / heads / 2;
   if (256 % half != 0 || rows > (1U << 31))
     return {ErrorCode::kInvalidArgument, "qkv_rope: head_dim / 2 must divide 256"};
-  hipLaunchKernelGGL(qkv_rope_kernel, dim3(static_cast<unsigned>(rows)), dim3(256), 0, stream,
-                     projected, width, heads, static_cast<int>(half), column_split ? 1 : 0,
-                     inv_freq, rope_scale, prefix, q, q_plane, k_cache, cache_plane);
-  EVO_TRY(launch_status("qkv_rope_kernel"));
-  hipLaunchKernelGGL(v_transpose_kernel, dim3(ceil_div(rows, 64), ceil_div(width, 64)),
-                     dim3(256), 0, stream, projected, rows, width, width / heads,
-                     column_split ? 1 : 0, prefix, v_cache, cache_plane, capacity,
-                     v_range_flag);
-  return launch_status("v_transpose_kernel");
+  const size_t value_blocks = static_cast<size_t>(ceil_div(rows, 64)) * ceil_div(width, 64);
+  // Four pairs or channels per thread where every run starts on 16 bytes of
+  // the projection and 8 of a plane.
+  const bool vec = half % 4 == 0 && reinterpret_cast<uintptr_t>(projected) % 16 == 0 &&
+                   (reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k_cache)) % 8 ==
+                       0 &&
+                   q_plane % 4 == 0 && cache_plane % 4 == 0;
+  // A few rows: a block per group of heads instead of one per row.
+  const size_t head_step = 256 / (half / (vec ? 4 : 1));
+  const size_t row_parts = rows >= 256 ? 1 : ceil_div(heads, head_step);
+  const size_t blocks = value_blocks + rows * row_parts;
+  if (blocks > (1U << 31))
+    return {ErrorCode::kInvalidArgument, "qkv_rope: grid too large"};
+  const QkvAppend append{projected, rows, width, heads, static_cast<int>(half),
+                         column_split ? 1 : 0, inv_freq, rope_scale, prefix, q, q_plane,
+                         k_cache, v_cache, cache_plane, capacity, v_range_flag,
+                         static_cast<unsigned>(value_blocks), static_cast<unsigned>(row_parts)};
+  hipLaunchKernelGGL(vec ? append_qkv_kernel<4> : append_qkv_kernel<1>,
+                     dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream, append);
+  return launch_status("append_qkv_kernel");
 }
 
 Status causal_attention(const uint16_t *q, size_t q_plane, const uint16_t *k_cache,

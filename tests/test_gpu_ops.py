@@ -976,6 +976,44 @@ def test_attention_split_over_keys(oracle, heads, head_dim, rows, prefix):
         assert np.array_equal(kc, caches[0][0]) and np.array_equal(vc, caches[0][1])
 
 
+@pytest.mark.parametrize("column_split", [0, 1])
+@pytest.mark.parametrize("heads,head_dim,rows,prefix", [
+    (3, 16, 1, 5), (20, 64, 1, 64), (2, 128, 63, 16), (5, 32, 64, 3), (17, 64, 255, 0),
+    (2, 128, 256, 7), (3, 128, 321, 32)])
+def test_qkv_append_vectors_equal_scalars(heads, head_dim, rows, prefix, column_split):
+    """Four rotation pairs or channels per thread (a 16-byte aligned
+    projection) leave the same caches and outputs, bit for bit, as one, and
+    touch no other cache position; V^T against its definition."""
+    width = heads * head_dim
+    capacity = (prefix + rows + 127) // 64 * 64
+    r = rng(heads + rows)
+    proj = r.standard_normal((rows, 3 * width)).astype(np.float32)
+    inv_freq = dev((1.0 / 10000 ** (np.arange(0, head_dim, 2) / head_dim)).astype(np.float32))
+    got = []
+    for offset in (0, 1):
+        source = empty((rows * 3 * width + offset,))
+        source[offset:] = dev(proj.reshape(-1))
+        kc, vc = zeros((2, capacity, width), np.uint16), zeros((2, width, capacity), np.uint16)
+        query, out = empty((2, rows, width), np.uint16), empty((rows, width))
+        N.call("evo_hip_attention", p(source) + 4 * offset, rows, width, heads, column_split,
+               p(inv_freq), 8.0, prefix, p(query), p(kc), p(vc), capacity, p(out), stream())
+        got.append([host(t) for t in (query, kc, vc, out)])
+    for a, b in zip(*got):
+        assert np.array_equal(a.view(np.uint8), b.view(np.uint8))
+    _, kc, vc, _ = got[0]
+    written = np.zeros(capacity, bool)
+    written[prefix:prefix + rows] = True
+    assert not kc[:, ~written].any() and kc[0, written].any(axis=1).all()
+    shape = (rows, heads, 3, head_dim) if column_split else (rows, 3, heads, head_dim)
+    v = proj.reshape(shape)[:, :, 2] if column_split else proj.reshape(shape)[:, 2]
+    pos = np.arange(capacity)
+    column = (pos & ~15) | (pos & 3) | ((pos & 4) << 1) | ((pos & 8) >> 1)
+    rows_v = vc[:, :, column].transpose(0, 2, 1)
+    assert not rows_v[:, ~written].any()
+    stored = bf16_to_f32(rows_v[0, written]) + bf16_to_f32(rows_v[1, written])
+    assert np.abs(stored - v.reshape(rows, width)).max() <= 2.0**-16 * np.abs(v).max()
+
+
 @pytest.mark.parametrize("value", [np.inf, np.nan])
 def test_attention_split_keeps_non_finite_rows(value):
     """A non-finite value at one position of one head reaches that head's
