@@ -61,6 +61,17 @@ __device__ inline float get_split(const uint16_t *hi, const uint16_t *lo, size_t
   return bf16_to_f32(hi[i]) + bf16_to_f32(lo[i]);
 }
 
+// hi + lo of 8 consecutive elements.
+__device__ inline void split_floats(const uint4 &hi, const uint4 &lo, float (&v)[8]) {
+  const uint32_t h[4] = {hi.x, hi.y, hi.z, hi.w}, l[4] = {lo.x, lo.y, lo.z, lo.w};
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    v[2 * i] = __builtin_bit_cast(float, h[i] << 16) + __builtin_bit_cast(float, l[i] << 16);
+    v[2 * i + 1] = __builtin_bit_cast(float, h[i] & 0xffff0000U) +
+                   __builtin_bit_cast(float, l[i] & 0xffff0000U);
+  }
+}
+
 // Position of key `pos` inside the transposed value cache.
 __host__ __device__ inline size_t vt_column(size_t pos) {
   return (pos & ~static_cast<size_t>(15)) | (pos & 3) | ((pos & 4) << 1) | ((pos & 8) >> 1);
@@ -780,127 +791,166 @@ Status launch_flash(const uint16_t *q, size_t q_plane, const uint16_t *k_cache,
 }
 
 // ---- Single-query (decode) attention, split over the keys: one block per
-// (head, chunk of 256 keys). Each lane scores one key (F32 dot of q with
-// the key's hi + lo planes), the block takes its max and exponentials, and
-// 256 threads form the chunk's P V with thread t on dimension t / 2 and
-// keys of half t % 2 (reading the transposed value cache row of that
-// dimension; its 16-key permutation swaps position bits 2 and 3, so column c
-// holds key vt_column(c)). The chunk leaves (max, sum, o[d]); a second
-// kernel per head rescales the chunks to the common max and sums them in
-// chunk order. Full-softmax semantics as `src/cpu/model.cpp:510-544`.
-constexpr int kDecodeKeys = 256;
+// (head, chunk of whole 64-key tiles). 16 lanes read a key's row of a plane
+// (16 bytes each) and 8 lanes a V^T row's 64 positions, so every load of a
+// tile, K and V, is a run of whole lines and all are in flight at once; the
+// dots are F32, reduced over the lanes, the softmax runs on the tile's 64
+// scores, and wave w sums the head's dimensions d % 32 / 8 == w (the V^T
+// permutation swaps position bits 2 and 3, so column c holds key
+// vt_column(c)). The chunk leaves (max, sum, o[d]); a second kernel per head
+// rescales the chunks to the common max and sums them in chunk order.
+// Full-softmax semantics as `src/cpu/model.cpp:510-544`.
+// Bound by the latency of its loads at short prefixes (keys in chunks of 256,
+// a key per lane, V after the softmax took 17.3 us at 1040 keys x 32 heads of
+// 128, this 10.3) and by the cache's bytes at long ones.
+constexpr int kDecodeKeys = 256;  // most keys per chunk of a minimal workspace
+constexpr int kDecodeTile = 64;
 
 template <int kD>
 __global__ __launch_bounds__(256) void decode_attention_kernel(
     const uint16_t *__restrict__ q, size_t q_plane, const uint16_t *__restrict__ k_cache,
     const uint16_t *__restrict__ v_cache, size_t cache_plane, size_t capacity,
-    size_t keys, size_t heads, float *__restrict__ part) {
-  __shared__ float q_s[kD];
-  __shared__ float p_s[kDecodeKeys];
-  __shared__ float red_s[4];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    size_t keys, size_t heads, int chunk_tiles, float *__restrict__ part) {
+  constexpr int kRowLanes = kD / 8;                // lanes per key row
+  constexpr int kKeysPerPass = 256 / kRowLanes;    // keys per block pass
+  constexpr int kKPasses = kDecodeTile / kKeysPerPass > 0 ? kDecodeTile / kKeysPerPass : 1;
+  constexpr int kVPasses = kD / 32;                // 32 dimensions per block pass
+  __shared__ float score_s[kDecodeTile];
+  __shared__ float p_s[kDecodeTile];
+  const int tid = threadIdx.x, lane = tid & 63;
   const size_t chunk = blockIdx.x, h = blockIdx.y;
   const size_t width = heads * kD;
-  if (tid < kD)
-    q_s[tid] = get_split(q, q + q_plane, h * kD + tid);
-  __syncthreads();
-  const size_t key = chunk * kDecodeKeys + tid;
-  float score = -INFINITY;
-  if (key < keys) {
-    const uint16_t *k_hi = k_cache + key * width + h * kD;
-    const uint16_t *k_lo = k_hi + cache_plane;
-    float dot = 0.0F;
+  const int row_lane = tid % kRowLanes, row_key = tid / kRowLanes;
+  float qv[8];
 #pragma unroll
-    for (int d0 = 0; d0 < kD; d0 += 8) {
-      const uint4 hv = *reinterpret_cast<const uint4 *>(k_hi + d0);
-      const uint4 lv = *reinterpret_cast<const uint4 *>(k_lo + d0);
-      const uint32_t hw[4] = {hv.x, hv.y, hv.z, hv.w}, lw[4] = {lv.x, lv.y, lv.z, lv.w};
+  for (int e = 0; e < 8; ++e)
+    qv[e] = get_split(q, q + q_plane, h * kD + row_lane * 8 + e);
+  const int v_lane = tid & 7, v_row = tid >> 3;
+  float o[kVPasses] = {};
+  float m = -INFINITY, l = 0.0F;
+  const size_t tile0 = chunk * chunk_tiles;
+  const size_t tile1 = min(tile0 + chunk_tiles, (keys + kDecodeTile - 1) / kDecodeTile);
+  for (size_t t = tile0; t < tile1; ++t) {
+    const size_t key0 = t * kDecodeTile;
+    uint4 kh[kKPasses], kl[kKPasses], vh[kVPasses], vl[kVPasses];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float k0 = __builtin_bit_cast(float, hw[i] << 16) +
-                         __builtin_bit_cast(float, lw[i] << 16);
-        const float k1 = __builtin_bit_cast(float, hw[i] & 0xffff0000U) +
-                         __builtin_bit_cast(float, lw[i] & 0xffff0000U);
-        dot = fmaf(q_s[d0 + 2 * i], k0, dot);
-        dot = fmaf(q_s[d0 + 2 * i + 1], k1, dot);
+    for (int i = 0; i < kKPasses; ++i) {
+      const int key = i * kKeysPerPass + row_key;
+      kh[i] = kl[i] = make_uint4(0, 0, 0, 0);
+      if (key < kDecodeTile && key0 + key < keys) {
+        const uint16_t *src = k_cache + (key0 + key) * width + h * kD + row_lane * 8;
+        kh[i] = *reinterpret_cast<const uint4 *>(src);
+        kl[i] = *reinterpret_cast<const uint4 *>(src + cache_plane);
       }
     }
-    score = dot * (1.0F / sqrtf(static_cast<float>(kD)));
-  }
-  float m = score;
 #pragma unroll
-  for (int offset = 32; offset > 0; offset >>= 1)
-    m = fmaxf(m, __shfl_xor(m, offset, 64));
-  if (lane == 0)
-    red_s[wave] = m;
-  __syncthreads();
-  m = fmaxf(fmaxf(red_s[0], red_s[1]), fmaxf(red_s[2], red_s[3]));
-  const float p = key < keys ? expf(score - m) : 0.0F;
-  p_s[tid] = p;
-  float l = p;
+    for (int i = 0; i < kVPasses; ++i) {
+      const uint16_t *src = v_cache + (h * kD + i * 32 + v_row) * capacity + key0 + v_lane * 8;
+      vh[i] = *reinterpret_cast<const uint4 *>(src);
+      vl[i] = *reinterpret_cast<const uint4 *>(src + cache_plane);
+    }
 #pragma unroll
-  for (int offset = 32; offset > 0; offset >>= 1)
-    l += __shfl_xor(l, offset, 64);
-  __syncthreads();  // p_s complete; red_s reads done
-  if (lane == 0)
-    red_s[wave] = l;
-  // P V: thread t -> dimension t / 2 (t < 2 kD), keys of half t % 2.
-  float o = 0.0F;
-  const int d = tid >> 1, part_half = tid & 1;
-  if (d < kD) {
-    const size_t row = h * kD + d;
-    const size_t col0 = chunk * kDecodeKeys + part_half * (kDecodeKeys / 2);
-    const uint16_t *v_hi = v_cache + row * capacity + col0;
-    const uint16_t *v_lo = v_hi + cache_plane;
-    // Whole 16-column blocks: the permutation moves a key up to 8 columns
-    // past its position inside its block (key 84 of 85 sits in column 88).
-    const size_t end = min(static_cast<size_t>(kDecodeKeys / 2),
-                           keys > col0 ? (keys - col0 + 15) / 16 * 16 : size_t{0});
-    for (size_t c0 = 0; c0 < end; c0 += 8) {
-      const uint4 hv = *reinterpret_cast<const uint4 *>(v_hi + c0);
-      const uint4 lv = *reinterpret_cast<const uint4 *>(v_lo + c0);
-      const uint32_t hw[4] = {hv.x, hv.y, hv.z, hv.w}, lw[4] = {lv.x, lv.y, lv.z, lv.w};
+    for (int i = 0; i < kKPasses; ++i) {
+      float kv[8], dot = 0.0F;
+      split_floats(kh[i], kl[i], kv);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const size_t c = part_half * (kDecodeKeys / 2) + c0 + 2 * i;
-        const float v0 = __builtin_bit_cast(float, hw[i] << 16) +
-                         __builtin_bit_cast(float, lw[i] << 16);
-        const float v1 = __builtin_bit_cast(float, hw[i] & 0xffff0000U) +
-                         __builtin_bit_cast(float, lw[i] & 0xffff0000U);
+      for (int e = 0; e < 8; ++e)
+        dot = fmaf(qv[e], kv[e], dot);
+#pragma unroll
+      for (int offset = 1; offset < kRowLanes; offset <<= 1)
+        dot += __shfl_xor(dot, offset, 64);
+      const int key = i * kKeysPerPass + row_key;
+      if (row_lane == 0 && key < kDecodeTile)
+        score_s[key] = key0 + key < keys ? dot * (1.0F / sqrtf(static_cast<float>(kD)))
+                                         : -INFINITY;
+    }
+    __syncthreads();
+    // Every wave holds the tile's scores (lane = key): the same maximum and
+    // sum in each.
+    const float score = score_s[lane];
+    float tile_max = score;
+#pragma unroll
+    for (int offset = 32; offset > 0; offset >>= 1)
+      tile_max = fmaxf(tile_max, __shfl_xor(tile_max, offset, 64));
+    const float next = fmaxf(m, tile_max);
+    const float reference = next == -INFINITY ? 0.0F : next;
+    const float p = key0 + lane < keys ? expf(score - reference) : 0.0F;
+    float sum = p;
+#pragma unroll
+    for (int offset = 32; offset > 0; offset >>= 1)
+      sum += __shfl_xor(sum, offset, 64);
+    const float scale = t == tile0 ? 0.0F : expf(m - reference);
+    l = t == tile0 ? sum : fmaf(l, scale, sum);
+    m = next;
+    if (tid < 64)
+      p_s[lane] = p;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kVPasses; ++i) {
+      float vv[8], acc = 0.0F;
+      split_floats(vh[i], vl[i], vv);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
         // Zero weights are skipped: columns of keys past the end may hold
         // unwritten cache.
-        const float p0 = p_s[vt_column(c)], p1 = p_s[vt_column(c + 1)];
-        if (p0 != 0.0F)
-          o = fmaf(p0, v0, o);
-        if (p1 != 0.0F)
-          o = fmaf(p1, v1, o);
+        const float weight = p_s[vt_column(v_lane * 8 + e)];
+        acc = weight != 0.0F ? fmaf(weight, vv[e], acc) : acc;
       }
+      o[i] = t == tile0 ? acc : fmaf(o[i], scale, acc);
     }
   }
-  o += __shfl_xor(o, 1, 64);
-  __syncthreads();
   float *dst = part + (h * gridDim.x + chunk) * (kD + 2);
-  if (d < kD && part_half == 0)
-    dst[2 + d] = o;
+#pragma unroll
+  for (int i = 0; i < kVPasses; ++i) {
+#pragma unroll
+    for (int offset = 1; offset < 8; offset <<= 1)
+      o[i] += __shfl_xor(o[i], offset, 64);
+    if (v_lane == 0)
+      dst[2 + i * 32 + v_row] = o[i];
+  }
   if (tid == 0) {
     dst[0] = m;
-    dst[1] = red_s[0] + red_s[1] + red_s[2] + red_s[3];
+    dst[1] = l;
   }
 }
 
+// 256 / kD groups of threads sum every group-th chunk, then each other.
 template <int kD, typename O>
-__global__ void decode_combine_kernel(const float *__restrict__ part, int chunks, O out) {
+__global__ __launch_bounds__(256) void decode_combine_kernel(const float *__restrict__ part,
+                                                             int chunks, O out) {
+  constexpr int kGroups = 256 / kD;
+  __shared__ float l_s[kGroups][kD], o_s[kGroups][kD], max_s[4];
   const size_t h = blockIdx.x;
-  const int d = threadIdx.x;
+  const int tid = threadIdx.x, d = tid % kD, group = tid / kD;
   const float *base = part + h * chunks * (kD + 2);
   float m = -INFINITY;
-  for (int c = 0; c < chunks; ++c)
-    m = fmaxf(m, base[c * (kD + 2)]);
+  for (int c = tid; c < chunks; c += 256)
+    m = fmaxf(m, base[static_cast<size_t>(c) * (kD + 2)]);
+#pragma unroll
+  for (int offset = 32; offset > 0; offset >>= 1)
+    m = fmaxf(m, __shfl_xor(m, offset, 64));
+  if ((tid & 63) == 0)
+    max_s[tid >> 6] = m;
+  __syncthreads();
+  m = fmaxf(fmaxf(max_s[0], max_s[1]), fmaxf(max_s[2], max_s[3]));
+  const float reference = m == -INFINITY ? 0.0F : m;
   float l = 0.0F, o = 0.0F;
-  for (int c = 0; c < chunks; ++c) {
-    const float scale = expf(base[c * (kD + 2)] - m);
-    l = fmaf(base[c * (kD + 2) + 1], scale, l);
-    o = fmaf(base[c * (kD + 2) + 2 + d], scale, o);
+#pragma unroll 4
+  for (int c = group; c < chunks; c += kGroups) {
+    const float *src = base + static_cast<size_t>(c) * (kD + 2);
+    const float scale = expf(src[0] - reference);
+    l = fmaf(src[1], scale, l);
+    o = fmaf(src[2 + d], scale, o);
+  }
+  l_s[group][d] = l;
+  o_s[group][d] = o;
+  __syncthreads();
+  if (group != 0)
+    return;
+#pragma unroll
+  for (int g = 1; g < kGroups; ++g) {
+    l += l_s[g][d];
+    o += o_s[g][d];
   }
   put(out, h * kD + d, o / l);
 }
@@ -908,12 +958,22 @@ __global__ void decode_combine_kernel(const float *__restrict__ part, int chunks
 template <int kD, typename O>
 Status launch_decode(const uint16_t *q, size_t q_plane, const uint16_t *k_cache,
                      const uint16_t *v_cache, size_t cache_plane, size_t capacity, size_t keys,
-                     size_t heads, float *workspace, O out, hipStream_t stream) {
-  const unsigned chunks = static_cast<unsigned>(ceil_div(keys, kDecodeKeys));
+                     size_t heads, float *workspace, size_t workspace_bytes, O out,
+                     hipStream_t stream) {
+  // The fewest tiles per chunk that leave at most about 8 blocks per CU (a
+  // combine over a bounded number of chunks) and whose parts fit.
+  const size_t tiles = ceil_div(keys, kDecodeTile);
+  const size_t part = heads * (kD + 2) * sizeof(float);
+  size_t chunk_tiles = std::max<size_t>(1, tiles * heads / 2048);
+  chunk_tiles = std::max<size_t>(chunk_tiles, ceil_div(tiles, 512));
+  if ((tiles + chunk_tiles - 1) / chunk_tiles * part > workspace_bytes)
+    chunk_tiles = std::max<size_t>(chunk_tiles, kDecodeKeys / kDecodeTile);
+  const unsigned chunks = static_cast<unsigned>((tiles + chunk_tiles - 1) / chunk_tiles);
   hipLaunchKernelGGL(decode_attention_kernel<kD>, dim3(chunks, heads), dim3(256), 0, stream, q,
-                     q_plane, k_cache, v_cache, cache_plane, capacity, keys, heads, workspace);
+                     q_plane, k_cache, v_cache, cache_plane, capacity, keys, heads,
+                     static_cast<int>(chunk_tiles), workspace);
   EVO_TRY(launch_status("decode_attention_kernel"));
-  hipLaunchKernelGGL((decode_combine_kernel<kD, O>), dim3(heads), dim3(kD), 0, stream,
+  hipLaunchKernelGGL((decode_combine_kernel<kD, O>), dim3(heads), dim3(256), 0, stream,
                      workspace, static_cast<int>(chunks), out);
   return launch_status("decode_combine_kernel");
 }
@@ -1002,13 +1062,13 @@ Status causal_attention(const uint16_t *q, size_t q_plane, const uint16_t *k_cac
       switch (head_dim) {
       case 32:
         return launch_decode<32>(q, q_plane, k_cache, v_cache, cache_plane, capacity, keys,
-                                 heads, workspace, out, stream);
+                                 heads, workspace, workspace_bytes, out, stream);
       case 64:
         return launch_decode<64>(q, q_plane, k_cache, v_cache, cache_plane, capacity, keys,
-                                 heads, workspace, out, stream);
+                                 heads, workspace, workspace_bytes, out, stream);
       default:
         return launch_decode<128>(q, q_plane, k_cache, v_cache, cache_plane, capacity, keys,
-                                  heads, workspace, out, stream);
+                                  heads, workspace, workspace_bytes, out, stream);
       }
     };
     if (out_f32 != nullptr)

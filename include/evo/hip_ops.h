@@ -251,9 +251,10 @@ EVO_API evo_status evo_hip_attention(const float *projected, size_t rows,
                                      float *out, void *stream);
 
 /* evo_hip_attention with an F32 device workspace: a single query (rows == 1,
- * head_dim 32/64/128) is then split over its keys in chunks of 256 (per
- * chunk and head: max, sum and head_dim partial outputs in the workspace),
- * the decode step's path; and a few rows, or the last rows of a prompt, over
+ * head_dim 32/64/128) is then split over its keys in chunks of at most 256
+ * where the workspace holds no more, and of 64 and up otherwise (per chunk
+ * and head: max, sum and head_dim partial outputs in the workspace), the
+ * decode step's path; and a few rows, or the last rows of a prompt, over
  * parts of their keys where the workspace holds the parts (rows x heads x
  * parts x (head_dim + 2) floats) and that is faster. The same reference
  * interface. */

@@ -1043,6 +1043,47 @@ def test_attention_split_keeps_non_finite_rows(value):
     assert np.array_equal(masks[0], masks[1])
 
 
+@pytest.mark.parametrize("heads,head_dim,prefix", [
+    (2, 128, 62), (2, 128, 63), (3, 64, 64), (40, 128, 5000), (2, 32, 32900)])
+def test_single_query_chunks(heads, head_dim, prefix):
+    """One query split in chunks of 64 keys (a large workspace) or more (a
+    minimal one, long prefixes), against the 64-bit softmax over the cached
+    planes: F32 dots and sums of head_dim and prefix terms of either sign,
+    1e-6 of the output in the root mean square. Cache columns past the last
+    key may hold anything."""
+    r = rng(prefix + heads)
+    width, keys = heads * head_dim, prefix + 1
+    capacity = (keys + 64 + 63) // 64 * 64
+    inv_freq = dev(np.ones(head_dim // 2, np.float32))
+    kc = bf16_bits(r.standard_normal((2, capacity, width)).astype(np.float32))
+    vc = bf16_bits(r.standard_normal((2, width, capacity)).astype(np.float32))
+    kc[1] = bf16_bits(bf16_to_f32(kc[1]) * np.float32(2.0**-9))
+    vc[1] = bf16_bits(bf16_to_f32(vc[1]) * np.float32(2.0**-9))
+    pos = np.arange(capacity)
+    column = (pos & ~15) | (pos & 3) | ((pos & 4) << 1) | ((pos & 8) >> 1)
+    vc[:, :, column[keys:]] = 0x7FC0  # NaN
+    kc[:, keys:] = 0x7FC0
+    proj = dev(r.standard_normal((1, 3 * width)).astype(np.float32))
+    least = heads * ((keys + 255) // 256) * (head_dim + 2)
+    for floats in (least, 16 * least):
+        k_dev, v_dev = dev(kc), dev(vc)
+        query, out = empty((2, 1, width), np.uint16), empty((1, width))
+        workspace = empty((floats + 64,))
+        workspace.fill_(7.0)
+        N.call("evo_hip_attention_ws", p(proj), 1, width, heads, 1, p(inv_freq), 8.0, prefix,
+               p(query), p(k_dev), p(v_dev), capacity, p(out), p(workspace), floats * 4, stream())
+        assert np.all(host(workspace)[floats:] == 7.0)
+        planes = [bf16_to_f32(host(t)).astype(np.float64) for t in (query, k_dev, v_dev)]
+        q, k, v = (t[0] + t[1] for t in planes)
+        q, k = q.reshape(heads, head_dim), k[:keys].reshape(keys, heads, head_dim)
+        v = v[:, column[:keys]].reshape(heads, head_dim, keys)
+        score = np.einsum("hd,khd->hk", q, k) / np.sqrt(head_dim)
+        weight = np.exp(score - score.max(axis=1, keepdims=True))
+        weight /= weight.sum(axis=1, keepdims=True)
+        expected = np.einsum("hk,hdk->hd", weight, v).reshape(1, width)
+        assert np.linalg.norm(host(out) - expected) < 1e-6 * np.linalg.norm(expected)
+
+
 def test_attention_rejects_unaligned_capacity():
     width, heads = 64, 2
     proj = zeros((4, 3 * width))
