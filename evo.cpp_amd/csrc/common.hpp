@@ -143,6 +143,27 @@ __host__ __device__ inline uint8_t encode_e4m3(const float value) {
   return sign | static_cast<uint8_t>(((exponent + 7) << 3) + (q - 8));
 }
 
+// Four codes, the first in the low byte, the same as encode_e4m3's for every
+// F32 (the hardware convert rounds to nearest even and, as its input is held
+// to +-448 here, never overflows; a NaN's sign is encode_e4m3's business).
+// About 10 instructions where four encode_e4m3 take 100 and branch.
+__device__ inline uint32_t encode_e4m3x4(const float (&v)[4]) {
+  float c[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    c[e] = __builtin_amdgcn_fmed3f(v[e], -448.0F, 448.0F);
+  int codes = __builtin_amdgcn_cvt_pk_fp8_f32(c[0], c[1], 0, false);
+  codes = __builtin_amdgcn_cvt_pk_fp8_f32(c[2], c[3], codes, true);
+  if (__builtin_isunordered(v[0], v[1]) || __builtin_isunordered(v[2], v[3])) {
+    uint8_t code[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      code[e] = encode_e4m3(v[e]);
+    return __builtin_bit_cast(uint32_t, code);
+  }
+  return static_cast<uint32_t>(codes);
+}
+
 // ---- Activation storage type of the inter-kernel tensors.
 enum class IoType : int { kF32 = 0, kBF16 = 1 };
 

@@ -457,11 +457,11 @@ __global__ __launch_bounds__(256) void fp8_gemv_kernel(
         const float4 g = *reinterpret_cast<const float4 *>(norm.scale + c);
         const float y[4] = {norm_value(v.x, denominator, g.x), norm_value(v.y, denominator, g.y),
                             norm_value(v.z, denominator, g.z), norm_value(v.w, denominator, g.w)};
-        uint8_t code[4];
+        float scaled[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-          code[e] = encode_e4m3(round_bf16(y[e]) * code_scale);
-        *reinterpret_cast<uint32_t *>(codes_s + m * K + c) = __builtin_bit_cast(uint32_t, code);
+          scaled[e] = round_bf16(y[e]) * code_scale;
+        *reinterpret_cast<uint32_t *>(codes_s + m * K + c) = encode_e4m3x4(scaled);
       }
       __syncthreads();
     }

@@ -457,6 +457,26 @@ def test_linear_normed_equals_norm_then_linear(m, k, n, split):
     assert np.array_equal(host(folded).view(np.uint32), host(two_step).view(np.uint32))
 
 
+@pytest.mark.parametrize("width,code_scale", [(4096, 1.0), (2048, 56.0), (8192, 2.0**-7),
+                                              (65536, 3.0)])
+def test_rms_norm_e4m3_codes_of_every_bf16(oracle, width, code_scale):
+    """A row of ones has the denominator 1 and passes the norm's scales on:
+    every BF16 value, infinities and NaN of both signs included, gets the
+    oracle's code, byte for byte."""
+    bits = np.arange(65536, dtype=np.uint16)
+    expected = np.zeros(65536, np.uint8)
+    oracle.oracle_e4m3_quantize_bf16(O.ptr(bits), bits.size, code_scale, O.ptr(expected))
+    values = bf16_to_f32(bits)
+    ones = dev(np.ones((1, width), np.float32))
+    got = []
+    for start in range(0, 65536, width):
+        codes = empty((1, width), np.uint8)
+        N.call("evo_hip_rms_norm_e4m3", p(ones), 1, width, p(dev(values[start:start + width])),
+               0.0, code_scale, p(codes), stream())
+        got.append(host(codes).reshape(-1))
+    assert np.array_equal(np.concatenate(got), expected)
+
+
 @pytest.mark.parametrize("m,k,n", [(1, 4096, 12288), (2, 1920, 1000), (4, 4096, 520)])
 @pytest.mark.parametrize("mode", [0, 1])
 def test_fp8_linear_normed_equals_norm_codes_then_linear(m, k, n, mode):
