@@ -37,6 +37,7 @@ public:
       reset();
       ptr_ = other.ptr_;
       bytes_ = other.bytes_;
+      owned_ = other.owned_;
       other.ptr_ = nullptr;
       other.bytes_ = 0;
     }
@@ -44,6 +45,8 @@ public:
   }
   Status allocate(size_t bytes, const char *what);
   Status upload(const void *host, size_t bytes, const char *what);
+  // A part of memory that another buffer owns (and outlives this one with).
+  void view(void *ptr, size_t bytes);
   void reset();
   template <typename T> T *as() const { return static_cast<T *>(ptr_); }
   size_t bytes() const { return bytes_; }
@@ -51,6 +54,7 @@ public:
 private:
   void *ptr_{nullptr};
   size_t bytes_{0};
+  bool owned_{true};
 };
 
 enum class Mixer { kHcs, kHcm, kHcl, kAttention };
@@ -145,7 +149,9 @@ public:
 private:
   Status enqueue(const uint32_t *device_tokens, size_t rows, bool initial,
                  float *device_logits, size_t capture_layer, float *capture);
-  Status finish();
+  // Downloads the flag and what follows it (`logit_bytes` of logits_) in one
+  // copy, synchronises and reports.
+  Status finish(size_t logit_bytes);
   Status run_layers(size_t rows, size_t capture_layer, float *capture);
   void reset_caches();
   // workspace_ holds pending_'s partials until the next norm of hidden_
@@ -164,6 +170,12 @@ private:
   hipStream_t stream_{nullptr};
   size_t capacity_{0}, cache_capacity_{0}, arena_rows_{0}, position_{0};
   bool valid_{false};
+  // One allocation for every buffer of up to 64 MiB, which are views of it.
+  DeviceBuffer arena_;
+  // Tokens, flag and logits are consecutive, so that a call's upload (its
+  // tokens, right-aligned, and a zero for the flag) and its download (flag
+  // and logits) are one copy each.
+  DeviceBuffer io_;
   DeviceBuffer tokens_, hidden_, residual_, normed_, projected_, mixed_, query_,
       gated_, logits_, codes_, workspace_, flag_;
   size_t workspace_bytes_{0};
@@ -175,8 +187,11 @@ private:
   // clears in one launch.
   DeviceBuffer reset_table_;
   size_t reset_count_{0}, reset_max_words_{0};
-  float *host_logits_{nullptr};
+  // Pinned: the upload [tokens][0], then the download [flag][logits].
+  void *pinned_{nullptr};
+  uint32_t *host_tokens_end_{nullptr};
   int *host_flag_{nullptr};
+  float *host_logits_{nullptr};
 };
 
 }  // namespace evo::hip

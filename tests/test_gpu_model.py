@@ -293,6 +293,38 @@ def test_decode_argument_errors(hip, tmp_path):
     assert ctx.decode(71).shape == (512,)  # a rejected call leaves the context usable
 
 
+@pytest.mark.parametrize("length", [1, 31, 32, 33, 77])
+def test_contexts_share_nothing(hip, tmp_path, length):
+    """A context's buffers are parts of one allocation and its tokens, flag
+    and logits of one copy: two contexts used in turn give what each gives
+    alone, and a call that raised the flag (a token past the vocabulary)
+    leaves no trace in another context's."""
+    from evo_hip import native as N
+    from gpu_util import dev, empty, host, p, release
+    shape = A.tiny_shape(width=64, layers=8, heads=2, inner=96, groups=4, attn=(3,))
+    path = make(tmp_path, shape, seed=47)
+    a, b = (A.acgt_tokens(length, seed=s).astype(np.uint8) for s in (1, 2))
+    alone = []
+    for tokens in (a, b):
+        ctx = open_context(hip, path, capacity=length + 1)
+        alone.append((ctx.prefill(tokens.tobytes()), ctx.decode(65)))
+    first, second, third = (open_context(hip, path, capacity=length + 1) for _ in range(3))
+    bad = a.astype(np.uint32)
+    bad[-1] = 512
+    logits = empty((length, 512))
+    with pytest.raises(N.OpError, match="vocabulary"):
+        N.call("evo_hip_context_prefill_resident", third.handle, p(dev(bad)), length, p(logits))
+    got = [(first.prefill(a.tobytes()), None), (second.prefill(b.tobytes()), None)]
+    steps = [first.decode(65), second.decode(65)]
+    for (logits_a, step_a), (logits_g, _), step in zip(alone, got, steps):
+        assert np.array_equal(logits_a.view(np.uint32), logits_g.view(np.uint32))
+        assert np.array_equal(step_a.view(np.uint32), step.view(np.uint32))
+    N.call("evo_hip_context_prefill_resident", first.handle, p(dev(b.astype(np.uint32))), length,
+           p(logits))
+    assert np.array_equal(host(logits).view(np.uint32), alone[1][0].view(np.uint32))
+    release()
+
+
 def test_product_timing_hooks(hip, tmp_path):
     """The measurement hooks bench.py reads: no timed launches by default;
     with timing on, one MLP l1/l2 launch per layer, each with a positive
