@@ -422,11 +422,11 @@ __global__ __launch_bounds__(256) void fp8_gemv_kernel(
     int M, int N, int K, float output_scale, const RowNorm norm, float code_scale) {
   constexpr int kLanesPerChunk = kChunk / 16;
   constexpr int kRowsPerWave = kGemv8Rows / 4;
-  // LDS: chunk sums [kGemv8Rows][M][K/kChunk], then (folded norm) the
-  // activation codes [M][K].
+  // LDS: chunk sums [kGemv8Rows][M][K/kChunk + 1] (a row's chain reads its
+  // own bank), then (folded norm) the activation codes [M][K].
   extern __shared__ float chunk_s[];
   __shared__ float norm_partial[4];
-  const int chunks = K / kChunk;
+  const int chunks = K / kChunk, stride = chunks + 1;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int row0 = blockIdx.x * kGemv8Rows + wave * kRowsPerWave;
   // The codes of the next 1024-K sweep load before this sweep is multiplied.
@@ -443,7 +443,7 @@ __global__ __launch_bounds__(256) void fp8_gemv_kernel(
     load_codes(k, codes);
   // (The first weights are in flight while the block forms the activation
   // codes of a folded norm.)
-  uint8_t *codes_s = reinterpret_cast<uint8_t *>(chunk_s + kGemv8Rows * M * chunks);
+  uint8_t *codes_s = reinterpret_cast<uint8_t *>(chunk_s + kGemv8Rows * M * stride);
   const bool folded = norm.x != nullptr;
   if (folded) {
     // The codes rms_norm would write, e4m3(bf16(norm(x)) * code_scale),
@@ -490,7 +490,7 @@ __global__ __launch_bounds__(256) void fp8_gemv_kernel(
         for (int offset = 1; offset < kLanesPerChunk; offset <<= 1)
           sum += __shfl_xor(sum, offset, 64);
         if ((lane % kLanesPerChunk) == 0)
-          chunk_s[((wave * kRowsPerWave + r) * M + m) * chunks + k / kChunk] = sum;
+          chunk_s[((wave * kRowsPerWave + r) * M + m) * stride + k / kChunk] = sum;
       }
     }
 #pragma unroll
@@ -505,8 +505,9 @@ __global__ __launch_bounds__(256) void fp8_gemv_kernel(
   if (m >= M || row >= N)
     return;
   float acc = 0.0F;
+#pragma unroll 8
   for (int c = 0; c < chunks; ++c)
-    acc = truncate_e8m13(acc + chunk_s[(r * M + m) * chunks + c]);
+    acc = truncate_e8m13(acc + chunk_s[(r * M + m) * stride + c]);
   put(out, static_cast<size_t>(m) * N + row, round_bf16(acc * output_scale));
 }
 
@@ -610,7 +611,7 @@ Status fp8_linear_impl(const uint8_t *in_codes, const uint8_t *w_codes, Out *out
   if (M <= static_cast<size_t>(kGemv8MaxM) && K <= static_cast<size_t>(kGemv8MaxK)) {
     const dim3 grid(static_cast<unsigned>(ceil_div(N, kGemv8Rows)));
     const int chunk = mode == kFp8MfmaK32 ? 32 : 128;
-    const size_t lds = kGemv8Rows * M * (K / chunk) * sizeof(float) +
+    const size_t lds = kGemv8Rows * M * (K / chunk + 1) * sizeof(float) +
                        (norm != nullptr ? M * K : 0);
     auto pick = [&](auto rows_c) {
       constexpr int kM = decltype(rows_c)::value;
