@@ -214,7 +214,7 @@ def kernel_rooflines(split):
                                         query.data_ptr(), keys.data_ptr(), values.data_ptr(),
                                         cap, att_out.data_ptr(), stream), 5)
     flops = 2.0 * length * length * width
-    out["attention"] = dict(kernel="qkv_rope_kernel + flash_attention_kernel", ms=ms,
+    out["attention"] = dict(kernel="append_qkv_kernel + flash_attention_kernel", ms=ms,
                             flops=flops, tflops=flops / ms / 1e9)
     return out
 
