@@ -1503,29 +1503,15 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 && !kTwoGroups ? 2 : 1) void hy
     for (int w = 0; w < PairRow<T>::kWords; ++w)
       dst.word[w] = src[w];
   };
-  // Rows before 0 (first segment, first step) come from the short history.
-  auto history_row = [&](long row, PairRow<T> &dst) {
+  // Rows before 0 (first segment, step 0) come from the short history, which
+  // holds F32 values also where the projection is BF16.
+  auto history_row = [&](long row, float (&dst)[6]) {
     const long hrow = static_cast<long>(short_len - 1) + row;
 #pragma unroll
-    for (int i = 0; i < PairRow<T>::kWords; ++i)
-      dst.word[i] = 0;
-    if (short_history != nullptr && hrow >= 0) {
-      float v[6];
-#pragma unroll
-      for (int col = 0; col < 6; ++col)
-        v[col] = short_history[static_cast<size_t>(hrow) * cols3 + 3 * cp + col];
-      if constexpr (sizeof(T) == 2) {
-        // BF16 inputs: the history holds BF16 values.
-#pragma unroll
-        for (int i = 0; i < 3; ++i)
-          dst.word[i] = (__builtin_bit_cast(uint32_t, v[2 * i]) >> 16) |
-                        (__builtin_bit_cast(uint32_t, v[2 * i + 1]) & 0xffff0000U);
-      } else {
-#pragma unroll
-        for (int i = 0; i < 6; ++i)
-          dst.word[i] = __builtin_bit_cast(uint32_t, v[i]);
-      }
-    }
+    for (int col = 0; col < 6; ++col)
+      dst[col] = short_history != nullptr && hrow >= 0
+                     ? short_history[static_cast<size_t>(hrow) * cols3 + 3 * cp + col]
+                     : 0.0F;
   };
 
   // ---- MFMA lane: channel slice `wave`, fragment group g.
@@ -1614,22 +1600,28 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 && !kTwoGroups ? 2 : 1) void hy
   const int x2_lane = 4 * rg * kMsChannels + 2 * pair;
   const int u_prod[2] = {2 * pair * kMsUStride + ms_ucol(2 * pair, 4 * rg),
                          (2 * pair + 1) * kMsUStride + ms_ucol(2 * pair + 1, 4 * rg)};
-  auto produce = [&](int step) __attribute__((always_inline)) {
+  auto produce = [&](auto first, int step) __attribute__((always_inline)) {
+    constexpr bool kFirst = decltype(first)::value;  // step 0: may reach rows before 0
     PairRow<T> cur[kRows];
-    const long first_row = static_cast<long>(t_start) + step * kMsStep + 4 * rg - (kWin - 1);
-    if (static_cast<long>(t_start) + step * kMsStep >= kWin - 1) {
+    float before[kFirst ? kWin - 1 : 1][6];  // rows -2, -1 of the lanes that own row 0
+    const bool from_history = kFirst && t_start == 0 && rg == 0;
 #pragma unroll
-      for (int i = 0; i < kRows; ++i)
-        stage_row(step, 4 * rg + i, cur[i]);
-    } else {
+    for (int i = 0; i < kRows; ++i)
+      stage_row(step, 4 * rg + i, cur[i]);
+    if constexpr (kFirst) {
+      if (from_history) {
 #pragma unroll
-      for (int i = 0; i < kRows; ++i) {
-        if (first_row + i >= 0)
-          stage_row(step, 4 * rg + i, cur[i]);
-        else
-          history_row(first_row + i, cur[i]);
+        for (int i = 0; i < kWin - 1; ++i)
+          history_row(i - (kWin - 1), before[i]);
       }
     }
+    auto value = [&](int i, int col) {
+      if constexpr (kFirst) {
+        if (i < kWin - 1)
+          return from_history ? before[i][col] : cur[i].at(col);
+      }
+      return cur[i].at(col);
+    };
     float *x2 = &xy_s[step % 3][0][0] + x2_lane;
     uint16_t *uplanes = &u_s[step & 1][0][0][0];
     float u[2][4];
@@ -1641,7 +1633,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 && !kTwoGroups ? 2 : 1) void hy
         float total = 0.0F;
 #pragma unroll
         for (int i = 0; i < kWin; ++i)
-          total += cur[j + i].at(c6) * stap[c6][i];
+          total += value(j + i, c6) * stap[c6][i];
         fir[c6] = total;
       }
       u[0][j] = fir[1] * fir[2];
@@ -1813,7 +1805,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 && !kTwoGroups ? 2 : 1) void hy
         }
         a[f][half][q] = __builtin_bit_cast(u32x4, taps);
       }
-  produce(0);
+  produce(std::true_type{}, 0);
   wait_dma<0>();
   __syncthreads();
 
@@ -1828,7 +1820,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 && !kTwoGroups ? 2 : 1) void hy
     if (step + 2 < steps)
       issue(step + 2);
     if (step + 1 < steps)
-      produce(step + 1);
+      produce(std::false_type{}, step + 1);
     multiply(rot, step);
     if (kTwoGroups && threadIdx.x == 0)
       flag_s[(step + 2) % 8] = 0U;  // step - 6's, read by no phase any more

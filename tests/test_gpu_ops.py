@@ -821,6 +821,42 @@ def test_hyena_group_size_15_continuation(kind, inner_len, split):
     assert np.array_equal(host(caches["short"]), case["projection"][-2:])
 
 
+def hyena_exact(kind, case, projection, short_history, inner_history):
+    """The FIR mixers in 64 bits, continued from the given caches."""
+    length, width = projection.shape[0], case["width"]
+    k, taps = case["inner_len"], bf16_to_f32(case["short"]).astype(np.float64)
+    rows = np.concatenate([short_history, projection]).astype(np.float64)
+    fir = sum(rows[t:t + length] * taps[:, t] for t in range(3)).reshape(length, width, 3)
+    u = np.concatenate([inner_history.astype(np.float64), fir[:, :, 1] * fir[:, :, 2]])
+    inner = np.repeat(case["inner"].astype(np.float64), width // case["groups"], axis=0)
+    if kind == N.HYENA_HCM:
+        inner = inner[:, ::-1]  # causal convolution: the oldest row meets the last tap
+    y = sum(u[t:t + length] * inner[:, t] for t in range(k))
+    if "direct" in case:
+        y = y + u[k - 1:] * case["direct"]
+    return fir[:, :, 0] * y
+
+
+@pytest.mark.parametrize("kind,inner_len,groups,width", [
+    (N.HYENA_HCM, 128, 64, 960), (N.HYENA_HCM, 128, 8, 128), (N.HYENA_HCM, 33, 8, 192),
+    (N.HYENA_HCS, 7, 64, 960), (N.HYENA_HCS, 7, 8, 128)])
+@pytest.mark.parametrize("length", [2, 40])
+def test_hyena_f32_histories_with_bf16_projection(kind, inner_len, groups, width, length):
+    """The caches hold F32: a history that is no BF16 value enters a BF16
+    projection's operator unrounded (cut to BF16 it would be off by up to 2^-7
+    relative in the first rows). F32 sums and the 2^-17 of the split planes."""
+    case = hyena_case(length + width + inner_len, kind, length, width, groups=groups,
+                      inner_len=inner_len)
+    r = rng(length + width)
+    short = r.standard_normal((2, 3 * width)).astype(np.float32)
+    inner = r.standard_normal((inner_len - 1, width)).astype(np.float32)
+    proj = bf16_to_f32(bf16_bits(case["projection"]))
+    expected = hyena_exact(kind, case, proj, short, inner)
+    actual = hyena_gpu(kind, case, dtype=N.DTYPE_BF16_SPLIT, projection=proj, bf16_taps=True,
+                       caches=dict(short=dev(short), inner=dev(inner)))
+    assert rel_err(actual, expected) < 2e-5
+
+
 @pytest.mark.parametrize("split", [1, 31, 32, 300, 1024, 1500])
 def test_hcm_stream_continuation(split):
     """Continuation through the caches with the streaming kernel: the first
