@@ -2863,6 +2863,14 @@ Status launch_fir_mfma(const T *projection, const float *short_history,
   return launch_status("hyena_fir_mfma_kernel");
 }
 
+bool is_aligned(const void *ptr, size_t bytes) {
+  return reinterpret_cast<uintptr_t>(ptr) % bytes == 0;
+}
+bool is_aligned(const F16Out &out, size_t bytes) { return is_aligned(out.out, bytes); }
+bool is_aligned(const SplitOut &out, size_t bytes) {
+  return is_aligned(out.hi, bytes) && is_aligned(out.lo, bytes);
+}
+
 // Rows per block of the HCM row stream: the length whose busiest CU walks the
 // fewest steps. A block walks its rows and, past the first segment, the
 // kMsLead steps before them, plus a prologue worth about four steps; a CU
@@ -2992,17 +3000,22 @@ Status hyena_forward(int kind, const T *projection, size_t length,
     const int causal = kind == kHyenaHcm ? 1 : 0;
     const float *direct = kind == kHyenaHcm ? wt.direct : nullptr;
     const size_t group_size = width / wt.groups;
+    const bool two_groups = group_size % 16 != 0;
     // (Odd group sizes only with the exact windows: in the padded ones an
-    // infinity would reach rows past the filter through a zero tap.)
+    // infinity would reach rows past the filter through a zero tap. Rows and
+    // outputs that do not start where the streams' accesses need it, 4 or 16
+    // bytes, run the kernel that reads and writes single elements.)
     if (k <= 8 && planar == 0 && width % 2 == 0 &&
-        (group_size % 2 == 0 || (short_len == 3 && k == 7))) {
+        (group_size % 2 == 0 ||
+         (short_len == 3 && k == 7 && is_aligned(projection, 4) && is_aligned(out, 4)))) {
       EVO_TRY((launch_fir_stream<T, O>(projection, short_history, wt, short_len, inner_history,
                                        group_size, k, causal, direct, length, width, out,
                                        stream)));
     } else if (wt.taps_bf16 && short_len == 3 && planar == 0 && width % kMsChannels == 0 &&
-               group_size >= 15 && direct != nullptr) {
+               direct != nullptr &&
+               (!two_groups || (group_size >= 15 && is_aligned(projection, 16) &&
+                                is_aligned(out, 16)))) {
       const unsigned cblocks = static_cast<unsigned>(width / kMsChannels);
-      const bool two_groups = group_size % 16 != 0;
       const unsigned seg_len = ms_segment(cblocks, length, sizeof(T) == 2 && !two_groups);
       const unsigned segments = ceil_div(length, seg_len);
       const auto kernel = two_groups ? hyena_fir_mfma_stream_kernel<T, O, true>

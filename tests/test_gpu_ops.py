@@ -857,6 +857,42 @@ def test_hyena_f32_histories_with_bf16_projection(kind, inner_len, groups, width
     assert rel_err(actual, expected) < 2e-5
 
 
+@pytest.mark.parametrize("kind,inner_len,groups,width", [
+    (N.HYENA_HCM, 128, 64, 960), (N.HYENA_HCM, 33, 8, 320), (N.HYENA_HCS, 7, 64, 960)])
+@pytest.mark.parametrize("dtype,proj_at,out_at", [
+    (N.DTYPE_BF16, 1, 0), (N.DTYPE_BF16, 0, 1), (N.DTYPE_BF16, 2, 2), (N.DTYPE_F16, 1, 0),
+    (N.DTYPE_F16, 0, 1), (N.DTYPE_F32, 3, 1)])
+def test_hyena_off_16_groups_at_any_element(kind, inner_len, groups, width, dtype, proj_at,
+                                            out_at):
+    """Projections and outputs that start at any element of a buffer (sizes of
+    filter groups that are no multiple of 16): the wide accesses of the row
+    streams are taken where they fit, single elements elsewhere. The elements
+    around the output stay untouched."""
+    length = 70
+    case = hyena_case(width + inner_len, kind, length, width, groups=groups, inner_len=inner_len)
+    bf16_in = dtype == N.DTYPE_BF16
+    proj = bf16_to_f32(bf16_bits(case["projection"])) if bf16_in else case["projection"]
+    expected = hyena_oracle(kind, case, projection=proj)
+    flat = (bf16_bits(proj) if bf16_in else proj).ravel()
+    held = dev(np.concatenate([np.zeros(proj_at, flat.dtype), flat]))
+    out_type = np.float32 if dtype == N.DTYPE_F32 else np.uint16
+    count = length * width
+    out = zeros((count + 8,), out_type)
+    N.call("evo_hip_hyena_forward", kind, dtype | N.DTYPE_BF16_TAPS, p(held[proj_at:]), length,
+           width, p(dev(case["short"])), 3, p(dev(case["inner"])), groups, inner_len,
+           p(dev(case["direct"]) if "direct" in case else None), None, None, 0, None, None, None,
+           None, 0, p(out[out_at:]), stream())
+    got = host(out)
+    assert not got[:out_at].any() and not got[out_at + count:].any()
+    got = got[out_at:out_at + count].reshape(length, width)
+    if dtype == N.DTYPE_BF16:
+        got = bf16_to_f32(got.view(np.uint16))
+    elif dtype == N.DTYPE_F16:
+        got = got.view(np.float16).astype(np.float32)
+    bound = {N.DTYPE_F32: 2e-6, N.DTYPE_F16: 2.0 ** -11, N.DTYPE_BF16: 2.0 ** -8}[dtype]
+    assert rel_err(got, expected) < bound
+
+
 @pytest.mark.parametrize("split", [1, 31, 32, 300, 1024, 1500])
 def test_hcm_stream_continuation(split):
     """Continuation through the caches with the streaming kernel: the first
