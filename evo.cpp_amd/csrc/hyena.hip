@@ -19,6 +19,7 @@
 // rescans each chunk from its true state and writes y. One thread owns one
 // channel and keeps its 16 modal states in registers.
 #include "common.hpp"
+#include "launch_rules.hpp"
 #include "ops.hpp"
 
 #include <cmath>
@@ -361,7 +362,7 @@ __global__ __launch_bounds__(256) void hyena_fir_kernel(
 // Each lane owns two adjacent channels: their six interleaved projection
 // columns are 12 (BF16) or 24 (F32) contiguous bytes of a row, and the two
 // outputs are one packed 32-bit store per plane. A wave streams a segment of
-// 16 to 128 rows (kStreamRows, kStreamMaxRows); it starts kLead rows early
+// 16 to 128 rows (hcs_stream_segment); it starts kLead rows early
 // so that its short-FIR window and its FIR window of u are full when the
 // segment begins (the lead rows are recomputed, not stored). Both windows
 // hold their taps right-aligned with zeros in front, so every sum runs oldest
@@ -373,16 +374,13 @@ __global__ __launch_bounds__(256) void hyena_fir_kernel(
 // are non-temporal: the outputs are never re-read here, and streaming them
 // past the L2 keeps it for the projection rows (-23 % kernel time on the 7B
 // shape).
-// Segment length: 16 rows, doubled up to 128 while the grid keeps at least
-// kStreamMinBlocks blocks (two per CU): longer segments recompute fewer lead
-// rows (7B, L = 8192: 64 rows 58 us, 128 rows 54; 256 measured no better),
-// shorter ones are what fills the chip for a short prompt, where a block's
-// serial walk is the time (611 rows at W = 4096, BF16, with both histories:
-// 23.5 us with 64-row segments, 16.2; W = 1920, whose odd groups ran tile by
-// tile in LDS before: 54.3 -> 13.9 us, 8192 rows 302 -> 26).
+// Segment length (hcs_stream_segment): short segments fill the chip for a short
+// prompt, where a block's serial walk is the time (611 rows at W = 4096, BF16,
+// with both histories: 23.5 us with 64-row segments, 16.2 with 16; W = 1920,
+// whose odd groups ran tile by tile in LDS before: 54.3 -> 13.9 us, 8192 rows
+// 302 -> 26), long ones recompute fewer lead rows.
 constexpr int kStreamRows = 16;
 constexpr int kStreamMaxRows = 128;
-constexpr unsigned kStreamMinBlocks = 512;
 constexpr int kStreamBatch = 4;
 constexpr int kStreamWaves = 4;              // waves per block
 constexpr int kStreamChannels = kStreamWaves * 64 * 2;
@@ -2788,10 +2786,7 @@ void launch_fir_stream_taps(const T *projection, const float *short_history,
                             size_t group_size, int k, int causal, const float *direct,
                             size_t length, size_t width, O out, hipStream_t stream) {
   const unsigned cblocks = ceil_div(width, kStreamChannels);
-  unsigned seg_len = kStreamRows;
-  while (seg_len < kStreamMaxRows &&
-         cblocks * ceil_div(length, 2 * static_cast<size_t>(seg_len)) >= kStreamMinBlocks)
-    seg_len *= 2;
+  const unsigned seg_len = hcs_stream_segment(width, length, sizeof(T) == 4 && kWin == 3);
   const unsigned segments = ceil_div(length, seg_len);
   const dim3 grid(cblocks * segments), block(kStreamWaves * 64);
   auto run = [&](auto direct_c, auto pair_c) {
@@ -2897,6 +2892,30 @@ unsigned ms_segment(unsigned channel_blocks, size_t length, bool pairs) {
 }
 
 }  // namespace
+
+// Segment length of the row stream: the longest of 16, 32, 64 and 128 rows
+// whose grid leaves more than a block per CU, for 128 rows two per CU. With
+// F32 rows and the exact windows (8 lead rows) 64 rows also need two: those
+// are bound by their reads. Measured at W = 4096, 16 / 32 / 64 / 128 rows per
+// segment, us:
+//   BF16, padded windows (14 lead rows): 1500 rows 18.9 / 16.1 / 18.7 / 29.6,
+//     2049 rows 26.0 / 25.6 / 23.3 / 30.1, 3000 rows 31.5 / 27.6 / 24.1 / 31.0,
+//     4096 rows 40.0 / 32.9 / 25.4 / 31.3, 8192 rows 73.2 / 60.0 / 51.8 / 43.6
+//   BF16, exact windows: 1024 rows 10.0 / 10.1 / 13.9 / 21.3, 3000 rows 25.2 /
+//     20.8 / 19.2 / 23.6, 8192 rows 52.2 / 51.6 / 44.3 / 39.9
+//   F32, exact windows: 2049 rows 32.5 / 29.7 / 34.0 / 39.4, 3000 rows 39.9 /
+//     33.6 / 35.7 / 41.5, 6000 rows 72.6 / 63.1 / 57.4 / 62.9.
+unsigned hcs_stream_segment(size_t width, size_t length, bool f32_exact) {
+  const unsigned channel_blocks = ceil_div(width, kStreamChannels);
+  unsigned rows = kStreamRows;
+  for (unsigned next = 2 * kStreamRows; next <= static_cast<unsigned>(kStreamMaxRows); next *= 2) {
+    const bool two_per_cu = next == 128 || (next == 64 && f32_exact);
+    if (channel_blocks * ceil_div(length, next) < (two_per_cu ? 512U : 257U))
+      break;
+    rows = next;
+  }
+  return rows;
+}
 
 size_t hyena_workspace_bytes(int kind, size_t length, size_t width,
                              size_t state) {
