@@ -2917,6 +2917,15 @@ unsigned hcs_stream_segment(size_t width, size_t length, bool f32_exact) {
   return rows;
 }
 
+// A slice of 16 channels touches at most two groups of 15 and more. With F32
+// rows the stream's prologue (two filters' Toeplitz fragments, 107 KB of LDS)
+// is longer than the tap-by-tap sums of a few rows of a short filter: 2 rows
+// of 40 taps with the caches take 17.9 us tap by tap and 19.1 here, 5 rows
+// 21.3 and 20.8, 2 rows of 128 taps 29.7 and 25.6.
+bool hcm_stream_two_groups(size_t group_size, size_t length, int taps, bool f32) {
+  return group_size >= 15 && !(f32 && length * static_cast<size_t>(taps) <= 96);
+}
+
 size_t hyena_workspace_bytes(int kind, size_t length, size_t width,
                              size_t state) {
   if (kind == kHyenaHcs || kind == kHyenaHcm) {
@@ -3032,8 +3041,8 @@ Status hyena_forward(int kind, const T *projection, size_t length,
                                        stream)));
     } else if (wt.taps_bf16 && short_len == 3 && planar == 0 && width % kMsChannels == 0 &&
                direct != nullptr &&
-               (!two_groups || (group_size >= 15 && is_aligned(projection, 16) &&
-                                is_aligned(out, 16)))) {
+               (!two_groups || (hcm_stream_two_groups(group_size, length, k, sizeof(T) == 4) &&
+                                is_aligned(projection, 16) && is_aligned(out, 16)))) {
       const unsigned cblocks = static_cast<unsigned>(width / kMsChannels);
       const unsigned seg_len = ms_segment(cblocks, length, sizeof(T) == 2 && !two_groups);
       const unsigned segments = ceil_div(length, seg_len);

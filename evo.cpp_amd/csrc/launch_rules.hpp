@@ -11,4 +11,8 @@ namespace evo::hip {
 // Rows per segment of the HCS row stream (hyena.hip).
 unsigned hcs_stream_segment(size_t width, size_t length, bool f32_exact);
 
+// Whether the HCM row stream takes filter groups that are no multiple of 16
+// (hyena.hip), rows and outputs aligned.
+bool hcm_stream_two_groups(size_t group_size, size_t length, int taps, bool f32);
+
 }  // namespace evo::hip

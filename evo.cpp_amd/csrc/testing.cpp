@@ -9,3 +9,8 @@
 EVO_TEST_API unsigned evo_test_hcs_stream_segment(size_t width, size_t length, int f32_exact) {
   return evo::hip::hcs_stream_segment(width, length, f32_exact != 0);
 }
+
+EVO_TEST_API int evo_test_hcm_stream_two_groups(size_t group_size, size_t length, int taps,
+                                                int f32) {
+  return evo::hip::hcm_stream_two_groups(group_size, length, taps, f32 != 0) ? 1 : 0;
+}

@@ -18,6 +18,7 @@ def rules():
     size = ctypes.c_size_t
     lib.evo_test_hcs_stream_segment.argtypes = [size, size, ctypes.c_int]
     lib.evo_test_hcs_stream_segment.restype = ctypes.c_uint
+    lib.evo_test_hcm_stream_two_groups.argtypes = [size, size, ctypes.c_int, ctypes.c_int]
     return lib
 
 
@@ -41,3 +42,23 @@ HCS_SEGMENTS = [
 def test_hcs_stream_segment(rules, width, length, f32_exact, times):
     rows = rules.evo_test_hcs_stream_segment(width, length, f32_exact)
     assert times[(16, 32, 64, 128).index(rows)] <= SLACK * min(times)
+
+
+# (group size, length, taps, F32 rows): us tap by tap and on the row stream,
+# with the caches.
+HCM_TWO_GROUPS = [
+    (15, 2, 40, 1, (18.1, 19.2)), (24, 2, 40, 1, (17.9, 19.1)), (17, 2, 40, 1, (18.0, 19.1)),
+    (15, 5, 40, 1, (21.3, 20.8)), (15, 2, 128, 1, (29.7, 25.6)), (15, 17, 40, 1, (32.4, 23.1)),
+    (15, 2, 128, 0, (31.2, 25.0)), (15, 5, 40, 0, (21.9, 20.0)),
+]
+
+
+@pytest.mark.parametrize("group_size,length,taps,f32,times", HCM_TWO_GROUPS)
+def test_hcm_stream_two_groups(rules, group_size, length, taps, f32, times):
+    streamed = rules.evo_test_hcm_stream_two_groups(group_size, length, taps, f32)
+    assert times[streamed] == min(times)
+
+
+def test_hcm_stream_leaves_small_groups(rules):
+    """A slice of 16 channels may touch three groups of 14."""
+    assert not rules.evo_test_hcm_stream_two_groups(14, 1000, 128, 0)
