@@ -25,6 +25,7 @@
 #include <type_traits>
 
 #include "common.hpp"
+#include "launch_rules.hpp"
 #include "row_norm.hpp"
 #include "ops.hpp"
 #include "tile_cost.hpp"
@@ -523,7 +524,7 @@ struct Fp8TileEntry {
   int bm, bn;
   TileCost k128, k32;
 };
-constexpr Fp8TileEntry kFp8Tiles[] = {
+constexpr Fp8TileEntry kFp8Tiles[kFp8TileCount] = {
     {128, 192, {0.85F, 0.81F, 0.113F, 2, {1.131F, 1.413F}}, {5.50F, 0.35F, 0.099F, 2, {1.404F, 2.248F}}},
     {96, 128, {0.44F, 0.0F, 0.047F, 2, {0.901F, 0.931F}}, {3.00F, 0.89F, 0.086F, 2, {0.912F, 1.163F}}},
     {64, 128, {2.39F, 0.0F, 0.013F, 2, {0.551F, 0.717F}}, {3.72F, 0.14F, 0.048F, 2, {0.633F, 0.876F}}},
@@ -532,10 +533,17 @@ constexpr Fp8TileEntry kFp8Tiles[] = {
     {32, 64, {2.23F, 1.20F, 0.0F, 2, {0.285F, 0.369F}}, {2.27F, 1.21F, 0.0F, 2, {0.428F, 0.499F}}},
 };
 
+unsigned elementwise_grid(size_t n) {
+  const size_t blocks = (n + 255) / 256;
+  return static_cast<unsigned>(blocks < 16384 ? blocks : 16384);
+}
+
+}  // namespace
+
 int choose_fp8_tile(size_t M, size_t N, size_t K, bool k32) {
   int best = 0;
   double best_us = 0.0;
-  for (int t = 0; t < static_cast<int>(sizeof(kFp8Tiles) / sizeof(kFp8Tiles[0])); ++t) {
+  for (int t = 0; t < kFp8TileCount; ++t) {
     const Fp8TileEntry &e = kFp8Tiles[t];
     const double us = tile_us(k32 ? e.k32 : e.k128,
                               static_cast<double>(ceil_div(M, e.bm)) * ceil_div(N, e.bn),
@@ -547,13 +555,6 @@ int choose_fp8_tile(size_t M, size_t N, size_t K, bool k32) {
   }
   return best;
 }
-
-unsigned elementwise_grid(size_t n) {
-  const size_t blocks = (n + 255) / 256;
-  return static_cast<unsigned>(blocks < 16384 ? blocks : 16384);
-}
-
-}  // namespace
 
 uint8_t e4m3_encode_host(float value) { return encode_e4m3(value); }
 
@@ -575,6 +576,46 @@ Status e4m3_quantize_bf16(const uint16_t *x, size_t n, float scale,
   hipLaunchKernelGGL(quantize_bf16_kernel, dim3(elementwise_grid(n)), dim3(256), 0,
                      stream, x, n, scale, codes);
   return launch_status("quantize_bf16_kernel");
+}
+
+namespace {
+
+template <typename Out>
+Status launch_mfma(int tile, const uint8_t *in_codes, const uint8_t *w_codes, Out *out, size_t M,
+                   size_t N, size_t K, float output_scale, Fp8Mode mode, hipStream_t stream) {
+  auto launch = [&](auto shape) -> Status {
+    using T = decltype(shape);
+    const auto kernel =
+        mode == kFp8MfmaK32 ? fp8_mfma_kernel<T, 32, Out> : fp8_mfma_kernel<T, 128, Out>;
+    if (T::kLds > 64 * 1024)  // opt in above the 64 KB default
+      EVO_TRY(hip_status(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize,
+                                             static_cast<int>(T::kLds)),
+                         "fp8_mfma_kernel LDS opt-in"));
+    const unsigned blocks = ceil_div(M, T::kBM) * ceil_div(N, T::kBN);
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(T::kWaves * 64), T::kLds, stream, in_codes,
+                       w_codes, out, static_cast<int>(M), static_cast<int>(N),
+                       static_cast<int>(K), output_scale);
+    return launch_status("fp8_mfma_kernel");
+  };
+  // The shapes of kFp8Tiles, in its order.
+  switch (tile) {
+  case 0: return launch(Fp8Tile<128, 192, 2, 2, 2>{});
+  case 1: return launch(Fp8Tile<96, 128, 1, 4, 2>{});
+  case 2: return launch(Fp8Tile<64, 128, 2, 2, 3>{});
+  case 3: return launch(Fp8Tile<64, 64, 2, 2, 5>{});
+  case 4: return launch(Fp8Tile<32, 128, 1, 4, 4>{});
+  case 5: return launch(Fp8Tile<32, 64, 1, 2, 5>{});
+  default: return {ErrorCode::kInternal, "fp8_linear: unknown tile"};
+  }
+}
+
+}  // namespace
+
+Status fp8_linear_on_tile(int tile, const uint8_t *in_codes, const uint8_t *w_codes,
+                          uint16_t *out, size_t M, size_t N, size_t K, float output_scale,
+                          Fp8Mode mode, hipStream_t stream) {
+  return launch_mfma(tile, in_codes, w_codes, out, M, N, K, output_scale, mode, stream);
 }
 
 template <typename Out>
@@ -631,28 +672,8 @@ Status fp8_linear_impl(const uint8_t *in_codes, const uint8_t *w_codes, Out *out
                        output_scale, folded, code_scale);
     return launch_status("fp8_gemv_kernel");
   }
-  auto launch = [&](auto tile) -> Status {
-    using T = decltype(tile);
-    const auto kernel =
-        mode == kFp8MfmaK32 ? fp8_mfma_kernel<T, 32, Out> : fp8_mfma_kernel<T, 128, Out>;
-    if (T::kLds > 64 * 1024)  // opt in above the 64 KB default
-      EVO_TRY(hip_status(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize,
-                                             static_cast<int>(T::kLds)),
-                         "fp8_mfma_kernel LDS opt-in"));
-    const unsigned blocks = ceil_div(M, T::kBM) * ceil_div(N, T::kBN);
-    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(T::kWaves * 64), T::kLds, stream, in_codes,
-                       w_codes, out, m, n, k, output_scale);
-    return launch_status("fp8_mfma_kernel");
-  };
-  switch (choose_fp8_tile(M, N, K, mode == kFp8MfmaK32)) {
-  case 1: return launch(Fp8Tile<96, 128, 1, 4, 2>{});
-  case 2: return launch(Fp8Tile<64, 128, 2, 2, 3>{});
-  case 3: return launch(Fp8Tile<64, 64, 2, 2, 5>{});
-  case 4: return launch(Fp8Tile<32, 128, 1, 4, 4>{});
-  case 5: return launch(Fp8Tile<32, 64, 1, 2, 5>{});
-  default: return launch(Fp8Tile<128, 192, 2, 2, 2>{});
-  }
+  return launch_mfma(choose_fp8_tile(M, N, K, mode == kFp8MfmaK32), in_codes, w_codes, out, M, N, K,
+                     output_scale, mode, stream);
 }
 
 Status fp8_linear(const uint8_t *in_codes, const uint8_t *w_codes, float *out,

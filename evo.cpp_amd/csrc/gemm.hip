@@ -892,6 +892,40 @@ Status split_planes(const float *x, size_t n, uint16_t *hi, uint16_t *lo,
   return launch_status("split_kernel");
 }
 
+LinearPlan plan_linear(size_t M, size_t N, size_t K, bool split, bool gated,
+                       size_t workspace_bytes, bool deferred) {
+  LinearPlan plan;
+  const size_t tiles = static_cast<size_t>(ceil_div(M, kBM)) * ceil_div(N, kBN);
+  // Few tiles (short prompts against W-wide outputs): split K so that about
+  // one tile per CU runs, partials in the workspace, then one reduction.
+  const size_t part_bytes = !gated && N % 4 == 0 ? workspace_bytes : 0;
+  int splits = 1;
+  if (tiles < 128) {
+    for (int s = 2; s <= 16 && tiles * s <= 256; s *= 2)
+      if (K % (static_cast<size_t>(s) * kBK) == 0 && K / s >= 8 * kBK &&
+          static_cast<size_t>(s) * M * N * sizeof(float) <= part_bytes)
+        splits = s;
+  }
+  // Tail split: when the last round would hold at most half the CUs, its
+  // tiles run as two K halves each (raw partials in the workspace), and
+  // gemm_tail_kernel sums them in order and applies the epilogue.
+  const size_t last = tiles > static_cast<size_t>(kGemmCUs) ? tiles % kGemmCUs : 0;
+  if (last != 0 && 2 * last <= static_cast<size_t>(kGemmCUs) && K % (2 * kBK) == 0 &&
+      K / 2 >= 8 * static_cast<size_t>(kBK) &&
+      2 * last * kBM * kBN * sizeof(float) <= workspace_bytes)
+    plan.tail = last;
+  // The small tiles of gemm_tile.hip where their measured cost is lower. A
+  // tail-split launch stays here: more than one full round of 256 x 256
+  // tiles, no CU left idle (7B MLP l1/l2 of 1000 rows: 296 us against 335
+  // on the best small tile, 348 without the tail split).
+  if (plan.tail == 0)
+    plan.choice = choose_gemm_tile(M, N, K, split, gated, static_cast<size_t>(splits), part_bytes,
+                                   deferred);
+  if (plan.choice.tile < 0)
+    plan.choice.splits = splits;
+  return plan;
+}
+
 namespace {
 
 // Shared body of gemm_bf16w (norm == nullptr) and gemm_bf16w_normed.
@@ -963,37 +997,15 @@ Status gemm_impl(const Activation &a, const RowNorm *norm, bool split, const uin
     return launch_status("gemv_kernel");
   }
   if (K % kBK == 0) {
-    // Few tiles (short prompts against W-wide outputs): split K so that about
-    // one tile per CU runs, partials in the workspace, then one reduction.
     // (The reduction reads the partials as 16-byte vectors.)
-    const bool partials = mode != kGemmGated && split_workspace != nullptr &&
-                          reinterpret_cast<uintptr_t>(split_workspace) % 16 == 0 && N % 4 == 0;
-    int splits = 1;
-    if (partials && tiles < 128) {
-      for (int s = 2; s <= 16 && tiles * s <= 256; s *= 2)
-        if (K % (static_cast<size_t>(s) * kBK) == 0 && K / s >= 8 * kBK &&
-            static_cast<size_t>(s) * M * N * sizeof(float) <= split_workspace_bytes)
-          splits = s;
-    }
-    // Tail split: when the last round would hold at most half the CUs, its
-    // tiles run as two K halves each (raw partials in the workspace), and
-    // gemm_tail_kernel sums them in order and applies the epilogue.
-    size_t tail = tiles > static_cast<size_t>(kGemmCUs) ? tiles % kGemmCUs : 0;
-    if (tail == 0 || 2 * tail > static_cast<size_t>(kGemmCUs) || split_workspace == nullptr ||
-        reinterpret_cast<uintptr_t>(split_workspace) % 16 != 0 || K % (2 * kBK) != 0 ||
-        K / 2 < 8 * static_cast<size_t>(kBK) ||
-        2 * tail * kBM * kBN * sizeof(float) > split_workspace_bytes)
-      tail = 0;
-    // The small tiles of gemm_tile.hip where their measured cost is lower. A
-    // tail-split launch stays here: more than one full round of 256 x 256
-    // tiles, no CU left idle (7B MLP l1/l2 of 1000 rows: 296 us against 335
-    // on the best small tile, 348 without the tail split).
-    TileChoice tile;
-    if (tail == 0)
-      tile = choose_gemm_tile(M, N, K, split, mode == kGemmGated, static_cast<size_t>(splits),
-                              partials ? split_workspace_bytes : 0, deferred != nullptr && ldc == n);
-    if (tile.tile >= 0)
-      splits = tile.splits;
+    const bool usable = split_workspace != nullptr &&
+                        reinterpret_cast<uintptr_t>(split_workspace) % 16 == 0;
+    const LinearPlan plan =
+        plan_linear(M, N, K, split, mode == kGemmGated, usable ? split_workspace_bytes : 0,
+                    deferred != nullptr && ldc == n);
+    const TileChoice &tile = plan.choice;
+    const int splits = tile.splits;
+    const size_t tail = plan.tail;
     const Epilogue store{kGemmStore, nullptr, nullptr, 0, 0};
     const size_t plane = M * N;
     if (tile.tile >= 0) {
@@ -1004,14 +1016,11 @@ Status gemm_impl(const Activation &a, const RowNorm *norm, bool split, const uin
       EVO_TRY(gemm_tile(tile.tile, call, stream));
       if (!parted)
         return Status::Ok();
-    }
-    if (splits > 1) {
+    } else if (splits > 1) {
       const dim3 split_grid(static_cast<unsigned>(tiles), static_cast<unsigned>(splits));
       const int ks = k / splits;
       const int all = static_cast<int>(tiles);
-      if (tile.tile >= 0)
-        ;  // the partials are stored
-      else if (split)
+      if (split)
         hipLaunchKernelGGL(gemm_kernel<true>, split_grid, dim3(512), 0, stream, a.hi, a.lo,
                            lda, W, k, m, n, ks, split_workspace, plane, nullptr, nullptr, n,
                            store, all, nullptr);
@@ -1024,6 +1033,8 @@ Status gemm_impl(const Activation &a, const RowNorm *norm, bool split, const uin
                            lda, W, k, m, n, ks, split_workspace, plane, nullptr, nullptr, n,
                            store, all, nullptr);
       EVO_TRY(launch_status("gemm_kernel (split K)"));
+    }
+    if (splits > 1) {
       if (deferred != nullptr && ldc == n) {
         const bool bias_mode = mode == kGemmBias || mode == kGemmBiasResidual;
         const bool res_mode = mode == kGemmResidual || mode == kGemmBiasResidual;

@@ -302,6 +302,7 @@ constexpr TileEntry kTiles[] = {
     {128, 192, 64, {1.28F, 7.28F, 0.280F, 1, {1.034F}}, {1.97F, 5.55F, 0.321F, 1, {0.709F}}},
 };
 constexpr int kTileCount = static_cast<int>(sizeof(kTiles) / sizeof(kTiles[0]));
+static_assert(kTileCount == kGemmTiles, "the tiles of gemm_tile()");
 // The 256 x 256 tile of gemm.hip, the other candidate.
 constexpr TileEntry kLargeTile = {256, 256, 32, {0.0F, 9.34F, 0.294F, 1, {1.094F}},
                                   {0.0F, 9.14F, 0.165F, 1, {0.737F}}};

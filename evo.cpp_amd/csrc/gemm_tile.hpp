@@ -6,20 +6,9 @@
 #include <hip/hip_runtime.h>
 
 #include "gemm_epilogue.hpp"
+#include "launch_rules.hpp"
 
 namespace evo::hip {
-
-// A block tile of gemm_tile.hip (-1: the 256 x 256 tile is the cheaper one)
-// and the number of K parts it runs as.
-struct TileChoice {
-  int tile = -1;
-  int splits = 1;
-};
-// The cheapest tile for C[M,N] of K by measured cost. `large_parts`: the K
-// parts the 256 x 256 tile would run as; workspace_bytes (0: none) bounds the
-// F32 partials of a split; `deferred`: the consumer sums the partials.
-TileChoice choose_gemm_tile(size_t M, size_t N, size_t K, bool split, bool gated,
-                            size_t large_parts, size_t workspace_bytes, bool deferred);
 
 struct TileCall {
   const uint16_t *a_hi, *a_lo;  // a_lo null: one plane

@@ -127,6 +127,11 @@ Status fp8_linear(const uint8_t *in_codes, const uint8_t *w_codes, float *out,
 Status fp8_linear(const uint8_t *in_codes, const uint8_t *w_codes, uint16_t *out,
                   size_t M, size_t N, size_t K, float output_scale,
                   Fp8Mode mode, hipStream_t stream);
+// The MFMA-mode product on block tile `tile` of fp8.hip (0 .. kFp8TileCount
+// - 1, K % 128 == 0): every tile gives the same bits.
+Status fp8_linear_on_tile(int tile, const uint8_t *in_codes, const uint8_t *w_codes,
+                          uint16_t *out, size_t M, size_t N, size_t K, float output_scale,
+                          Fp8Mode mode, hipStream_t stream);
 // The MFMA-mode product (M <= 4) of the codes e4m3(bf16(norm(x)) *
 // input_scale), which the blocks form themselves (the codes rms_norm writes).
 Status fp8_linear_normed(const RowNorm &norm, float input_scale, const uint8_t *w_codes,

@@ -4,6 +4,9 @@
 Tolerances are stated per test: bit-exact for FP8 codes and the exact QGMMA
 mode; relative (to the output scale) for floating-point kernels.
 """
+import ctypes
+import os
+
 import numpy as np
 import pytest
 
@@ -267,9 +270,9 @@ def test_linear_tail_split_matches_unsplit(m, n, k, bias, residual):
     (130, 77, 64)])
 @pytest.mark.parametrize("planes,bias,residual", [(2, True, True), (1, False, False)])
 def test_linear_small_tiles_match_oracle(m, n, k, planes, bias, residual):
-    """Each block tile of the few-to-thousand-row products: ragged last tiles
-    in M and N, K of one step, of whole steps and with a last step of 1-3
-    32-K slices. The error of a split product is its activation's rounding,
+    """The few-to-thousand-row products on the tiles the launch rule picks for
+    them (test_linear_on_every_tile forces each): ragged last tiles in M and
+    N, K of one step, of whole steps and with a last step of 1-3 32-K slices. The error of a split product is its activation's rounding,
     2^-17 per term; F32 sums of K <= 416 terms add less. Rows past the
     output stay untouched."""
     r = rng(m + n + k + planes)
@@ -317,8 +320,9 @@ def test_linear_small_tiles_split_k(m, n, k):
                                            (300, 224, 4096), (520, 288, 4504)])
 @pytest.mark.parametrize("gelu,planes", [(1, 2), (0, 1)])
 def test_gated_mlp_small_tiles(m, width, inner, gelu, planes):
-    """The gated epilogue of each small tile (l1 and l2 columns of one tile
-    pair up), inner widths that end inside a 32-row block. One plane rounds
+    """The gated epilogue on the tiles the launch rule picks (l1 and l2 columns
+    of one tile pair up; test_gated_on_every_tile forces each), inner widths
+    that end inside a 32-row block. One plane rounds
     the gated activation to BF16: 2^-9 relative per term of the l3 sums."""
     from scipy.special import erf
     r = rng(m + width + inner + planes)
@@ -339,6 +343,114 @@ def test_gated_mlp_small_tiles(m, width, inner, gelu, planes):
     act = 0.5 * first * (1 + erf(first / np.sqrt(2))) if gelu else first
     expected = O.linear_bf16w((act * second).astype(np.float32), l3)
     assert rel_err(host(out), expected) < (1e-4 if planes == 2 else 2.0 ** -8)
+
+
+@pytest.fixture(scope="module")
+def tiles():
+    """Products on a given block tile (the library of test entry points)."""
+    N.load()
+    lib = ctypes.CDLL(os.path.join(os.path.dirname(N.LIBRARY_PATH), "libevo_hip_testing.so"))
+    size, void, number = ctypes.c_size_t, ctypes.c_void_p, ctypes.c_int
+    lib.evo_test_linear_on_tile.argtypes = [number, number, void, void, number, void, void, size,
+                                            size, size, void, void, void]
+    lib.evo_test_gated_on_tile.argtypes = [number, void, void, void, size, size, size, number,
+                                           void, void, void]
+    lib.evo_test_fp8_on_tile.argtypes = [number, void, void, void, size, size, size,
+                                         ctypes.c_float, number, void]
+    return lib
+
+
+# Block tiles of gemm_tile.hip: rows, columns.
+TILES = [(16, 16), (16, 32), (32, 32), (32, 64), (32, 96), (64, 64), (64, 128), (64, 192),
+         (128, 128), (128, 192)]
+
+
+def test_tile_list_is_complete(tiles):
+    assert tiles.evo_test_linear_tiles() == len(TILES) and tiles.evo_test_fp8_tiles() == 6
+
+
+@pytest.mark.parametrize("tile", range(len(TILES)))
+@pytest.mark.parametrize("planes", ["split", "bf16", "f16"])
+@pytest.mark.parametrize("k,parts", [(128, 1), (352, 1), (1088, 2), (2176, 4)])
+def test_linear_on_every_tile(tiles, tile, planes, k, parts):
+    """Each block tile with split-BF16, BF16 and FP16 operands: one row and
+    column past a whole number of tiles, K of whole steps and with a partial
+    last step of 1 to 3 32-K slices, in one part and in K parts that end in a
+    partial step (544 K). Operands on the oracle's side are the rounded ones;
+    F32 sums of up to 2176 products."""
+    bm, bn = TILES[tile]
+    m, n = 2 * bm + 1, 3 * bn + 4
+    r = rng(100 * tile + k + parts)
+    x = r.standard_normal((m, k)).astype(np.float32)
+    w = r.standard_normal((n, k)).astype(np.float32) / np.float32(np.sqrt(k))
+    res = r.standard_normal((m, n)).astype(np.float32)
+    if planes == "f16":
+        hi, lo, w_d = dev(x.astype(np.float16).view(np.uint16)), None, dev(
+            w.astype(np.float16).view(np.uint16))
+        x, w = x.astype(np.float16), w.astype(np.float16)
+    else:
+        hi, lo = split_gpu(x)
+        w_d = dev(bf16_bits(w))
+        w = bf16_to_f32(bf16_bits(w))
+        if planes == "bf16":
+            lo, x = None, bf16_to_f32(bf16_bits(x))
+    out, workspace = empty((m + 1, n)), empty((parts * m * n,))
+    out.fill_(7.0)
+    assert tiles.evo_test_linear_on_tile(tile, parts, p(hi), p(lo), int(planes == "f16"), p(w_d),
+                                         p(dev(res)), m, n, k, p(out), p(workspace),
+                                         stream()) == 0
+    got = host(out)
+    expected = x.astype(np.float64) @ w.astype(np.float64).T + res
+    assert rel_err(got[:m], expected) < 2e-5
+    assert np.all(got[m] == 7.0)
+
+
+@pytest.mark.parametrize("tile", range(1, len(TILES)))
+@pytest.mark.parametrize("planes,gelu", [(2, 1), (2, 0), (1, 0)])
+def test_gated_on_every_tile(tiles, tile, planes, gelu):
+    """The gated epilogue of each block tile that holds l1 and l2 columns
+    (16-column tiles do not), rows and inner width past whole tiles and inside
+    a 32-row weight block. Split output planes carry 2^-17 of a value, one
+    plane 2^-9."""
+    from scipy.special import erf
+    bm, bn = TILES[tile]
+    m, inner, width = bm + 3, 3 * (bn // 2) + 8, 352
+    r = rng(31 * tile + planes + gelu)
+    x = r.standard_normal((m, width)).astype(np.float32)
+    l1, l2 = (bf16_bits(r.standard_normal((inner, width)).astype(np.float32) / 18)
+              for _ in range(2))
+    w12 = zeros((2 * ((inner + 31) // 32 * 32), width), np.uint16)
+    N.call("evo_hip_pack_mlp", p(dev(l1)), p(dev(l2)), inner, width, p(w12), stream())
+    hi, lo = split_gpu(x)
+    if planes == 1:
+        x = bf16_to_f32(bf16_bits(x))
+    out = zeros((2, m + 1, inner), np.uint16)
+    assert tiles.evo_test_gated_on_tile(tile, p(hi), p(lo) if planes == 2 else None, p(w12), m,
+                                        width, inner, gelu, p(out[0]),
+                                        p(out[1]) if planes == 2 else None, stream()) == 0
+    got = host(out).view(np.uint16)
+    assert not got[:, m].any()
+    first = x.astype(np.float64) @ bf16_to_f32(l1).astype(np.float64).T
+    second = x.astype(np.float64) @ bf16_to_f32(l2).astype(np.float64).T
+    expected = (0.5 * first * (1 + erf(first / np.sqrt(2))) if gelu else first) * second
+    value = bf16_to_f32(got[0, :m]).astype(np.float64) + bf16_to_f32(got[1, :m])
+    assert rel_err(value, expected) < (2e-5 if planes == 2 else 2.0 ** -8)
+
+
+@pytest.mark.parametrize("tile", range(1, 6))
+@pytest.mark.parametrize("mode", [0, 1])
+@pytest.mark.parametrize("m,n,k", [(5, 70, 128), (131, 197, 640), (257, 449, 1152)])
+def test_fp8_on_every_tile_equals_the_first(tiles, tile, mode, m, n, k):
+    """Every block tile of the FP8 product gives the bits of the 128 x 192
+    tile, rows and columns past whole tiles, fewer steps than stages."""
+    r = rng(tile + m + k)
+    x, w = (dev(r.integers(0, 127, (rows, k)).astype(np.uint8)
+                | (r.integers(0, 2, (rows, k)).astype(np.uint8) << 7)) for rows in (m, n))
+    first, out = zeros((m + 1, n), np.uint16), zeros((m + 1, n), np.uint16)
+    for t, target in ((0, first), (tile, out)):
+        assert tiles.evo_test_fp8_on_tile(t, p(x), p(w), p(target), m, n, k, 2.0 ** -9, mode,
+                                          stream()) == 0
+    assert host(first).any() and np.array_equal(host(out), host(first))
 
 
 def split_gpu(x):
