@@ -16,13 +16,13 @@
 // the fragment reads a wave shape of the whole step would repeat; their sums
 // meet in LDS at the end.
 //
-// Measured (MI355X, split planes, weights from HBM; floor: their bytes at
-// the copy rate of 5 TB/s), against 256 x 256 tiles without a workspace:
-//   N = 22528, K = 4096 (gated):   5 rows 156 -> 34 us, 61 rows 150 -> 46,
-//     200 rows 157 -> 83, 700 rows 336 -> 239 (floor 37)
-//   N = 4096, K = 11264: 5 rows 390 -> 21 us, 61 rows 398 -> 37, 300 rows
-//     406 -> 89, 1000 rows 428 -> 157 (floor 18)
-//   N = K = 1920: 61 rows 79 -> 8 us, 1000 rows 88 -> 22.
+// Measured (MI355X, split planes, weights that no cache holds; floor: their
+// bytes at 5.4 TB/s), against 256 x 256 tiles without a workspace:
+//   N = 22528, K = 4096: 5 rows 154 -> 38 us, 61 rows 154 -> 50, 200 rows
+//     166 -> 89, 700 rows 351 -> 255 (floor 34)
+//   N = 4096, K = 11264: 5 rows 392 -> 22 us, 61 rows 393 -> 38, 300 rows
+//     416 -> 97, 1000 rows 434 -> 155 (floor 17)
+//   N = K = 1920: 61 rows 80 -> 8 us, 1000 rows 90 -> 23.
 #include <algorithm>
 #include <type_traits>
 
@@ -286,17 +286,18 @@ struct TileEntry {
   int bm, bn, seg;
   TileCost split, plane;  // hi + lo activation planes, one plane
 };
-// Least-squares fits over 5 to 8192 rows of the nine (N, K) of the 7B and 1B
-// topologies (median error 3-7 %; on that grid the tile the fit picks is
-// within 1 % of the fastest one in the geometric mean).
+// Least-squares fits over 5 to 3000 rows of twelve (N, K), those of the 7B and
+// 1B topologies among them (median error 3-6 %). With and without a workspace
+// the choice takes 0.3 to 0.8 % more than the fastest tile and split in the
+// geometric mean, 23 % at worst (2000 rows of 512 x 4096, no workspace).
 constexpr TileEntry kTiles[] = {
-    {16, 16, 128, {2.11F, 1.10F, 0.027F, 2, {0.186F, 0.292F}}, {2.59F, 0.66F, 0.004F, 3, {0.185F, 0.269F, 0.347F}}},
-    {16, 32, 128, {2.57F, 0.77F, 0.050F, 2, {0.256F, 0.379F}}, {2.40F, 0.94F, 0.017F, 2, {0.234F, 0.310F}}},
-    {32, 32, 128, {1.30F, 2.12F, 0.088F, 1, {0.276F}}, {1.75F, 1.83F, 0.030F, 1, {0.249F}}},
-    {32, 64, 128, {1.21F, 2.63F, 0.147F, 1, {0.350F}}, {1.53F, 2.18F, 0.055F, 1, {0.310F}}},
-    {32, 96, 128, {1.22F, 2.85F, 0.181F, 1, {0.429F}}, {1.56F, 2.32F, 0.095F, 1, {0.375F}}},
-    {64, 64, 64, {1.41F, 2.70F, 0.103F, 1, {0.276F}}, {2.01F, 2.15F, 0.040F, 2, {0.251F, 0.404F}}},
-    {64, 128, 64, {1.37F, 4.30F, 0.139F, 1, {0.406F}}, {1.63F, 3.55F, 0.074F, 1, {0.329F}}},
+    {16, 16, 128, {1.85F, 1.31F, 0.013F, 2, {0.209F, 0.361F}, 7.33F}, {2.09F, 1.09F, 0.0F, 3, {0.203F, 0.302F, 0.397F}, 5.36F}},
+    {16, 32, 128, {2.37F, 1.05F, 0.020F, 2, {0.276F, 0.481F}, 5.16F}, {2.12F, 1.09F, 0.013F, 2, {0.251F, 0.375F}, 5.22F}},
+    {32, 32, 128, {1.63F, 1.90F, 0.112F, 1, {0.278F}, 8.2F}, {1.73F, 1.77F, 0.040F, 1, {0.255F}, 5.39F}},
+    {32, 64, 128, {2.05F, 1.92F, 0.173F, 1, {0.381F}, 4.82F}, {2.11F, 1.83F, 0.078F, 1, {0.326F}, 4.90F}},
+    {32, 96, 128, {2.43F, 2.08F, 0.145F, 1, {0.510F}, 4.86F}, {2.40F, 1.88F, 0.076F, 1, {0.459F}, 4.93F}},
+    {64, 64, 64, {1.72F, 2.44F, 0.087F, 1, {0.296F}, 8.0F}, {2.10F, 2.31F, 0.017F, 2, {0.262F, 0.457F}, 5.07F}},
+    {64, 128, 64, {1.85F, 4.22F, 0.110F, 1, {0.412F}, 4.91F}, {1.99F, 3.66F, 0.051F, 1, {0.348F}, 4.82F}},
     {64, 192, 64, {1.17F, 5.72F, 0.144F, 1, {0.577F}}, {1.61F, 4.82F, 0.077F, 1, {0.474F}}},
     {128, 128, 64, {0.68F, 7.12F, 0.180F, 1, {0.691F}}, {1.06F, 6.14F, 0.149F, 1, {0.410F}}},
     {128, 192, 64, {1.28F, 7.28F, 0.280F, 1, {1.034F}}, {1.97F, 5.55F, 0.321F, 1, {0.709F}}},
@@ -317,11 +318,13 @@ double entry_us(const TileEntry &t, bool split, size_t M, size_t N, size_t K, si
 
 TileChoice choose_gemm_tile(size_t M, size_t N, size_t K, bool split, bool gated,
                             size_t large_parts, size_t workspace_bytes, bool deferred) {
-  // Partial products cost their reduction: a launch unless the next norm
-  // sums them as it reads its rows, and their bytes at ~4 TB/s.
+  // Partial products cost their reduction: a launch that grows with the parts
+  // (5 rows of 1920 x 5120, two planes: 4 parts 9.8 us, 8 parts 11.1) unless
+  // the next norm sums them as it reads its rows, and their bytes at ~4 TB/s.
   auto reduction = [&](size_t parts) {
     return parts == 1 ? 0.0
-                      : (deferred ? 0.0 : 3.0) + 4.0 * static_cast<double>(parts) * M * N / 4.0e6;
+                      : (deferred ? 0.0 : 2.0 + 0.3 * static_cast<double>(parts)) +
+                            4.0 * static_cast<double>(parts) * M * N / 4.0e6;
   };
   TileChoice best;
   double best_us = entry_us(kLargeTile, split, M, N, K, large_parts) + reduction(large_parts);
