@@ -105,3 +105,35 @@ def test_linear_tile(rules, m, n, k, planes, workspace, times):
                                       ctypes.byref(parts), ctypes.byref(tail))
     choice = LARGE if tile < 0 else (tile, parts.value)
     assert choice in times and times[choice] <= 1.10 * min(times.values())
+
+
+# (rows, N, K, promotion every 128 K or 32): us on the six block tiles of the
+# FP8 product, 128 x 192 first, weights that no cache holds.
+FP8 = [
+    (5, 12288, 4096, 1, (39.5, 33.9, 19.6, 13.5, 15.0, 13.1)),
+    (64, 12288, 4096, 1, (40.7, 34.7, 21.0, 14.7, 16.3, 19.0)),
+    (200, 12288, 4096, 1, (41.8, 34.6, 27.5, 29.3, 32.5, 41.1)),
+    (300, 12288, 4096, 1, (40.9, 35.4, 30.0, 37.2, 41.8, 55.2)),
+    (520, 12288, 4096, 1, (46.5, 67.9, 52.8, 59.8, 73.6, 89.0)),
+    (640, 12288, 4096, 1, (50.0, 68.3, 55.8, 66.3, 72.7, 102.7)),
+    (1024, 12288, 4096, 1, (56.2, 92.2, 78.7, 97.0, 110.8, 156.8)),
+    (8192, 12288, 4096, 1, (418.5, 484.3, 550.4, 679.1, 727.7, 1178.4)),
+    (130, 5760, 1920, 1, (21.5, 17.6, 10.9, 10.6, 8.5, 9.8)),
+    (777, 5760, 1920, 1, (22.7, 19.4, 22.5, 25.0, 24.9, 34.8)),
+    (1300, 5760, 1920, 1, (27.7, 35.2, 28.7, 35.3, 36.1, 54.3)),
+    (2049, 5760, 1920, 1, (32.2, 39.4, 42.3, 52.4, 59.2, 83.3)),
+    (1024, 3072, 1024, 1, (15.7, 12.2, 10.5, 11.7, 12.0, 17.0)),
+    (16, 12288, 4096, 0, (51.2, 35.5, 24.6, 17.6, 18.0, 17.5)),
+    (200, 12288, 4096, 0, (53.2, 44.4, 33.9, 35.5, 38.8, 54.1)),
+    (400, 12288, 4096, 0, (54.3, 48.3, 52.8, 57.6, 60.3, 88.7)),
+    (900, 12288, 4096, 0, (86.2, 90.8, 95.5, 113.0, 117.6, 187.2)),
+    (3000, 12288, 4096, 0, (251.0, 261.9, 276.7, 327.3, 341.9, 591.4)),
+    (640, 5760, 1920, 0, (28.9, 24.5, 19.9, 23.1, 24.8, 37.4)),
+    (1300, 5760, 1920, 0, (41.8, 38.2, 35.3, 42.1, 43.1, 69.2)),
+]
+
+
+@pytest.mark.parametrize("m,n,k,k128,times", FP8)
+def test_fp8_tile(rules, m, n, k, k128, times):
+    tile = rules.evo_test_fp8_tile(m, n, k, k128)
+    assert times[tile] <= SLACK * min(times) and times[tile] <= 1.02 * times[0]
