@@ -286,10 +286,11 @@ struct TileEntry {
   int bm, bn, seg;
   TileCost split, plane;  // hi + lo activation planes, one plane
 };
-// Least-squares fits over 5 to 3000 rows of twelve (N, K), those of the 7B and
-// 1B topologies among them (median error 3-6 %). With and without a workspace
-// the choice takes 0.3 to 0.8 % more than the fastest tile and split in the
-// geometric mean, 23 % at worst (2000 rows of 512 x 4096, no workspace).
+// Least-squares fits over 5 to 8192 rows of ten (N, K), those of the 7B and 1B
+// topologies among them (median error 2-6 %). With and without a workspace
+// the choice takes 1.2 % (up to 150 rows) or 0.4 % more than the fastest tile
+// and split in the geometric mean, 24 % at worst (1000 rows of 512 x 4096), and
+// nowhere over 1 % more than the 256 x 256 tile.
 constexpr TileEntry kTiles[] = {
     {16, 16, 128, {1.85F, 1.31F, 0.013F, 2, {0.209F, 0.361F}, 7.33F}, {2.09F, 1.09F, 0.0F, 3, {0.203F, 0.302F, 0.397F}, 5.36F}},
     {16, 32, 128, {2.37F, 1.05F, 0.020F, 2, {0.276F, 0.481F}, 5.16F}, {2.12F, 1.09F, 0.013F, 2, {0.251F, 0.375F}, 5.22F}},
@@ -297,21 +298,32 @@ constexpr TileEntry kTiles[] = {
     {32, 64, 128, {2.05F, 1.92F, 0.173F, 1, {0.381F}, 4.82F}, {2.11F, 1.83F, 0.078F, 1, {0.326F}, 4.90F}},
     {32, 96, 128, {2.43F, 2.08F, 0.145F, 1, {0.510F}, 4.86F}, {2.40F, 1.88F, 0.076F, 1, {0.459F}, 4.93F}},
     {64, 64, 64, {1.72F, 2.44F, 0.087F, 1, {0.296F}, 8.0F}, {2.10F, 2.31F, 0.017F, 2, {0.262F, 0.457F}, 5.07F}},
-    {64, 128, 64, {1.85F, 4.22F, 0.110F, 1, {0.412F}, 4.91F}, {1.99F, 3.66F, 0.051F, 1, {0.348F}, 4.82F}},
-    {64, 192, 64, {1.17F, 5.72F, 0.144F, 1, {0.577F}}, {1.61F, 4.82F, 0.077F, 1, {0.474F}}},
-    {128, 128, 64, {0.68F, 7.12F, 0.180F, 1, {0.691F}}, {1.06F, 6.14F, 0.149F, 1, {0.410F}}},
-    {128, 192, 64, {1.28F, 7.28F, 0.280F, 1, {1.034F}}, {1.97F, 5.55F, 0.321F, 1, {0.709F}}},
+    {64, 128, 64, {2.49F, 4.02F, 0.121F, 1, {0.413F}, 4.39F, 6.93F}, {3.07F, 3.34F, 0.069F, 1, {0.338F}, 4.30F}},
+    {64, 192, 64, {2.30F, 5.65F, 0.158F, 1, {0.564F}, 4.56F, 6.36F}, {3.16F, 4.74F, 0.068F, 1, {0.488F}, 4.27F}},
+    {128, 128, 64, {1.97F, 5.73F, 0.181F, 1, {0.700F}, 9.0F, 6.66F}, {1.30F, 6.29F, 0.120F, 1, {0.439F}, 4.39F, 6.42F}},
+    {128, 192, 64, {2.69F, 6.49F, 0.250F, 1, {1.059F}, 4.33F, 5.59F}, {3.66F, 5.62F, 0.209F, 1, {0.834F}, 4.12F}},
 };
 constexpr int kTileCount = static_cast<int>(sizeof(kTiles) / sizeof(kTiles[0]));
 static_assert(kTileCount == kGemmTiles, "the tiles of gemm_tile()");
 // The 256 x 256 tile of gemm.hip, the other candidate.
-constexpr TileEntry kLargeTile = {256, 256, 32, {0.0F, 9.34F, 0.294F, 1, {1.094F}},
-                                  {0.0F, 9.14F, 0.165F, 1, {0.737F}}};
+constexpr TileEntry kLargeTile = {256, 256, 32, {0.0F, 7.29F, 0.532F, 1, {1.041F}},
+                                  {0.0F, 7.71F, 0.233F, 1, {0.750F}}};
+// A small tile has to come out this much below 256 x 256, twice the fits'
+// error: with less, products of a few thousand rows were slower than there by
+// up to 10 % (5000 rows of 4096 x 4096, two planes: 407 us on 128 x 128, 366 on
+// 256 x 256), and without it the choice is no faster in the mean.
+constexpr double kSmallMargin = 1.07;
 
 double entry_us(const TileEntry &t, bool split, size_t M, size_t N, size_t K, size_t parts) {
-  return tile_us(split ? t.split : t.plane,
-                 static_cast<double>(ceil_div(M, t.bm)) * ceil_div(N, t.bn) * parts,
-                 ceil_div(K / parts, t.seg), 2.0 * static_cast<double>(N) * K);
+  const TileCost &cost = split ? t.split : t.plane;
+  const double blocks = static_cast<double>(ceil_div(M, t.bm)) * ceil_div(N, t.bn) * parts;
+  // An XCD's resident blocks are consecutive, rows first: 32 row blocks and
+  // more share no activation rows, which each block column then reads again.
+  const double resident = std::min(32.0 * cost.slots, std::max(1.0, blocks / 8.0));
+  const double down = std::min<double>(ceil_div(M, t.bm), resident);
+  const double rows = down * t.bm * (split ? 2 : 1) + std::max(1.0, resident / down) * t.bn;
+  return tile_us(cost, blocks, ceil_div(K / parts, t.seg), 2.0 * static_cast<double>(N) * K,
+                 blocks / resident * rows * 2.0 * static_cast<double>(K / parts));
 }
 
 }  // namespace
@@ -338,7 +350,8 @@ TileChoice choose_gemm_tile(size_t M, size_t N, size_t K, bool split, bool gated
       if (parts > 1 && (K / parts < 4 * seg || N % 4 != 0 || gated ||
                         parts * M * N * sizeof(float) > workspace_bytes))
         continue;
-      const double us = entry_us(kTiles[t], split, M, N, K, parts) + reduction(parts);
+      const double us =
+          kSmallMargin * (entry_us(kTiles[t], split, M, N, K, parts) + reduction(parts));
       if (us < best_us) {
         best_us = us;
         best = TileChoice{t, static_cast<int>(parts)};
