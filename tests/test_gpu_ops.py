@@ -876,8 +876,9 @@ def test_hcm_stream_mfma_matches_oracle(inner_len, length, width, groups, dtype)
 @pytest.mark.parametrize("length", [2, 31, 129, 300, 1025])
 @pytest.mark.parametrize("dtype", [N.DTYPE_F32, N.DTYPE_SPLIT, N.DTYPE_BF16_F16])
 def test_hyena_group_sizes_off_16(kind, inner_len, groups, width, length, dtype):
-    """Filter groups whose size is no multiple of 16 (15 channels in the 1B
-    topology; 48, 16 and 17 here too): slices with two groups' filters. F32
+    """Filter groups of 15 channels (the 1B topology; 16-channel slices with two
+    groups' filters), 17 (odd HCS pairs), and for comparison 48 and 16, whose
+    slices hold one (test_hcm_group_sizes_above_16 has the others). F32
     output: u in three BF16 planes (2^-24) and F32 sums of 128 terms; the
     16-bit outputs round once (2^-17, 2^-11)."""
     case = hyena_case(length + width + inner_len, kind, length, width, groups=groups,
@@ -947,6 +948,70 @@ def hyena_exact(kind, case, projection, short_history, inner_history):
     if "direct" in case:
         y = y + u[k - 1:] * case["direct"]
     return fir[:, :, 0] * y
+
+
+@pytest.mark.parametrize("groups,width", [(64, 1088), (8, 192), (8, 320)])
+@pytest.mark.parametrize("inner_len", [128, 33])
+@pytest.mark.parametrize("dtype", [N.DTYPE_F32, N.DTYPE_BF16_F16])
+@pytest.mark.parametrize("length", [31, 300])
+def test_hcm_group_sizes_above_16(groups, width, inner_len, dtype, length):
+    """Groups of 17, 24 and 40 channels: some 16-channel slices touch two groups
+    and some lie in one. Against 64 bits, whole and continued after a first
+    call; bounds as in test_hyena_group_sizes_off_16."""
+    case = hyena_case(length + width + inner_len, N.HYENA_HCM, length, width, groups=groups,
+                      inner_len=inner_len)
+    proj = case["projection"]
+    if dtype == N.DTYPE_BF16_F16:
+        proj = bf16_to_f32(bf16_bits(proj))
+    none = np.zeros((2, 3 * width)), np.zeros((inner_len - 1, width))
+    expected = hyena_exact(N.HYENA_HCM, case, proj, *none)
+    bound = 2e-6 if dtype == N.DTYPE_F32 else 2.0 ** -11
+    assert rel_err(hyena_gpu(N.HYENA_HCM, case, dtype=dtype, projection=proj, bf16_taps=True),
+                   expected) < bound
+    for split in (1, length // 2):
+        caches = dict(short=zeros((2, 3 * width)), inner=zeros((inner_len - 1, width)))
+        parts = [hyena_gpu(N.HYENA_HCM, case, dtype=dtype, projection=part, caches=caches,
+                           bf16_taps=True) for part in (proj[:split], proj[split:])]
+        assert rel_err(np.concatenate(parts), expected) < bound
+
+
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan, 3.39e38])
+@pytest.mark.parametrize("kind,inner_len,groups,width", [
+    (N.HYENA_HCM, 128, 64, 960), (N.HYENA_HCM, 33, 8, 192), (N.HYENA_HCM, 128, 8, 320),
+    (N.HYENA_HCS, 7, 64, 960)])
+@pytest.mark.parametrize("dtype", [N.DTYPE_F32, N.DTYPE_BF16])
+@pytest.mark.parametrize("length", [3, 200])
+def test_hyena_non_finite_histories_stay_local(value, kind, inner_len, groups, width, dtype,
+                                               length):
+    """Infinities, NaN and values that round to an infinite BF16 one, in the
+    oldest, a middle and the newest row of the inner history and in the short
+    history, reach the outputs whose windows hold them, of their own channels,
+    and no other."""
+    case = hyena_case(length + width, kind, length, width, groups=groups, inner_len=inner_len)
+    r = rng(width + inner_len)
+    short = r.standard_normal((2, 3 * width)).astype(np.float32)
+    inner = r.standard_normal((inner_len - 1, width)).astype(np.float32)
+    for row, channel in ((0, 14), (inner_len // 2, 15), (inner_len - 2, width - 16)):
+        inner[row, channel] = value
+    short[1, 3 * (width - 1) + 1] = value
+    proj = case["projection"]
+    if dtype == N.DTYPE_BF16:
+        proj = bf16_to_f32(bf16_bits(proj))
+    with np.errstate(invalid="ignore", over="ignore"):
+        expected = hyena_exact(kind, case, proj, short, inner)
+    actual = hyena_gpu(kind, case, dtype=dtype, projection=proj, bf16_taps=True,
+                       caches=dict(short=dev(short), inner=dev(inner)))
+    reached = np.zeros((length, width), bool)
+    for row, channel in ((0, 14), (inner_len // 2, 15), (inner_len - 2, width - 16)):
+        reached[:row + 1, channel] = True
+    reached[:inner_len + 1, width - 1] = True
+    assert rel_err(actual[~reached], expected[~reached]) < (
+        2e-6 if dtype == N.DTYPE_F32 else 2.0 ** -8)
+    if not np.isfinite(value):
+        assert np.array_equal(np.isnan(actual), np.isnan(expected))
+        odd = ~np.isfinite(expected)
+        assert odd[0, 14] and odd[0, 15] and odd[0, width - 16] and odd[0, width - 1]
+        assert np.array_equal(actual[odd], expected[odd].astype(np.float32), equal_nan=True)
 
 
 @pytest.mark.parametrize("kind,inner_len,groups,width", [
