@@ -802,8 +802,12 @@ Status launch_flash(const uint16_t *q, size_t q_plane, const uint16_t *k_cache,
 // Full-softmax semantics as `src/cpu/model.cpp:510-544`.
 // Bound by the latency of its loads at short prefixes (keys in chunks of 256,
 // a key per lane, V after the softmax took 17.3 us at 1040 keys x 32 heads of
-// 128, this 10.3) and by the cache's bytes at long ones.
-constexpr int kDecodeKeys = 256;  // most keys per chunk of a minimal workspace
+// 128, this 10.3) and by the cache's bytes at long ones (with the append, 32
+// heads of 128: 8192 keys 175 -> 53.5 us, 32768 keys 772 -> 204, 131072 keys
+// 2866 -> 802, 5.4 TB/s).
+// Keys per chunk for which a workspace has to hold the parts; one that holds
+// no more runs chunks of at least this length.
+constexpr int kDecodeKeys = 256;
 constexpr int kDecodeTile = 64;
 
 template <int kD>
@@ -960,8 +964,8 @@ Status launch_decode(const uint16_t *q, size_t q_plane, const uint16_t *k_cache,
                      const uint16_t *v_cache, size_t cache_plane, size_t capacity, size_t keys,
                      size_t heads, float *workspace, size_t workspace_bytes, O out,
                      hipStream_t stream) {
-  // The fewest tiles per chunk that leave at most about 8 blocks per CU (a
-  // combine over a bounded number of chunks) and whose parts fit.
+  // One tile per chunk below 4096 blocks (16 per CU), then the most tiles that
+  // leave 2048; no more than 512 chunks to combine, and parts that fit.
   const size_t tiles = ceil_div(keys, kDecodeTile);
   const size_t part = heads * (kD + 2) * sizeof(float);
   size_t chunk_tiles = std::max<size_t>(1, tiles * heads / 2048);

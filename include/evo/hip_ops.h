@@ -250,14 +250,17 @@ EVO_API evo_status evo_hip_attention(const float *projected, size_t rows,
                                      uint16_t *value_cache, size_t capacity,
                                      float *out, void *stream);
 
-/* evo_hip_attention with an F32 device workspace: a single query (rows == 1,
- * head_dim 32/64/128) is then split over its keys in chunks of at most 256
- * where the workspace holds no more, and of 64 and up otherwise (per chunk
- * and head: max, sum and head_dim partial outputs in the workspace), the
- * decode step's path; and a few rows, or the last rows of a prompt, over
- * parts of their keys where the workspace holds the parts (rows x heads x
- * parts x (head_dim + 2) floats) and that is faster. The same reference
- * interface. */
+/* evo_hip_attention with an F32 device workspace, the decode step's path:
+ * - A single query (rows == 1, head_dim 32/64/128) is split over its keys if
+ *   the workspace holds a part (max, sum and head_dim outputs: head_dim + 2
+ *   floats) per head and 256 keys. Chunks are whole 64-key tiles: one each
+ *   below 4096 blocks (tiles x heads) and up to 512 chunks, more beyond that,
+ *   and at least four where the workspace holds no more parts (32 heads: 64
+ *   keys per chunk at 4096 keys, 512 at 32768, 2048 at 131072).
+ * - A few rows, or the last rows of a prompt, are split over parts of their
+ *   keys where that is faster and the workspace holds the parts (rows, rounded
+ *   up to 128 or 256, x heads x parts x (head_dim + 2) floats).
+ * The same reference interface. */
 EVO_API evo_status evo_hip_attention_ws(const float *projected, size_t rows,
                                         size_t width, size_t heads,
                                         int column_split, const float *inv_freq,

@@ -1313,10 +1313,11 @@ def test_attention_split_keeps_non_finite_rows(value):
 
 
 @pytest.mark.parametrize("heads,head_dim,prefix", [
-    (2, 128, 62), (2, 128, 63), (3, 64, 64), (40, 128, 5000), (2, 32, 32900)])
+    (2, 128, 62), (2, 128, 63), (3, 64, 64), (40, 128, 5000), (2, 32, 32900),
+    (64, 32, 13000)])
 def test_single_query_chunks(heads, head_dim, prefix):
     """One query split in chunks of 64 keys (a large workspace) or more (a
-    minimal one, long prefixes), against the 64-bit softmax over the cached
+    minimal one, long prefixes, many heads: six tiles of 64), against the 64-bit softmax over the cached
     planes: F32 dots and sums of head_dim and prefix terms of either sign,
     1e-6 of the output in the root mean square. Cache columns past the last
     key may hold anything."""
