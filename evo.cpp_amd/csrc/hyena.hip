@@ -1357,8 +1357,6 @@ template <> struct MsOut<SplitOut> {
   }
 };
 
-// Two blocks per CU for BF16 projections (71 KB of LDS); F32 projection
-// rows double the DMA stage (97 KB), so one block per CU.
 // Y + d u of one output, tap by tap in the reference's order (short FIR of
 // 3), u recomputed from the projection or read from the inner history.
 template <typename T>
@@ -1398,6 +1396,9 @@ __device__ float hcm_window_sum(const T *P, const float *short_history,
 // zero taps: production flags such steps, and outputs whose window holds one
 // are summed tap by tap (hcm_window_sum). 8192 rows at W = 1920:
 // 2505 -> 74 us (BF16), 2529 -> 97 us (F32).
+// Two blocks per CU for BF16 projections (71 KB of LDS); one where F32
+// projection rows double the DMA stage (97 KB) or u has a third plane (81 KB,
+// with F32 rows 107).
 template <typename T, typename O, bool kTwoGroups>
 __global__ __launch_bounds__(256, sizeof(T) == 2 && !kTwoGroups ? 2 : 1) void hyena_fir_mfma_stream_kernel(
     const T *__restrict__ P, const float *__restrict__ short_history,

@@ -501,7 +501,6 @@ Status Context::initialize(std::shared_ptr<const Model> model, size_t capacity,
     r.buffer->view(arena_.as<char>() + offset, r.bytes);
     offset += (r.bytes + kPage - 1) / kPage * kPage;
   }
-  tokens_.view(io_.as<char>(), token_bytes);
   flag_.view(io_.as<char>() + token_bytes, sizeof(int));
   logits_.view(io_.as<char>() + token_bytes + kFlagBytes, logit_bytes);
   EVO_TRY(hip_check(hipHostMalloc(&pinned_, token_bytes + 2 * kFlagBytes + logit_bytes,

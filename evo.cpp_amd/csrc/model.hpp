@@ -176,7 +176,7 @@ private:
   // tokens, right-aligned, and a zero for the flag) and its download (flag
   // and logits) are one copy each.
   DeviceBuffer io_;
-  DeviceBuffer tokens_, hidden_, residual_, normed_, projected_, mixed_, query_,
+  DeviceBuffer hidden_, residual_, normed_, projected_, mixed_, query_,
       gated_, logits_, codes_, workspace_, flag_;
   size_t workspace_bytes_{0};
   struct Cache {
