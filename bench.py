@@ -19,6 +19,7 @@ of the same artifact.
 """
 import argparse
 import ctypes
+import itertools
 import json
 import re
 import os
@@ -129,22 +130,27 @@ def kernel_rooflines(split):
     # (the FP8 projection's output), out as one BF16 plane (config 2's
     # format), one FP16 plane (the benchmarked context's) and split BF16
     # planes [2, 8192, 4096] (contexts without +f16-out), 7B filter groups
-    # (256) and tap counts (HCS 7, HCM 128, HCL 16 states).
+    # (256) and tap counts (HCS 7, HCM 128, HCL 16 states). Four projections
+    # and outputs in turn: one projection (201 MB) would stay in the 256 MB
+    # memory-side cache, and its reads would not be HBM's.
     length, width, state, groups = 8192, 4096, 16, 256
-    proj = torch.randn(length, 3 * width, device="cuda", generator=g).to(torch.bfloat16)
+    turns = 4
+    proj = [torch.randn(length, 3 * width, device="cuda", generator=g).to(torch.bfloat16)
+            for _ in range(turns)]
     short = (torch.randn(3 * width, 3, device="cuda", generator=g) * 0.3).to(torch.bfloat16)
     poles = torch.rand(width, state, device="cuda", generator=g) * 0.49 + 0.5
     residues = torch.randn(width, state, device="cuda", generator=g) * 0.02
     direct = torch.randn(width, device="cuda", generator=g) * 0.02
-    planes_out = torch.empty(2, length, width, dtype=torch.int16, device="cuda")
+    planes_out = [torch.empty(2, length, width, dtype=torch.int16, device="cuda")
+                  for _ in range(turns)]
     hbm_bytes = length * 3 * width * 2 + length * width * 4
     bf16_bytes = length * 3 * width * 2 + length * width * 2
     out["hyena"] = []
     for kind, name, taps, profiled in (
             (1, "HCM FIR, 128 taps (hyena_fir_mfma_stream_kernel)", 128,
-             "hyena_fir_mfma_stream_kernel<unsigned short, unsigned short*>"),
+             "hyena_fir_mfma_stream_kernel<unsigned short, unsigned short*, false>"),
             (0, "HCS FIR, 7 taps (hyena_fir_stream_kernel)", 7,
-             "hyena_fir_stream_kernel<unsigned short, unsigned short*, 3, 7, false>"),
+             "hyena_fir_stream_kernel<unsigned short, unsigned short*, 3, 7, false, false>"),
             (2, "HCL, 16 modal states (hcl_mfma_kernel)", 0,
              "hcl_mfma_kernel<unsigned short, unsigned short*>")):
         filt = (torch.randn(groups, max(taps, 1), device="cuda", generator=g)
@@ -154,12 +160,17 @@ def kernel_rooflines(split):
         ws = torch.empty(max(ws_bytes, 256), dtype=torch.uint8, device="cuda")
         times = {}
         for dtype in (native.DTYPE_BF16, native.DTYPE_BF16_SPLIT, native.DTYPE_BF16_F16):
-            times[dtype] = event_time(lambda: native.call(
-                "evo_hip_hyena_forward", kind, dtype | native.DTYPE_BF16_TAPS,
-                proj.data_ptr(), length,
-                width, short.data_ptr(), 3, filt.data_ptr(), groups, taps, direct.data_ptr(),
-                poles.data_ptr(), residues.data_ptr(), st, None, None, None, ws.data_ptr(),
-                ws_bytes, planes_out.data_ptr(), stream), 10)
+            turn = itertools.cycle(range(turns))
+
+            def launch():
+                i = next(turn)
+                native.call(
+                    "evo_hip_hyena_forward", kind, dtype | native.DTYPE_BF16_TAPS,
+                    proj[i].data_ptr(), length, width, short.data_ptr(), 3, filt.data_ptr(),
+                    groups, taps, direct.data_ptr(), poles.data_ptr(), residues.data_ptr(), st,
+                    None, None, None, ws.data_ptr(), ws_bytes, planes_out[i].data_ptr(), stream)
+
+            times[dtype] = event_time(launch, 10)
         ms, ms_split = times[native.DTYPE_BF16], times[native.DTYPE_BF16_SPLIT]
         ms_f16 = times[native.DTYPE_BF16_F16]
         out["hyena"].append(dict(kernel=name, profiled=profiled, ms=ms, bytes=bf16_bytes, gbs=bf16_bytes / ms / 1e6,
