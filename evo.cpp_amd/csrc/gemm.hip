@@ -915,9 +915,11 @@ LinearPlan plan_linear(size_t M, size_t N, size_t K, bool split, bool gated,
       2 * last * kBM * kBN * sizeof(float) <= workspace_bytes)
     plan.tail = last;
   // The small tiles of gemm_tile.hip where their measured cost is lower. A
-  // tail-split launch stays here: more than one full round of 256 x 256
-  // tiles, no CU left idle (7B MLP l1/l2 of 1000 rows: 296 us against 335
-  // on the best small tile, 348 without the tail split).
+  // tail-split launch stays here without a comparison: more than one full
+  // round of 256 x 256 tiles, no CU left idle. It is the faster one in most
+  // cases (7B MLP l1/l2 of 1000 rows: 296 us against 335 on the best small
+  // tile, 348 without the tail split) but not in all (520 rows of it 264 us,
+  // 235 on 64 x 192; 1300 rows of 12288 x 4096 289 and 261).
   if (plan.tail == 0)
     plan.choice = choose_gemm_tile(M, N, K, split, gated, static_cast<size_t>(splits), part_bytes,
                                    deferred);
