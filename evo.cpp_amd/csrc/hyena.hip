@@ -2918,13 +2918,20 @@ unsigned hcs_stream_segment(size_t width, size_t length, bool f32_exact) {
   return rows;
 }
 
-// A slice of 16 channels touches at most two groups of 15 and more. With F32
-// rows the stream's prologue (two filters' Toeplitz fragments, 107 KB of LDS)
-// is longer than the tap-by-tap sums of a few rows of a short filter: 2 rows
-// of 40 taps with the caches take 17.9 us tap by tap and 19.1 here, 5 rows
-// 21.3 and 20.8, 2 rows of 128 taps 29.7 and 25.6.
-bool hcm_stream_two_groups(size_t group_size, size_t length, int taps, bool f32) {
-  return group_size >= 15 && !(f32 && length * static_cast<size_t>(taps) <= 96);
+// A slice of 16 channels touches at most two groups of 15 and more. The
+// stream's prologue (two filters' Toeplitz fragments, 81 or 107 KB of LDS, the
+// window's rows of the inner history) is longer than the tap-by-tap sums of a
+// few rows of a short filter, and longer still where the filters can't come by
+// DMA (taps % 4). Tap by tap and here, us, with the caches: F32 2 rows of 40
+// taps 17.9 and 19.1, 4 rows 17.7 and 18.6, 5 rows 20.6 and 19.3, 4 rows of 33
+// 16.7 and 18.3; BF16 2 rows of 10 14.2 and 16.5, 4 rows of 20 15.6 and 16.6, 5
+// rows 18.1 and 17.4, 2 rows of 64 21.1 and 19.2. Without: F32 3 rows of 40 9.5
+// and 8.8, of 33 8.5 and 9.0; BF16 2 rows of 20 8.9 and 8.2, of 10 8.0 and 8.7.
+bool hcm_stream_two_groups(size_t group_size, size_t length, int taps, bool f32, bool caches) {
+  size_t row_taps = f32 ? (caches ? 160 : 99) : (caches ? 80 : 30);
+  if (taps % 4 != 0)
+    row_taps += row_taps / 3;
+  return group_size >= 15 && length * static_cast<size_t>(taps) > row_taps;
 }
 
 size_t hyena_workspace_bytes(int kind, size_t length, size_t width,
@@ -3042,7 +3049,8 @@ Status hyena_forward(int kind, const T *projection, size_t length,
                                        stream)));
     } else if (wt.taps_bf16 && short_len == 3 && planar == 0 && width % kMsChannels == 0 &&
                direct != nullptr &&
-               (!two_groups || (hcm_stream_two_groups(group_size, length, k, sizeof(T) == 4) &&
+               (!two_groups || (hcm_stream_two_groups(group_size, length, k, sizeof(T) == 4,
+                                                       inner_history != nullptr) &&
                                 is_aligned(projection, 16) && is_aligned(out, 16)))) {
       const unsigned cblocks = static_cast<unsigned>(width / kMsChannels);
       const unsigned seg_len = ms_segment(cblocks, length, sizeof(T) == 2 && !two_groups);

@@ -41,6 +41,6 @@ unsigned hcs_stream_segment(size_t width, size_t length, bool f32_exact);
 
 // Whether the HCM row stream takes filter groups that are no multiple of 16
 // (hyena.hip), rows and outputs aligned.
-bool hcm_stream_two_groups(size_t group_size, size_t length, int taps, bool f32);
+bool hcm_stream_two_groups(size_t group_size, size_t length, int taps, bool f32, bool caches);
 
 }  // namespace evo::hip

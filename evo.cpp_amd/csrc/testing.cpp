@@ -15,8 +15,8 @@ EVO_TEST_API unsigned evo_test_hcs_stream_segment(size_t width, size_t length, i
 }
 
 EVO_TEST_API int evo_test_hcm_stream_two_groups(size_t group_size, size_t length, int taps,
-                                                int f32) {
-  return evo::hip::hcm_stream_two_groups(group_size, length, taps, f32 != 0) ? 1 : 0;
+                                                int f32, int caches) {
+  return evo::hip::hcm_stream_two_groups(group_size, length, taps, f32 != 0, caches != 0) ? 1 : 0;
 }
 
 // Tile of a dense product (-1: 256 x 256); its K parts and tail tiles.

@@ -18,7 +18,7 @@ def rules():
     size = ctypes.c_size_t
     lib.evo_test_hcs_stream_segment.argtypes = [size, size, ctypes.c_int]
     lib.evo_test_hcs_stream_segment.restype = ctypes.c_uint
-    lib.evo_test_hcm_stream_two_groups.argtypes = [size, size, ctypes.c_int, ctypes.c_int]
+    lib.evo_test_hcm_stream_two_groups.argtypes = [size, size] + 3 * [ctypes.c_int]
     lib.evo_test_linear_plan.argtypes = [size, size, size, ctypes.c_int, ctypes.c_int, size,
                                          ctypes.POINTER(ctypes.c_int), ctypes.POINTER(size)]
     lib.evo_test_fp8_tile.argtypes = [size, size, size, ctypes.c_int]
@@ -47,24 +47,33 @@ def test_hcs_stream_segment(rules, width, length, f32_exact, times):
     assert times[(16, 32, 64, 128).index(rows)] <= SLACK * min(times)
 
 
-# (group size, length, taps, F32 rows): us tap by tap and on the row stream,
-# with the caches.
+# (group size, length, taps, F32 rows, caches): us tap by tap and on the row
+# stream.
 HCM_TWO_GROUPS = [
-    (15, 2, 40, 1, (18.1, 19.2)), (24, 2, 40, 1, (17.9, 19.1)), (17, 2, 40, 1, (18.0, 19.1)),
-    (15, 5, 40, 1, (21.3, 20.8)), (15, 2, 128, 1, (29.7, 25.6)), (15, 17, 40, 1, (32.4, 23.1)),
-    (15, 2, 128, 0, (31.2, 25.0)), (15, 5, 40, 0, (21.9, 20.0)),
+    (15, 2, 40, 1, 1, (18.1, 19.2)), (24, 2, 40, 1, 1, (17.9, 19.1)),
+    (17, 2, 40, 1, 1, (18.0, 19.1)), (15, 5, 40, 1, 1, (21.3, 20.8)),
+    (15, 2, 128, 1, 1, (29.7, 25.6)), (15, 17, 40, 1, 1, (32.4, 23.1)),
+    (15, 2, 128, 0, 1, (31.2, 25.0)), (15, 5, 40, 0, 1, (21.9, 20.0)),
+    (15, 2, 10, 0, 1, (14.2, 16.5)), (24, 4, 10, 0, 0, (8.3, 8.7)), (15, 7, 10, 0, 1, (16.7, 17.3)),
+    (24, 4, 20, 0, 1, (15.6, 16.6)), (15, 2, 20, 0, 0, (8.9, 8.2)),
+    (24, 3, 33, 0, 1, (17.0, 17.8)),
+    (15, 7, 20, 0, 1, (18.4, 17.4)), (24, 2, 64, 0, 1, (21.1, 19.2)),
+    (15, 3, 33, 1, 1, (16.5, 18.3)),
+    (24, 4, 33, 1, 0, (8.6, 9.0)), (15, 4, 40, 1, 1, (17.7, 18.6)), (15, 5, 20, 1, 0, (9.6, 8.9)),
+    (15, 5, 20, 1, 1, (17.3, 18.1)), (24, 3, 64, 1, 1, (19.9, 19.7)), (15, 5, 40, 1, 1, (20.6, 19.3)),
+    (15, 3, 40, 1, 0, (9.5, 8.8)),
 ]
 
 
-@pytest.mark.parametrize("group_size,length,taps,f32,times", HCM_TWO_GROUPS)
-def test_hcm_stream_two_groups(rules, group_size, length, taps, f32, times):
-    streamed = rules.evo_test_hcm_stream_two_groups(group_size, length, taps, f32)
+@pytest.mark.parametrize("group_size,length,taps,f32,caches,times", HCM_TWO_GROUPS)
+def test_hcm_stream_two_groups(rules, group_size, length, taps, f32, caches, times):
+    streamed = rules.evo_test_hcm_stream_two_groups(group_size, length, taps, f32, caches)
     assert times[streamed] == min(times)
 
 
 def test_hcm_stream_leaves_small_groups(rules):
     """A slice of 16 channels may touch three groups of 14."""
-    assert not rules.evo_test_hcm_stream_two_groups(14, 1000, 128, 0)
+    assert not rules.evo_test_hcm_stream_two_groups(14, 1000, 128, 0, 1)
 
 
 LARGE = "256 x 256"
