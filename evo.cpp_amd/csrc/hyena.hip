@@ -2787,7 +2787,8 @@ void launch_fir_stream_taps(const T *projection, const float *short_history,
                             size_t group_size, int k, int causal, const float *direct,
                             size_t length, size_t width, O out, hipStream_t stream) {
   const unsigned cblocks = ceil_div(width, kStreamChannels);
-  const unsigned seg_len = hcs_stream_segment(width, length, sizeof(T) == 4 && kWin == 3);
+  const unsigned seg_len = hcs_stream_segment(width, length, sizeof(T) == 4, kWin == 3,
+                                              std::is_same<O, float *>::value);
   const unsigned segments = ceil_div(length, seg_len);
   const dim3 grid(cblocks * segments), block(kStreamWaves * 64);
   auto run = [&](auto direct_c, auto pair_c) {
@@ -2895,23 +2896,29 @@ unsigned ms_segment(unsigned channel_blocks, size_t length, bool pairs) {
 }  // namespace
 
 // Segment length of the row stream: the longest of 16, 32, 64 and 128 rows
-// whose grid leaves more than a block per CU, for 128 rows two per CU. With
-// F32 rows and the exact windows (8 lead rows) 64 rows also need two: those
-// are bound by their reads. Measured at W = 4096, 16 / 32 / 64 / 128 rows per
-// segment, us:
+// whose grid leaves more than a block per CU, for 128 rows two per CU. F32 rows
+// are bound by their reads: with the exact windows (8 lead rows) 64 rows need
+// 1.6 blocks per CU, but with F32 outputs 144 blocks are enough. Measured at W = 4096, 16 / 32 / 64 / 128
+// rows per segment, us (F32: inputs from HBM, then from the memory-side cache):
 //   BF16, padded windows (14 lead rows): 1500 rows 18.9 / 16.1 / 18.7 / 29.6,
 //     2049 rows 26.0 / 25.6 / 23.3 / 30.1, 3000 rows 31.5 / 27.6 / 24.1 / 31.0,
 //     4096 rows 40.0 / 32.9 / 25.4 / 31.3, 8192 rows 73.2 / 60.0 / 51.8 / 43.6
 //   BF16, exact windows: 1024 rows 10.0 / 10.1 / 13.9 / 21.3, 3000 rows 25.2 /
 //     20.8 / 19.2 / 23.6, 8192 rows 52.2 / 51.6 / 44.3 / 39.9
-//   F32, exact windows: 2049 rows 32.5 / 29.7 / 34.0 / 39.4, 3000 rows 39.9 /
-//     33.6 / 35.7 / 41.5, 6000 rows 72.6 / 63.1 / 57.4 / 62.9.
-unsigned hcs_stream_segment(size_t width, size_t length, bool f32_exact) {
+//   F32, exact windows, 16-bit outputs: 1800 rows 28.4 / 26.9 / 28.8 / 41.2 and
+//     24.1 / 19.4 / 19.4 / 29.6, 3000 rows 43.1 / 39.4 / 42.5 / 46.1 and 37.1 /
+//     32.9 / 29.8 / 31.0, 3500 rows 52.3 / 47.3 / 46.6 / 48.0 and 43.9 / 39.5 /
+//     32.4 / 32.7
+//   F32 outputs: 1100 rows 22.1 / 22.9 / 22.2 / 34.4 and 17.4 / 16.9 / 16.2 /
+//     25.3, 1800 rows 29.8 / 28.9 / 26.9 / 37.8 and 25.5 / 21.3 / 21.0 / 26.4,
+//     3500 rows 54.6 / 50.4 / 46.1 / 46.0 and 46.2 / 42.0 / 35.9 / 35.8.
+unsigned hcs_stream_segment(size_t width, size_t length, bool f32_rows, bool exact, bool f32_out) {
   const unsigned channel_blocks = ceil_div(width, kStreamChannels);
+  const unsigned blocks64 = f32_rows && f32_out ? 144U : f32_rows && exact ? 400U : 257U;
   unsigned rows = kStreamRows;
   for (unsigned next = 2 * kStreamRows; next <= static_cast<unsigned>(kStreamMaxRows); next *= 2) {
-    const bool two_per_cu = next == 128 || (next == 64 && f32_exact);
-    if (channel_blocks * ceil_div(length, next) < (two_per_cu ? 512U : 257U))
+    const unsigned least = next == 32 ? 257U : next == 64 ? blocks64 : 512U;
+    if (channel_blocks * ceil_div(length, next) < least)
       break;
     rows = next;
   }

@@ -36,8 +36,9 @@ LinearPlan plan_linear(size_t M, size_t N, size_t K, bool split, bool gated,
 int choose_fp8_tile(size_t M, size_t N, size_t K, bool k32);
 constexpr int kFp8TileCount = 6;
 
-// Rows per segment of the HCS row stream (hyena.hip).
-unsigned hcs_stream_segment(size_t width, size_t length, bool f32_exact);
+// Rows per segment of the HCS row stream (hyena.hip); exact: a short FIR of 3
+// and 7 taps.
+unsigned hcs_stream_segment(size_t width, size_t length, bool f32_rows, bool exact, bool f32_out);
 
 // Whether the HCM row stream takes filter groups that are no multiple of 16
 // (hyena.hip), rows and outputs aligned.

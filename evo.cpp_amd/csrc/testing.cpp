@@ -10,8 +10,9 @@
 
 #define EVO_TEST_API extern "C" __attribute__((visibility("default")))
 
-EVO_TEST_API unsigned evo_test_hcs_stream_segment(size_t width, size_t length, int f32_exact) {
-  return evo::hip::hcs_stream_segment(width, length, f32_exact != 0);
+EVO_TEST_API unsigned evo_test_hcs_stream_segment(size_t width, size_t length, int f32_rows,
+                                                  int exact, int f32_out) {
+  return evo::hip::hcs_stream_segment(width, length, f32_rows != 0, exact != 0, f32_out != 0);
 }
 
 EVO_TEST_API int evo_test_hcm_stream_two_groups(size_t group_size, size_t length, int taps,

@@ -16,7 +16,7 @@ SLACK = 1.06
 def rules():
     lib = ctypes.CDLL(LIB)
     size = ctypes.c_size_t
-    lib.evo_test_hcs_stream_segment.argtypes = [size, size, ctypes.c_int]
+    lib.evo_test_hcs_stream_segment.argtypes = [size, size] + 3 * [ctypes.c_int]
     lib.evo_test_hcs_stream_segment.restype = ctypes.c_uint
     lib.evo_test_hcm_stream_two_groups.argtypes = [size, size] + 3 * [ctypes.c_int]
     lib.evo_test_linear_plan.argtypes = [size, size, size, ctypes.c_int, ctypes.c_int, size,
@@ -25,8 +25,10 @@ def rules():
     return lib
 
 
-# (width, length, F32 rows and exact windows): us with segments of 16, 32, 64
-# and 128 rows. BF16 rows with 5 taps (padded windows) or 7 (exact), F32 with 7.
+# (width, length, kind): us with segments of 16, 32, 64 and 128 rows. Kinds:
+# 0 BF16 rows, 5 taps (padded windows) or 7 (exact); 1 F32 rows, 7 taps, 16-bit
+# outputs; 2 F32 rows and outputs, 7 taps; 3 those with 5 taps.
+HCS_KINDS = [(0, 0, 0), (1, 1, 0), (1, 1, 1), (1, 0, 1)]  # F32 rows, exact, F32 outputs
 HCS_SEGMENTS = [
     (4096, 130, 0, (8.7, 11.6, 17.4, 28.9)), (4096, 611, 0, (11.2, 12.2, 17.7, 29.2)),
     (4096, 1024, 0, (12.6, 13.1, 18.1, 29.3)), (4096, 1500, 0, (18.9, 16.1, 18.7, 29.6)),
@@ -38,12 +40,17 @@ HCS_SEGMENTS = [
     (4096, 611, 1, (12.5, 12.0, 17.7, 30.2)), (4096, 2049, 1, (32.5, 29.7, 34.0, 39.4)),
     (4096, 3000, 1, (39.9, 33.6, 35.7, 41.5)), (4096, 6000, 1, (72.6, 63.1, 57.4, 62.9)),
     (1920, 611, 1, (8.9, 11.7, 18.3, 31.4)), (1920, 6000, 1, (38.0, 32.9, 34.6, 39.9)),
+    (4096, 3500, 1, (43.9, 39.5, 32.4, 32.7)), (4096, 4000, 1, (55.7, 50.5, 50.9, 51.2)),
+    (4096, 950, 2, (17.7, 18.0, 22.0, 34.9)), (4096, 1100, 2, (17.4, 16.9, 16.2, 25.3)),
+    (4096, 1800, 2, (29.8, 28.9, 26.9, 37.8)), (4096, 2700, 2, (43.1, 40.4, 41.0, 42.7)),
+    (4096, 3000, 2, (39.5, 36.1, 31.9, 31.8)), (4096, 3500, 2, (54.6, 50.4, 46.1, 46.0)),
+    (4096, 1800, 3, (36.1, 31.3, 29.1, 40.0)), (4096, 3000, 3, (53.4, 52.2, 45.1, 46.5)),
 ]
 
 
-@pytest.mark.parametrize("width,length,f32_exact,times", HCS_SEGMENTS)
-def test_hcs_stream_segment(rules, width, length, f32_exact, times):
-    rows = rules.evo_test_hcs_stream_segment(width, length, f32_exact)
+@pytest.mark.parametrize("width,length,kind,times", HCS_SEGMENTS)
+def test_hcs_stream_segment(rules, width, length, kind, times):
+    rows = rules.evo_test_hcs_stream_segment(width, length, *HCS_KINDS[kind])
     assert times[(16, 32, 64, 128).index(rows)] <= SLACK * min(times)
 
 
@@ -60,8 +67,8 @@ HCM_TWO_GROUPS = [
     (15, 7, 20, 0, 1, (18.4, 17.4)), (24, 2, 64, 0, 1, (21.1, 19.2)),
     (15, 3, 33, 1, 1, (16.5, 18.3)),
     (24, 4, 33, 1, 0, (8.6, 9.0)), (15, 4, 40, 1, 1, (17.7, 18.6)), (15, 5, 20, 1, 0, (9.6, 8.9)),
-    (15, 5, 20, 1, 1, (17.3, 18.1)), (24, 3, 64, 1, 1, (19.9, 19.7)), (15, 5, 40, 1, 1, (20.6, 19.3)),
-    (15, 3, 40, 1, 0, (9.5, 8.8)),
+    (15, 5, 20, 1, 1, (17.3, 18.1)), (24, 3, 64, 1, 1, (19.9, 19.7)),
+    (15, 5, 40, 1, 1, (20.6, 19.3)),     (15, 3, 40, 1, 0, (9.5, 8.8)),
 ]
 
 
