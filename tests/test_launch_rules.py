@@ -68,7 +68,7 @@ HCM_TWO_GROUPS = [
     (15, 3, 33, 1, 1, (16.5, 18.3)),
     (24, 4, 33, 1, 0, (8.6, 9.0)), (15, 4, 40, 1, 1, (17.7, 18.6)), (15, 5, 20, 1, 0, (9.6, 8.9)),
     (15, 5, 20, 1, 1, (17.3, 18.1)), (24, 3, 64, 1, 1, (19.9, 19.7)),
-    (15, 5, 40, 1, 1, (20.6, 19.3)),     (15, 3, 40, 1, 0, (9.5, 8.8)),
+    (15, 5, 40, 1, 1, (20.6, 19.3)), (15, 3, 40, 1, 0, (9.5, 8.8)),
 ]
 
 
