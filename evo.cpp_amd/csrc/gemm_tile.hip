@@ -287,32 +287,30 @@ struct TileEntry {
   TileCost split, plane;  // hi + lo activation planes, one plane
 };
 // Least-squares fits over 5 to 8192 rows of ten (N, K), those of the 7B and 1B
-// topologies among them (median error 2-6 %). With and without a workspace
-// the choice takes 1.2 % (up to 150 rows) or 0.4 % more than the fastest tile
-// and split in the geometric mean, 24 % at worst (1000 rows of 512 x 4096), and
-// nowhere over 1 % more than the 256 x 256 tile.
+// topologies among them (median error 2-6 %), each then scaled by 1.00 to 1.15
+// so that the choice among the tiles is the best one: with the plain fits,
+// products of a few thousand rows were up to 10 % slower than on 256 x 256
+// tiles (5000 rows of 4096 x 4096, two planes: 407 us on 128 x 128, 366 there).
+// Over 1060 products, with and without a workspace, the choice takes 0.4 % more
+// than the fastest tile and split in the geometric mean, 21 % at worst (5 rows
+// of 512 x 4096, one plane), and 4 % more than 256 x 256 at worst.
 constexpr TileEntry kTiles[] = {
-    {16, 16, 128, {1.85F, 1.31F, 0.013F, 2, {0.209F, 0.361F}, 7.33F}, {2.09F, 1.09F, 0.0F, 3, {0.203F, 0.302F, 0.397F}, 5.36F}},
-    {16, 32, 128, {2.37F, 1.05F, 0.020F, 2, {0.276F, 0.481F}, 5.16F}, {2.12F, 1.09F, 0.013F, 2, {0.251F, 0.375F}, 5.22F}},
-    {32, 32, 128, {1.63F, 1.90F, 0.112F, 1, {0.278F}, 8.2F}, {1.73F, 1.77F, 0.040F, 1, {0.255F}, 5.39F}},
-    {32, 64, 128, {2.05F, 1.92F, 0.173F, 1, {0.381F}, 4.82F}, {2.11F, 1.83F, 0.078F, 1, {0.326F}, 4.90F}},
-    {32, 96, 128, {2.43F, 2.08F, 0.145F, 1, {0.510F}, 4.86F}, {2.40F, 1.88F, 0.076F, 1, {0.459F}, 4.93F}},
-    {64, 64, 64, {1.72F, 2.44F, 0.087F, 1, {0.296F}, 8.0F}, {2.10F, 2.31F, 0.017F, 2, {0.262F, 0.457F}, 5.07F}},
-    {64, 128, 64, {2.49F, 4.02F, 0.121F, 1, {0.413F}, 4.39F, 6.93F}, {3.07F, 3.34F, 0.069F, 1, {0.338F}, 4.30F}},
-    {64, 192, 64, {2.30F, 5.65F, 0.158F, 1, {0.564F}, 4.56F, 6.36F}, {3.16F, 4.74F, 0.068F, 1, {0.488F}, 4.27F}},
-    {128, 128, 64, {1.97F, 5.73F, 0.181F, 1, {0.700F}, 9.0F, 6.66F}, {1.30F, 6.29F, 0.120F, 1, {0.439F}, 4.39F, 6.42F}},
-    {128, 192, 64, {2.69F, 6.49F, 0.250F, 1, {1.059F}, 4.33F, 5.59F}, {3.66F, 5.62F, 0.209F, 1, {0.834F}, 4.12F}},
+    {16, 16, 128, {1.91F, 1.35F, 0.013F, 2, {0.215F, 0.372F}, 7.12F}, {2.09F, 1.09F, 0.0F, 3, {0.203F, 0.302F, 0.397F}, 5.36F}},
+    {16, 32, 128, {2.56F, 1.13F, 0.022F, 2, {0.298F, 0.519F}, 4.78F}, {2.14F, 1.1F, 0.013F, 2, {0.254F, 0.379F}, 5.17F}},
+    {32, 32, 128, {1.83F, 2.13F, 0.125F, 1, {0.311F}, 7.32F}, {1.87F, 1.91F, 0.043F, 1, {0.275F}, 4.99F}},
+    {32, 64, 128, {2.09F, 1.96F, 0.176F, 1, {0.389F}, 4.73F}, {2.26F, 1.96F, 0.083F, 1, {0.349F}, 4.58F}},
+    {32, 96, 128, {2.67F, 2.29F, 0.16F, 1, {0.561F}, 4.42F}, {2.76F, 2.16F, 0.087F, 1, {0.528F}, 4.29F}},
+    {64, 64, 64, {1.89F, 2.68F, 0.096F, 1, {0.326F}, 7.27F}, {2.31F, 2.54F, 0.019F, 2, {0.288F, 0.503F}, 4.61F}},
+    {64, 128, 64, {2.59F, 4.18F, 0.126F, 1, {0.43F}, 4.22F, 6.66F}, {3.25F, 3.54F, 0.073F, 1, {0.358F}, 4.06F}},
+    {64, 192, 64, {2.39F, 5.88F, 0.164F, 1, {0.587F}, 4.38F, 6.12F}, {3.41F, 5.12F, 0.073F, 1, {0.527F}, 3.95F}},
+    {128, 128, 64, {2.07F, 6.02F, 0.19F, 1, {0.735F}, 8.57F, 6.34F}, {1.37F, 6.6F, 0.126F, 1, {0.461F}, 4.18F, 6.11F}},
+    {128, 192, 64, {2.91F, 7.01F, 0.27F, 1, {1.144F}, 4.01F, 5.18F}, {3.84F, 5.9F, 0.219F, 1, {0.876F}, 3.92F}},
 };
 constexpr int kTileCount = static_cast<int>(sizeof(kTiles) / sizeof(kTiles[0]));
 static_assert(kTileCount == kGemmTiles, "the tiles of gemm_tile()");
 // The 256 x 256 tile of gemm.hip, the other candidate.
 constexpr TileEntry kLargeTile = {256, 256, 32, {0.0F, 7.29F, 0.532F, 1, {1.041F}},
                                   {0.0F, 7.71F, 0.233F, 1, {0.750F}}};
-// A small tile has to come out this much below 256 x 256, twice the fits'
-// error: with less, products of a few thousand rows were slower than there by
-// up to 10 % (5000 rows of 4096 x 4096, two planes: 407 us on 128 x 128, 366 on
-// 256 x 256), and without it the choice is no faster in the mean.
-constexpr double kSmallMargin = 1.07;
 
 double entry_us(const TileEntry &t, bool split, size_t M, size_t N, size_t K, size_t parts) {
   const TileCost &cost = split ? t.split : t.plane;
@@ -350,8 +348,7 @@ TileChoice choose_gemm_tile(size_t M, size_t N, size_t K, bool split, bool gated
       if (parts > 1 && (K / parts < 4 * seg || N % 4 != 0 || gated ||
                         parts * M * N * sizeof(float) > workspace_bytes))
         continue;
-      const double us =
-          kSmallMargin * (entry_us(kTiles[t], split, M, N, K, parts) + reduction(parts));
+      const double us = entry_us(kTiles[t], split, M, N, K, parts) + reduction(parts);
       if (us < best_us) {
         best_us = us;
         best = TileChoice{t, static_cast<int>(parts)};
