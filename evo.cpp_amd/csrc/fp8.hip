@@ -539,7 +539,7 @@ constexpr Fp8TileEntry kFp8Tiles[kFp8TileCount] = {
 // Another tile has to come out at least this much below 128 x 192, the fits'
 // error: 1300 rows at W = 4096, K32, took 132 us on 64 x 128, whose estimate
 // was 2 % lower, against 122.
-constexpr double kFp8Margin = 1.04;
+constexpr float kFp8Margin = 1.04F;
 
 unsigned elementwise_grid(size_t n) {
   const size_t blocks = (n + 255) / 256;
@@ -549,15 +549,16 @@ unsigned elementwise_grid(size_t n) {
 }  // namespace
 
 int choose_fp8_tile(size_t M, size_t N, size_t K, bool k32) {
+  const float weight_bytes = static_cast<float>(N) * static_cast<float>(K);
   int best = 0;
-  double best_us = 0.0;
+  float best_us = INFINITY;
   for (int t = 0; t < kFp8TileCount; ++t) {
     const Fp8TileEntry &e = kFp8Tiles[t];
-    const double us = (t == 0 ? 1.0 : kFp8Margin) *
-                      tile_us(k32 ? e.k32 : e.k128,
-                              static_cast<double>(ceil_div(M, e.bm)) * ceil_div(N, e.bn),
-                              static_cast<double>(K / kBK), static_cast<double>(N) * K);
-    if (t == 0 || us < best_us) {
+    const float margin = t == 0 ? 1.0F : kFp8Margin;
+    const float us = margin * tile_us(k32 ? e.k32 : e.k128, ceil_div(M, e.bm) * ceil_div(N, e.bn),
+                                      static_cast<uint32_t>(K / kBK), weight_bytes, 0.0F,
+                                      best_us / margin);
+    if (us < best_us) {
       best = t;
       best_us = us;
     }

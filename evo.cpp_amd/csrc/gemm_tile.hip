@@ -24,6 +24,7 @@
 //     416 -> 97, 1000 rows 434 -> 155 (floor 17)
 //   N = K = 1920: 61 rows 80 -> 8 us, 1000 rows 90 -> 23.
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "common.hpp"
@@ -312,16 +313,21 @@ static_assert(kTileCount == kGemmTiles, "the tiles of gemm_tile()");
 constexpr TileEntry kLargeTile = {256, 256, 32, {0.0F, 7.29F, 0.532F, 1, {1.041F}},
                                   {0.0F, 7.71F, 0.233F, 1, {0.750F}}};
 
-double entry_us(const TileEntry &t, bool split, size_t M, size_t N, size_t K, size_t parts) {
+float entry_us(const TileEntry &t, bool split, uint32_t M, uint32_t N, uint32_t k_part,
+               uint32_t parts, float weight_bytes, float limit) {
   const TileCost &cost = split ? t.split : t.plane;
-  const double blocks = static_cast<double>(ceil_div(M, t.bm)) * ceil_div(N, t.bn) * parts;
-  // An XCD's resident blocks are consecutive, rows first: 32 row blocks and
-  // more share no activation rows, which each block column then reads again.
-  const double resident = std::min(32.0 * cost.slots, std::max(1.0, blocks / 8.0));
-  const double down = std::min<double>(ceil_div(M, t.bm), resident);
-  const double rows = down * t.bm * (split ? 2 : 1) + std::max(1.0, resident / down) * t.bn;
-  return tile_us(cost, blocks, ceil_div(K / parts, t.seg), 2.0 * static_cast<double>(N) * K,
-                 blocks / resident * rows * 2.0 * static_cast<double>(K / parts));
+  const uint32_t down = (M + t.bm - 1) / t.bm, blocks = down * ((N + t.bn - 1) / t.bn) * parts;
+  float fill_bytes = 0.0F;
+  if (cost.fill > 0.0F) {
+    // An XCD's resident blocks are consecutive, rows first: 32 row blocks and
+    // more share no activation rows, which each block column then reads again.
+    const float all = static_cast<float>(blocks);
+    const float resident = std::min(32.0F * cost.slots, std::max(1.0F, all / 8.0F));
+    const float shared = std::min(static_cast<float>(down), resident);
+    const float rows = shared * t.bm * (split ? 2 : 1) + std::max(1.0F, resident / shared) * t.bn;
+    fill_bytes = all / resident * rows * 2.0F * static_cast<float>(k_part);
+  }
+  return tile_us(cost, blocks, (k_part + t.seg - 1) / t.seg, weight_bytes, fill_bytes, limit);
 }
 
 }  // namespace
@@ -331,24 +337,33 @@ TileChoice choose_gemm_tile(size_t M, size_t N, size_t K, bool split, bool gated
   // Partial products cost their reduction: a launch that grows with the parts
   // (5 rows of 1920 x 5120, two planes: 4 parts 9.8 us, 8 parts 11.1) unless
   // the next norm sums them as it reads its rows, and their bytes at ~4 TB/s.
+  const float weight_bytes = 2.0F * static_cast<float>(N) * static_cast<float>(K);
+  const float part_us = static_cast<float>(M) * static_cast<float>(N) * 1.0e-6F;
   auto reduction = [&](size_t parts) {
-    return parts == 1 ? 0.0
-                      : (deferred ? 0.0 : 2.0 + 0.3 * static_cast<double>(parts)) +
-                            4.0 * static_cast<double>(parts) * M * N / 4.0e6;
+    return parts == 1 ? 0.0F
+                      : (deferred ? 0.0F : 2.0F + 0.3F * static_cast<float>(parts)) +
+                            static_cast<float>(parts) * part_us;
   };
+  const auto m = static_cast<uint32_t>(M), n = static_cast<uint32_t>(N);
   TileChoice best;
-  double best_us = entry_us(kLargeTile, split, M, N, K, large_parts) + reduction(large_parts);
-  for (int t = 0; t < kTileCount; ++t) {
-    const size_t seg = static_cast<size_t>(kTiles[t].seg);
-    if (gated && kTiles[t].bn % 32 != 0)
-      continue;  // a gated tile pairs whole 16-column tiles
-    for (size_t parts = 1; parts <= 8; parts *= 2) {
-      if (K % (32 * parts) != 0 || K / parts < seg)
+  float best_us = entry_us(kLargeTile, split, m, n, static_cast<uint32_t>(K / large_parts),
+                           static_cast<uint32_t>(large_parts), weight_bytes, INFINITY) +
+                  reduction(large_parts);
+  const size_t plane_bytes = M * N * sizeof(float);
+  const bool splittable = !gated && N % 4 == 0;
+  for (size_t parts = 1; parts <= 8; parts *= 2) {
+    if (K % (32 * parts) != 0 || (parts > 1 && (!splittable || parts * plane_bytes > workspace_bytes)))
+      break;
+    const auto k_part = static_cast<uint32_t>(K / parts);
+    const float reduce_us = reduction(parts);
+    for (int t = 0; t < kTileCount; ++t) {
+      if (gated && kTiles[t].bn % 32 != 0)
+        continue;  // a gated tile pairs whole 16-column tiles
+      if (k_part < static_cast<uint32_t>((parts > 1 ? 4 : 1) * kTiles[t].seg))
         continue;
-      if (parts > 1 && (K / parts < 4 * seg || N % 4 != 0 || gated ||
-                        parts * M * N * sizeof(float) > workspace_bytes))
-        continue;
-      const double us = entry_us(kTiles[t], split, M, N, K, parts) + reduction(parts);
+      const float us = entry_us(kTiles[t], split, m, n, k_part, static_cast<uint32_t>(parts),
+                                weight_bytes, best_us - reduce_us) +
+                       reduce_us;
       if (us < best_us) {
         best_us = us;
         best = TileChoice{t, static_cast<int>(parts)};

@@ -4,6 +4,8 @@
 // products on a given block tile. No part of the product's interface.
 #include <hip/hip_runtime.h>
 
+#include <chrono>
+
 #include "gemm_tile.hpp"
 #include "launch_rules.hpp"
 #include "ops.hpp"
@@ -28,6 +30,16 @@ EVO_TEST_API int evo_test_linear_plan(size_t m, size_t n, size_t k, int split, i
   *parts = plan.choice.splits;
   *tail = plan.tail;
   return plan.choice.tile;
+}
+// Mean host time of that choice, in ns.
+EVO_TEST_API double evo_test_linear_plan_ns(size_t m, size_t n, size_t k, size_t workspace_bytes,
+                                            int calls) {
+  using Clock = std::chrono::steady_clock;
+  volatile int tile = 0;
+  const auto start = Clock::now();
+  for (int i = 0; i < calls; ++i)
+    tile = evo::hip::plan_linear(m, n, k, true, false, workspace_bytes, false).choice.tile;
+  return std::chrono::duration<double, std::nano>(Clock::now() - start).count() / calls;
 }
 EVO_TEST_API int evo_test_linear_tiles(void) { return evo::hip::kGemmTiles; }
 EVO_TEST_API int evo_test_fp8_tiles(void) { return evo::hip::kFp8TileCount; }

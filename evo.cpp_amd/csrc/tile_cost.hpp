@@ -5,6 +5,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstdint>
 
 namespace evo::hip {
 
@@ -24,22 +25,26 @@ struct TileCost {
 
 // The bounds join in a 6-norm: under a hard maximum every tile that stays
 // below the bytes' time cost the same, and the order of the table picked among
-// them (17 to 32 rows of 22528 x 4096: 44 to 49 us against 39).
-inline double tile_us(const TileCost &c, double blocks, double steps, double weight_bytes,
-                      double fill_bytes = 0.0) {
-  const double per_round = 256.0 * c.slots;
-  const double rounds = std::floor(blocks / per_round);
-  const int rest = static_cast<int>(std::ceil((blocks - rounds * per_round) / 256.0));
-  double us = c.launch + rounds * (c.epilogue + steps * c.step[c.slots - 1]) +
-              c.load * steps * blocks / 256.0;
+// them (17 to 32 rows of 22528 x 4096: 44 to 49 us against 39). A candidate
+// that can't come out below `limit` returns any time of at least `limit`: each
+// call weighs up to 40 of them, and its launch waits for that.
+inline float tile_us(const TileCost &c, uint32_t blocks, uint32_t steps, float weight_bytes,
+                     float fill_bytes, float limit) {
+  const uint32_t per_round = 256U * static_cast<uint32_t>(c.slots);
+  const uint32_t rounds = blocks / per_round, rest = (blocks - rounds * per_round + 255U) / 256U;
+  const float k_steps = static_cast<float>(steps);
+  float us = c.launch + static_cast<float>(rounds) * (c.epilogue + k_steps * c.step[c.slots - 1]) +
+             c.load * k_steps * static_cast<float>(blocks) * (1.0F / 256.0F);
   if (rest > 0)
-    us += c.epilogue + steps * c.step[rest - 1];
-  const double bytes_us = 1.0 + weight_bytes / (1.0e6 * c.rate);
-  const double fill_us = c.fill > 0.0F ? fill_bytes / (1.0e6 * c.fill) : 0.0;
-  const double longest = std::max({us, bytes_us, fill_us});
-  double sum = 0.0;
-  for (const double bound : {us, bytes_us, fill_us}) {
-    const double ratio = bound / longest, cube = ratio * ratio * ratio;
+    us += c.epilogue + k_steps * c.step[rest - 1];
+  const float bytes_us = 1.0F + weight_bytes / (1.0e6F * c.rate);
+  const float fill_us = c.fill > 0.0F ? fill_bytes / (1.0e6F * c.fill) : 0.0F;
+  const float longest = std::max({us, bytes_us, fill_us});
+  if (longest >= limit)
+    return longest;
+  float sum = 0.0F;
+  for (const float bound : {us, bytes_us, fill_us}) {
+    const float ratio = bound / longest, cube = ratio * ratio * ratio;
     sum += cube * cube;
   }
   return longest * std::cbrt(std::sqrt(sum));

@@ -21,6 +21,8 @@ def rules():
     lib.evo_test_hcm_stream_two_groups.argtypes = [size, size] + 3 * [ctypes.c_int]
     lib.evo_test_linear_plan.argtypes = [size, size, size, ctypes.c_int, ctypes.c_int, size,
                                          ctypes.POINTER(ctypes.c_int), ctypes.POINTER(size)]
+    lib.evo_test_linear_plan_ns.argtypes = 4 * [size] + [ctypes.c_int]
+    lib.evo_test_linear_plan_ns.restype = ctypes.c_double
     lib.evo_test_fp8_tile.argtypes = [size, size, size, ctypes.c_int]
     return lib
 
@@ -165,3 +167,11 @@ FP8 = [
 def test_fp8_tile(rules, m, n, k, k128, times):
     tile = rules.evo_test_fp8_tile(m, n, k, k128)
     assert times[tile] <= SLACK * min(times) and times[tile] <= 1.02 * times[0]
+
+
+def test_linear_choice_is_cheap(rules):
+    """A product of a few rows is over in 6 us: the choice of its tile may not
+    take a good part of that (0.55 us; 3.6 us with a root per candidate). The
+    least of 20 batches, so that a busy host does not count."""
+    times = [rules.evo_test_linear_plan_ns(5, 512, 4096, 1 << 26, 500) for _ in range(20)]
+    assert min(times) < 1800
